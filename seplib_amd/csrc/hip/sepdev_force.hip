@@ -437,7 +437,7 @@ __global__ void k_quantize(sepk_state s, long npad, double q0, double q1, double
 		s.qpos[t] = sepk_quant(s.pos[t], q0, q1, q2);
 }
 
-static int sepk_fresh_qpos(sepdev *d, const double *L)
+int sepk_fresh_qpos(sepdev *d, const double *L)
 {
 	if (!d->qpos_stale && d->qL[0] == L[0] && d->qL[1] == L[1] && d->qL[2] == L[2])
 		return 0;

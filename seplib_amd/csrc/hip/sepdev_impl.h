@@ -475,6 +475,8 @@ __device__ __forceinline__ void sepk_add_sym9(double *dst9, const double *w6,
 int sepk_materialize_forces(sepdev *d);
 // Launches the owed bonded gathers (one kernel for all of them).
 int sepk_flush_gathers(sepdev *d);
+// requantizes qpos for the box L if it is stale (sepdev_force.hip)
+int sepk_fresh_qpos(sepdev *d, const double *L);
 // launches a pair call recorded for a fused step, if any (sepdev_force.hip)
 int sepk_flush_pair(sepdev *d);
 int sepk_flush_nh(sepdev *d);

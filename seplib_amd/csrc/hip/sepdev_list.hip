@@ -13,10 +13,10 @@
 //                  index (so the device order and every list are independent
 //                  of atomic timing) and move each member's state to its new
 //                  cell-sorted index in the spare copy
-//   k_build        one workgroup per cell: stage the stencil cells' segments
-//                  in LDS and append the candidates within the list cutoff
-//                  (each wave every fourth home atom, 64 candidates a round),
-//                  then copy the cells' permuted state home
+//   k_build_q      a wave per slab of a cell's atoms (k_build: a workgroup per
+//                  cell, for boxes that are not cubic): the stencil's atoms
+//                  within the list cutoff, 64 candidates at a time; then copy
+//                  the cells' permuted state home
 // and a BUILD task for the step's finisher.  With conditional = 1 every
 // kernel returns at once unless the device rebuild flag is set, so the
 // sequence can sit in a captured graph.
@@ -485,54 +485,50 @@ __device__ __forceinline__ void sepk_copy_home(const sepk_state &src, const sepk
 		sepk_copy_partners(src, dst, t, t, npad);
 }
 
-// One workgroup per home cell at a time (cells split into one contiguous
-// range per XCD, walked with a stride of the range's workgroup count).
-// The stencil cells' segments are staged in LDS as SoA chunks of
-// SEPK_BCHUNK candidates (position, device index, stencil offset, molecule,
-// quantized position) and the cell's members ("home" atoms, SEPK_BHOME at a
-// time) beside them.  Each wave owns every fourth home atom: a round takes
-// 64 staged candidates into registers (one a lane) and tests them against
-// each of the wave's atoms, whose position is an LDS broadcast; the lanes
-// that pass store their candidate to the atom's list at once, each at the
-// atom's length so far plus its rank among the passing lanes (mbcnt), and
-// the length (lane kk of a register for the wave's kk-th atom) grows by
-// their number.  Lists therefore come out in stencil-offset order and,
-// within a cell, in device order.  Entry k of atom t goes to slot
-// sepk_entry(k, t, npad).
+// Lists come out in stencil-offset order and, within a cell, in device order;
+// entry k of atom t goes to slot sepk_entry(k, t, npad).  Cells (and the
+// slices of their atoms) are split into one contiguous range per XCD, walked
+// with a stride of the range's workgroups or waves.
 //
-// SHIFT: with at least 5 cells on every axis and every atom inside its own
-// cell, |x_i - x_j| < 2l <= 0.4 L for a target cell reached without
-// crossing the box and > L - 2l >= 0.6 L for one reached across it, so the
-// reference's single-image wrap (subtract or add L exactly when |d| > L/2)
-// is the constant shift of the target cell; d + shift rounds exactly like
-// its d - L / d + L, and d + 0 is d.  Otherwise the wrap is evaluated per
-// candidate.
-//
-// Quantized test (SHIFT and a cubic box): every coordinate is also held as
-// floor(x * 65536 / L) mod 2^16, x and y in one word and z in the low half
-// of another.  A packed 16-bit subtraction gives the minimum-image
-// difference in units of u = L / 65536, each component within one unit of
-// the exact one (|x_i - x_j| < 0.4 L keeps it away from the wrap), and two
+// Quantized build (k_build_q): a cubic box of at least 3 cells an axis with
+// every atom inside it, the usual case.  Every coordinate is held as
+// floor(x * 65536 / L) mod 2^16 (the upper half of the pair kernels'
+// quantized record), x and y in one word and z in the low half of another.  A
+// packed 16-bit subtraction gives the minimum-image difference in units of
+// u = L / 65536, each component within one unit of the exact one, and two
 // saturating packed dot products its square r2q.  With R = r_list / u the
 // distance is below r_list - 0.26 u when r2q < floor((R - 2)^2) and above
 // r_list + 0.26 u when r2q > ceil((R + 2)^2) (sqrt(3) < 1.74), far outside
-// the rounding of the FP64 r2; only candidates between the two bounds (a
-// shell about 4 u thick: a few in ten thousand) take the FP64 test, the
-// reference's own, so the accepted set is the FP64 test's exactly.
+// the rounding of the FP64 r2 (a component near half the box, whose sign may
+// go either way, has |d| >= L/2 - u > 1.4 r_list); only candidates between
+// the two bounds (a shell about 4 u thick: a few in ten thousand) take the
+// FP64 test, the reference's own, so the accepted set is the FP64 test's
+// exactly.
+//
+// FP64 build (k_build): every other box, each candidate by the reference's
+// test.  SHIFT: with at least 5 cells on every axis and every atom inside
+// its own cell, |x_i - x_j| < 2l <= 0.4 L for a target cell reached without
+// crossing the box and > L - 2l >= 0.6 L for one reached across it, so the
+// reference's single-image wrap (subtract or add L exactly when |d| > L/2) is
+// the constant shift of the target cell; d + shift rounds exactly like its
+// d - L / d + L, and d + 0 is d.  Otherwise the wrap is evaluated per
+// candidate.
 #define SEPK_BT 256      // threads of a build workgroup (4 waves)
-#define SEPK_BCHUNK 384  // candidates staged at a time
-#define SEPK_BHOME 64    // home atoms staged at a time
+#define SEPK_BCHUNK 384  // candidates staged at a time, FP64 build
+#define SEPK_BHOME 64    // home atoms at a time
+// rounds of 64 candidates that a lane holds, quantized build (fewer with the
+// same-molecule rule, whose molecule numbers take registers and LDS too)
+#define SEPK_QROUNDS(EXCL) ((EXCL) == 3 ? 4 : 5)
 #define SEPK_BGRID 1792  // build workgroups at most (a multiple of 8)
+#define SEPK_QSLICE 11   // home atoms of a wave, quantized build, in large systems
 static_assert(SEPK_BCHUNK % 64 == 0, "candidates are tested 64 at a time");
 static_assert(SEPK_BHOME <= 64 * (SEPK_BT / 64), "a wave's home atoms fit its lanes");
 
 struct sepk_build_lds {
 	double cx[SEPK_BCHUNK], cy[SEPK_BCHUNK], cz[SEPK_BCHUNK];
-	uint2 cq[SEPK_BCHUNK];
 	int cj[SEPK_BCHUNK], cm[SEPK_BCHUNK];
 	unsigned char co[SEPK_BCHUNK];
 	double hx[SEPK_BHOME], hy[SEPK_BHOME], hz[SEPK_BHOME];
-	uint2 hq[SEPK_BHOME];
 	int horig[SEPK_BHOME], hmol[SEPK_BHOME];
 	int segjs[SEPDEV_MAX_OFF], segpre[SEPDEV_MAX_OFF + 1];
 	int segrule[SEPDEV_MAX_OFF]; // rule when the target is the home cell, else -1
@@ -540,46 +536,55 @@ struct sepk_build_lds {
 	int hs, h, anyshift;
 };
 
-// Lists of fewer than 2^20 padded atoms and under 4 GiB: a list slot is a
-// 32-bit byte offset from its atom's first slot, formed with a 24-bit
-// multiply (otherwise sepk_entry's 64-bit arithmetic).
-__device__ __forceinline__ bool sepk_np32(long npad, int cap)
-{
-	return npad < (1l << 20) &&
-	       (long)((cap + SEPK_PAD - 1) / SEPK_PAD) * npad * SEPK_PAD * 4 < (1l << 32);
-}
-
-// Bounds of the quantized test; on = the test applies (SHIFT, cubic box).
+// Bounds of the quantized test, in units of L / 2^16, and of the second one
+// for the candidates between them, in units of L / 2^21.
 struct sepk_qtest {
-	double scale; // 65536 / L
+	double lo2f, hi2f;
 	int lo2, hi2;
-	bool on;
+	double icell[2], islice; // reciprocals: cells along x and y, slices a cell
 };
 
-__device__ __forceinline__ sepk_qtest sepk_qtest_of(const sepdev_grid &g, bool shift)
+// Whether the quantized build serves a grid (once its binning finds every
+// atom inside the box): three cells of at least r_list an axis, so that
+// R <= 21846 and both bounds are below 2^30 (SEPK_QNONE).
+static bool sepk_qtest_of(const sepdev_grid &g, sepk_qtest &q)
 {
-	sepk_qtest q;
-	q.scale = 65536.0 / g.L[0];
-	const double R = sqrt(g.rlist2) * q.scale;
-	// SHIFT has L >= 5 r_list, so R <= 13108 and both bounds fit 31 bits
-	q.on = shift && g.L[0] == g.L[1] && g.L[1] == g.L[2] && R < 30000.0;
-	q.lo2 = R > 2.0 ? (int)floor((R - 2.0) * (R - 2.0)) : 0;
-	q.hi2 = q.on ? (int)ceil((R + 2.0) * (R + 2.0)) : 0;
-	return q;
+	const double R = sqrt(g.rlist2) * (65536.0 / g.L[0]), Rf = 32.0 * R;
+	const bool on = g.n[0] >= 3 && g.n[1] >= 3 && g.n[2] >= 3 && g.noff == 27 &&
+			g.L[0] == g.L[1] && g.L[1] == g.L[2] && R > 2.0 && R < 21900.0;
+	q.lo2 = on ? (int)floor((R - 2.0) * (R - 2.0)) : 0;
+	q.hi2 = on ? (int)ceil((R + 2.0) * (R + 2.0)) : 0;
+	q.lo2f = floor((Rf - 2.0) * (Rf - 2.0));
+	q.hi2f = ceil((Rf + 2.0) * (Rf + 2.0));
+	q.icell[0] = 1.0 / g.n[0];
+	q.icell[1] = 1.0 / g.n[1];
+	return on;
 }
 
-// x and y in the low and high halves of .x, z in the low half of .y
-__device__ __forceinline__ uint2 sepk_quantize(const sepk_pos &p, double scale)
+// The build's form of a quantized record (sepk_quant): the upper 21 bits of
+// each coordinate, of which the upper 16 are x and y in the low and high
+// halves of .x and z in the low half of .y, and the lower 5 of x, y and z in
+// bits 16..30 of .y.
+__device__ __forceinline__ uint2 sepk_quant21(const int4 &q)
 {
-	const unsigned qx = (unsigned)(int)floor(p.x * scale) & 0xffffu;
-	const unsigned qy = (unsigned)(int)floor(p.y * scale) & 0xffffu;
-	const unsigned qz = (unsigned)(int)floor(p.z * scale) & 0xffffu;
-	return make_uint2(qx | qy << 16, qz);
+	const unsigned lx = (unsigned)q.x >> 11 & 31u, ly = (unsigned)q.y >> 11 & 31u,
+		       lz = (unsigned)q.z >> 11 & 31u;
+	return make_uint2((unsigned)q.x >> 16 | ((unsigned)q.y & 0xffff0000u),
+			  (unsigned)q.z >> 16 | ((lz << 5 | ly) << 5 | lx) << 16);
+}
+
+// The 21-bit coordinates of such a record in the upper bits of three words.
+__device__ __forceinline__ void sepk_words21(uint2 q, unsigned &x, unsigned &y, unsigned &z)
+{
+	x = q.x << 16 | (q.y >> 5 & 0xf800u);
+	y = (q.x & 0xffff0000u) | (q.y >> 10 & 0xf800u);
+	z = q.y << 16 | (q.y >> 15 & 0xf800u);
 }
 
 typedef short sepk_short2 __attribute__((ext_vector_type(2)));
 
-// Squared quantized minimum-image distance, saturated at 2^31 - 1.
+// Squared quantized minimum-image distance (16 bits a coordinate, .y without
+// the lower bits), saturated at 2^31 - 1.
 __device__ __forceinline__ int sepk_r2q(uint2 a, uint2 b)
 {
 	const sepk_short2 dxy =
@@ -596,26 +601,410 @@ __device__ __forceinline__ void sepk_writelane(int &v, int val, int lane)
 	asm volatile("v_writelane_b32 %0, %1, %2" : "+v"(v) : "s"(val), "{m0}"(lane));
 }
 
-// One round: the 64 staged candidates [q0, q0 + 64) of a chunk of kn
-// against the wave's home atoms i = wid, wid + 4, ... < hn, storing the
-// accepted ones to their lists.  Lane kk of cnt holds the list length of
-// the wave's kk-th home atom; entries at or beyond cap are counted but not
-// stored.
-// QNT: the quantized test (SHIFT holds).  SH: some stencil target of the
-// cell lies across the box (shift adds; the quantized test needs none).
-// EXCL: 0 = SEP_ALL, 2 = SEP_EXCL_BONDED, 3 = SEP_EXCL_SAME_MOL.
-template <bool SHIFT, bool SH, int EXCL, bool QNT, bool NP32>
+// SEP_EXCL_BONDED: whether the pair (t, j) stays in the list.
+__device__ __forceinline__ bool sepk_keep_bonded(const sepk_state &s, const sepdev_grid &g, long t,
+						 int j, long npad)
+{
+	const int oi = s.orig[t], oj = s.orig[j];
+	int sh = sepk_share(s.partners, npad, t, j, 0, 10, oi, oj);
+	if (g.bonded_all)
+		sh += sepk_share(s.partners, npad, t, j, 10, 10, oi, oj) +
+		      sepk_share(s.partners, npad, t, j, 20, 20, oi, oj);
+	// rule 2 is the Coulomb brute-force test of source/sepcoulomb.c:44, which
+	// excludes only when exactly one kind of partnership holds
+	return g.bonded_all == 2 ? sh != 1 : sh == 0;
+}
+
+// Number of set bits of m below this lane.
+__device__ __forceinline__ int sepk_rank(unsigned long long m)
+{
+	return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
+					      __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+}
+
+// Orders a wave's accesses to its own LDS row (the hardware executes them in
+// order; this keeps the compiler to it).
+__device__ __forceinline__ void sepk_wave_lds()
+{
+	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+	__builtin_amdgcn_wave_barrier();
+	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The candidates in `near` (record cq, index j) that are within the list
+// cutoff of atom t (record q): by the 21-bit records, and the few that lie
+// within two of their units of the cutoff by the reference's FP64 test
+// (there the image by rint is the reference's single-image wrap bit for bit,
+// sepk_wrap_fast).  One atom in three has a candidate in `near`, one in a
+// hundred needs positions from memory: a load here waits for the list
+// stores in flight as well.
+__device__ __forceinline__ unsigned long long sepk_near_test(const sepk_state &s,
+							     const sepdev_grid &g,
+							     const sepk_qtest &qt,
+							     unsigned long long near, uint2 q,
+							     const uint2 *cq, int t, int j)
+{
+	unsigned ax, ay, az, bx, by, bz;
+	sepk_words21(q, ax, ay, az);
+	sepk_words21(*cq, bx, by, bz);
+	const double ux = (double)((int)(ax - bx) >> 11), uy = (double)((int)(ay - by) >> 11),
+		     uz = (double)((int)(az - bz) >> 11);
+	const double u2 = fma(ux, ux, fma(uy, uy, uz * uz)); // exact
+	unsigned long long in = __ballot(u2 < qt.lo2f) & near;
+	const unsigned long long edge = __ballot(u2 <= qt.hi2f) & near & ~in;
+	if (edge) {
+		bool ok = false;
+		if (__builtin_amdgcn_inverse_ballot_w64(edge)) {
+			// the address is formed here, not held through the caller's loop
+			asm volatile("" : "+v"(j));
+			const sepk_pos pi = sepk_at(s.pos, (unsigned)t);
+			const sepk_pos pj = sepk_at(s.pos, (unsigned)j);
+			const double L = g.L[0], iL = 1.0 / L;
+			const double dx = sepk_wrap_fast(pi.x - pj.x, L, iL);
+			const double dy = sepk_wrap_fast(pi.y - pj.y, L, iL);
+			const double dz = sepk_wrap_fast(pi.z - pj.z, L, iL);
+			ok = dx * dx + dy * dy + dz * dz < g.rlist2;
+		}
+		in |= __ballot(ok);
+	}
+	return in;
+}
+
+// A packed 16-bit difference held within 16 bits.
+__device__ __forceinline__ sepk_short2 sepk_sub_sat(sepk_short2 a, sepk_short2 b)
+{
+	return __builtin_elementwise_sub_sat(a, b);
+}
+
+// One wave's LDS of the quantized build.
+template <int EXCL>
+struct sepk_qwave {
+	static constexpr int NR = SEPK_QROUNDS(EXCL), CAP = 64 * NR;
+	uint2 cq[CAP];                  // its candidates
+	int cj[CAP], cm[EXCL == 3 ? CAP : 1];
+	// an atom's accepted ones, the phantom after them
+	__align__(16) int row[CAP + SEPK_PAD];
+};
+
+// Quantized build: the wave's home atoms tb + i, i the bits of mine (lane i
+// holds the record and molecule of atom tb + i) against the nf candidates in
+// its LDS, appending the accepted ones to the lists.  Lane i of cnt holds the
+// list length of atom tb + i; entries at or beyond cap are counted but not stored.
+// last: the entries are padded with the phantom slot to a multiple of
+// SEPK_PAD.
+// A lane holds one candidate of every round in registers for all of the
+// atoms; for one atom all rounds are tested (one ballot a round), the passing
+// lanes put their candidate into the LDS row at the number of those before
+// them (mbcnt), and the row goes to the list, four slots a lane.
+template <int EXCL>
+__device__ __forceinline__ void sepk_build_pass(
+	sepk_qwave<EXCL> &W, const sepk_state &s, const sepdev_grid &g, const sepk_qtest &qt,
+	int nf, int tb, unsigned long long mine, uint2 hq, int hm, long npad, int cap, int phantom, bool last,
+	int *nbr, int &cnt)
+{
+	constexpr int NR = sepk_qwave<EXCL>::NR;
+	const int lane = threadIdx.x & 63;
+	const int nr = (nf + 63) / 64;
+	// this lane's four consecutive slots of 256, and the first of the four
+	// entries (SEPK_SUB apart) that they hold
+	const size_t lslot = (size_t)(lane / SEPK_SUB) * npad * SEPK_PAD + lane % SEPK_SUB * SEPK_BATCH;
+	const int lent = lane / SEPK_SUB * SEPK_PAD + lane % SEPK_SUB;
+	static_assert(SEPK_SUB == 4 && SEPK_BATCH == 4, "four slots a lane");
+	uint2 cq[NR];
+	int cj[NR], cm[NR];
+#pragma unroll
+	for (int r = 0; r < NR; r++)
+		if (r < nr) {
+			const int f = 64 * r + lane;
+			cq[r] = W.cq[f];
+			cq[r].y &= 0xffffu;
+			cj[r] = W.cj[f];
+			if (EXCL == 3)
+				cm[r] = W.cm[f];
+		}
+	// the candidates of the last round
+	const unsigned long long some = nf & 63 ? ~(~0ull << (nf & 63)) : ~0ull;
+	for (; mine; mine &= mine - 1ull) {
+		const int i = __builtin_ctzll(mine), t = tb + i;
+		const uint2 q = make_uint2((unsigned)__builtin_amdgcn_readlane((int)hq.x, i),
+					   (unsigned)__builtin_amdgcn_readlane((int)hq.y, i));
+		const int mi = EXCL == 3 ? __builtin_amdgcn_readlane(hm, i) : -1;
+		int m = 0; // accepted in this pass
+#pragma unroll
+		for (int r = 0; r < NR; r++) {
+			if (r >= nr)
+				continue;
+			const int r2q = sepk_r2q(make_uint2(q.x, q.y & 0xffffu), cq[r]);
+			// the lanes that hold a candidate: the others' records and
+			// indices are left over and must reach nothing below
+			const unsigned long long held = r == nr - 1 ? some : ~0ull;
+			unsigned long long take = __ballot(r2q < qt.lo2) & held;
+			const unsigned long long near = __ballot(r2q <= qt.hi2) & held & ~take;
+			if (near)
+				take |= sepk_near_test(s, g, qt, near, q, W.cq + 64 * r + lane, t, cj[r]);
+			take &= __ballot(cj[r] != t); // not the atom itself
+			if (EXCL == 3) {
+				if (mi != -1)
+					take &= __ballot(cm[r] != mi);
+			}
+			if (__builtin_amdgcn_inverse_ballot_w64(take))
+				(W.row + m)[sepk_rank(take)] = cj[r];
+			m += __popcll(take);
+		}
+		sepk_wave_lds();
+		if (EXCL == 2) {
+			// drop the bonded ones from the row, in place and in order
+			int keep = 0;
+			for (int b = 0; b < m; b += 64) {
+				const int j = W.row[min(b + lane, m - 1)];
+				const bool ok = b + lane < m && sepk_keep_bonded(s, g, t, j, npad);
+				const unsigned long long in = __ballot(ok);
+				sepk_wave_lds();
+				if (ok)
+					(W.row + keep)[sepk_rank(in)] = j;
+				keep += __popcll(in);
+				sepk_wave_lds();
+			}
+			m = keep;
+		}
+		const int e0 = __builtin_amdgcn_readlane(cnt, i), e1 = e0 + m;
+		if (last && e0 == 0) {
+			// the whole list at once (up to 256 entries a store)
+			if (lane < SEPK_PAD)
+				W.row[m + lane] = phantom;
+			sepk_wave_lds();
+			int *list = nbr + (size_t)t * SEPK_PAD + lslot;
+			const int end = min(m, cap);
+			for (int b = lent; b < end + lane % SEPK_SUB; b += 64 * SEPK_BATCH) {
+				const int *w = W.row + b;
+				*(int4 *)list = make_int4(w[0], w[SEPK_SUB], w[2 * SEPK_SUB], w[3 * SEPK_SUB]);
+				list += 16 * SEPK_PAD * npad;
+			}
+		} else {
+			const int end = min(last ? (e1 + SEPK_PAD - 1) / SEPK_PAD * SEPK_PAD : e1, cap);
+			for (int e = e0 + lane; e < end; e += 64)
+				nbr[sepk_entry(e, t, npad)] = e < e1 ? W.row[e - e0] : phantom;
+		}
+		sepk_wave_lds();
+		sepk_writelane(cnt, e1, i);
+	}
+}
+
+// a / b for 0 <= a < 2^31 and b > 0 from ib = 1 / b: (a + 1/2) / b is at
+// least 1 / (2 b) from a whole number, the product's error below 2^-20 / b.
+__device__ __forceinline__ int sepk_quotient(int a, double ib)
+{
+	return (int)(((double)a + 0.5) * ib);
+}
+
+// Segment of lane l < 18 of cell c's stencil: cells next to each other along
+// x hold consecutive atoms, so the three of a row are one segment, or two
+// where the box ends between them (lanes 2 r and 2 r + 1 take row r, in
+// stencil order); lane 18: the cell itself.  js, len: first atom, atoms.
+__device__ __forceinline__ void sepk_build_segment(const sepdev_grid &g, const sepk_qtest &qt,
+						   int c, const int *start, int &js, int &len)
+{
+	const int lane = threadIdx.x & 63;
+	js = len = 0;
+	if (lane > 18)
+		return;
+	const int n0 = g.n[0], n1 = g.n[1], n2 = g.n[2];
+	const int zy = sepk_quotient(c, qt.icell[0]), cz = sepk_quotient(zy, qt.icell[1]);
+	const int cx = c - zy * n0, cy = zy - cz * n1;
+	int row = c, xa = 0, xb = 0;
+	if (lane < 18) {
+		const int r = lane >> 1;
+		int y = cy + r % 3 - 1, z = cz + r / 3 - 1;
+		y += y < 0 ? n1 : y >= n1 ? -n1 : 0;
+		z += z < 0 ? n2 : z >= n2 ? -n2 : 0;
+		row = (y + z * n1) * n0;
+		xa = cx - 1; // cells xa .. xb
+		xb = cx + 1;
+		if (xa < 0 || xb >= n0) {
+			const bool two = xb >= n0; // two cells before the end
+			xa = lane & 1 ? 0 : two ? n0 - 2 : n0 - 1;
+			xb = lane & 1 ? (two ? 0 : 1) : n0 - 1;
+		} else if (lane & 1) {
+			return;
+		}
+	}
+	js = start[row + xa];
+	len = start[row + xb + 1] - js;
+}
+
+// Quantized build of home atoms tb + i, i the bits of mine, when some atom
+// lies outside the box: the same segments, the reference's FP64 test of every candidate,
+// the accepted ones stored as they come (rare: an atom at x == L exactly, or
+// a starting configuration that reaches outside).
+template <int EXCL>
+__device__ void sepk_build_outside(int js, int len, const sepk_state &s, const sepdev_grid &g,
+				   int tb, unsigned long long mine, long npad, int cap,
+				   int phantom, int *nbr, int &cnt)
+{
+	const int lane = threadIdx.x & 63;
+	for (; mine; mine &= mine - 1ull) {
+		const int t = tb + __builtin_ctzll(mine);
+		const sepk_pos pi = sepk_at(s.pos, (unsigned)t);
+		const int mi = EXCL == 3 ? sepk_at(s.mol, (unsigned)t) : -1;
+		int m = 0;
+		for (int o = 0; o < 18; o++) {
+			const int n = __builtin_amdgcn_readlane(len, o);
+			for (int q0 = 0; q0 < n; q0 += 64) {
+				const int q = q0 + lane;
+				const int j = __builtin_amdgcn_readlane(js, o) + min(q, n - 1);
+				const sepk_pos pj = sepk_at(s.pos, (unsigned)j);
+				const double dx = sepk_wrap(pi.x - pj.x, g.L[0]);
+				const double dy = sepk_wrap(pi.y - pj.y, g.L[1]);
+				const double dz = sepk_wrap(pi.z - pj.z, g.L[2]);
+				bool in = q < n && j != t && dx * dx + dy * dy + dz * dz < g.rlist2;
+				if (EXCL == 3 && mi != -1)
+					in = in && sepk_at(s.mol, (unsigned)j) != mi;
+				if (EXCL == 2 && in)
+					in = sepk_keep_bonded(s, g, t, j, npad);
+				const unsigned long long take = __ballot(in);
+				const int e = m + sepk_rank(take);
+				if (in && e < cap)
+					nbr[sepk_entry(e, t, npad)] = j;
+				m += __popcll(take);
+			}
+		}
+		const int pad = min((m + SEPK_PAD - 1) / SEPK_PAD * SEPK_PAD, cap);
+		if (m + lane < pad)
+			nbr[sepk_entry(m + lane, t, npad)] = phantom;
+		sepk_writelane(cnt, m, t - tb);
+	}
+}
+
+// The wave's candidates for home atoms tb + i, i the bits of mine (lane i
+// holds the record of atom tb + i): those of the stencil's T atoms that come
+// within the list cutoff of the atoms' bounding box (in order, through the
+// wave's LDS), sepk_qwave::CAP at a time.
+// Segment o of the stencil (the bits of used) starts at candidate pre of the
+// wave's T, its atom k at k + off: lane o holds pre and off.
+template <int EXCL>
+__device__ __forceinline__ void sepk_build_home(
+	sepk_qwave<EXCL> &W, unsigned used, int pre, int off, int T, const sepk_state &s,
+	const sepdev_grid &g, const sepk_qtest &qt, int tb, unsigned long long mine, uint2 hq,
+	int hm, long npad, int cap, int phantom, int *nbr, int &cnt)
+{
+	constexpr int NR = sepk_qwave<EXCL>::NR, CAP = sepk_qwave<EXCL>::CAP;
+	const int lane = threadIdx.x & 63;
+	// the box of the atoms: centre and half edges (rounded up)
+	const sepk_short2 zero = {0, 0};
+	sepk_short2 cxy, hxy, cz, hz;
+	{
+		typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+		// the other lanes stand in for the first of the atoms
+		const int one = __builtin_ctzll(mine);
+		const bool in = mine >> lane & 1ull;
+		const unsigned x1 = (unsigned)__builtin_amdgcn_readlane((int)hq.x, one);
+		const unsigned y1 = (unsigned)__builtin_amdgcn_readlane((int)hq.y, one);
+		us2 axy = __builtin_bit_cast(us2, in ? hq.x : x1), bxy = axy;
+		us2 az = __builtin_bit_cast(us2, (in ? hq.y : y1) & 0xffffu), bz = az;
+		for (int o = 32; o > 0; o >>= 1) {
+			const unsigned p = __shfl_xor(__builtin_bit_cast(unsigned, axy), o, 64);
+			const unsigned q = __shfl_xor(__builtin_bit_cast(unsigned, bxy), o, 64);
+			const unsigned u = __shfl_xor(__builtin_bit_cast(unsigned, az), o, 64);
+			const unsigned v = __shfl_xor(__builtin_bit_cast(unsigned, bz), o, 64);
+			axy = __builtin_elementwise_min(axy, __builtin_bit_cast(us2, p));
+			bxy = __builtin_elementwise_max(bxy, __builtin_bit_cast(us2, q));
+			az = __builtin_elementwise_min(az, __builtin_bit_cast(us2, u));
+			bz = __builtin_elementwise_max(bz, __builtin_bit_cast(us2, v));
+		}
+		const unsigned a = __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, axy));
+		const unsigned b = __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, bxy));
+		const int a2 = __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, az));
+		const int b2 = __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, bz));
+		const int a0 = (int)(a & 0xffffu), a1 = (int)(a >> 16);
+		const int b0 = (int)(b & 0xffffu), b1 = (int)(b >> 16);
+		cxy = sepk_short2{(short)((a0 + b0) >> 1), (short)((a1 + b1) >> 1)};
+		hxy = sepk_short2{(short)min((b0 - a0 + 1) >> 1, 32767), (short)min((b1 - a1 + 1) >> 1, 32767)};
+		cz = sepk_short2{(short)((a2 + b2) >> 1), 0};
+		hz = sepk_short2{(short)min((b2 - a2 + 1) >> 1, 32767), 0};
+	}
+	int ko = 0, kn = 0; // this segment's offset, the next one's first candidate
+	int nf = 0;
+	for (int k0 = 0;; k0 += CAP) {
+		const bool end = k0 >= T;
+		int jq[NR], mq[NR], nb = 0;
+		uint2 cq[NR];
+		unsigned long long in[NR];
+		if (!end) {
+			// the atom of every lane's candidate: the segment is followed
+			// along the rounds, the lanes past its end moved to the next
+#pragma unroll
+			for (int r = 0; r < NR; r++) {
+				const int k = min(k0 + 64 * r + lane, T - 1);
+				jq[r] = k + ko;
+				while (kn <= k0 + 64 * r + 63) { // the next segment starts in this round
+					const int o = __builtin_ctz(used);
+					ko = __builtin_amdgcn_readlane(off, o);
+					jq[r] = k >= kn ? k + ko : jq[r];
+					used &= used - 1u;
+					kn = used ? __builtin_amdgcn_readlane(pre, __builtin_ctz(used)) : INT_MAX;
+				}
+			}
+			int4 pq[NR];
+#pragma unroll
+			for (int r = 0; r < NR; r++) {
+				pq[r] = sepk_at(s.qpos, (unsigned)jq[r]);
+				if (EXCL == 3)
+					mq[r] = sepk_at(s.mol, (unsigned)jq[r]);
+			}
+#pragma unroll
+			for (int r = 0; r < NR; r++) {
+				// the distance to the box is no larger than to any atom in it,
+				// in the same units
+				cq[r] = sepk_quant21(pq[r]);
+				sepk_short2 dxy = __builtin_bit_cast(sepk_short2, cq[r].x) - cxy;
+				sepk_short2 dz = __builtin_bit_cast(sepk_short2, (unsigned)pq[r].z >> 16) - cz;
+				dxy = __builtin_elementwise_max(dxy, sepk_sub_sat(zero, dxy));
+				dz = __builtin_elementwise_max(dz, sepk_sub_sat(zero, dz));
+				dxy = __builtin_elementwise_max(sepk_sub_sat(dxy, hxy), zero);
+				dz = __builtin_elementwise_max(sepk_sub_sat(dz, hz), zero);
+				const int d2 = __builtin_amdgcn_sdot2(
+					dz, dz, __builtin_amdgcn_sdot2(dxy, dxy, 0, true), true);
+				in[r] = __ballot(d2 <= qt.hi2 && k0 + 64 * r + lane < T);
+				nb += __popcll(in[r]);
+			}
+		}
+		if (end || nf + nb > CAP) {
+			sepk_wave_lds();
+			sepk_build_pass<EXCL>(W, s, g, qt, nf, tb, mine, hq, hm, npad, cap, phantom, end,
+					      nbr, cnt);
+			if (end)
+				return;
+			nf = 0;
+		}
+#pragma unroll
+		for (int r = 0; r < NR; r++) {
+			if (__builtin_amdgcn_inverse_ballot_w64(in[r])) {
+				const int f = nf + sepk_rank(in[r]);
+				W.cq[f] = cq[r];
+				W.cj[f] = jq[r];
+				if (EXCL == 3)
+					W.cm[f] = mq[r];
+			}
+			nf += __popcll(in[r]);
+		}
+	}
+}
+
+// FP64 build, one round: the 64 staged candidates [q0, q0 + 64) of a chunk
+// of kn against the wave's home atoms i = wid, wid + 4, ... < hn, storing the
+// accepted ones to their lists, each at the atom's length so far plus its
+// rank among the passing lanes.  cnt and cap as above.
+// SH: some stencil target of the cell lies across the box (shift adds).
+template <bool SHIFT, bool SH, int EXCL>
 __device__ __forceinline__ void sepk_build_round(
-	sepk_build_lds &L, const sepk_state &s, const sepdev_grid &g, const sepk_qtest &qt,
-	int q0, int kn, long tbase, int hn, long npad, int cap, int *nbr, int &cnt)
+	sepk_build_lds &L, const sepk_state &s, const sepdev_grid &g, int q0, int kn, long tbase,
+	int hn, long npad, int cap, int *nbr, int &cnt)
 {
 	const int lane = threadIdx.x & 63;
 	const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); // wave-uniform
 	const int q = min(q0 + lane, kn - 1);
-	// lanes past the staged candidates take bounds that no distance meets
+	// lanes past the staged candidates take a bound that no distance meets
 	const bool valid = lane < kn - q0;
-	// NP32 (sepk_np32): 32-bit byte offsets with a full-rate 24-bit multiply
-	const unsigned npad16 = (unsigned)npad * SEPK_PAD;
 	const int j = L.cj[q];
 	const int o = L.co[q];
 	const int rule = L.segrule[o];
@@ -625,24 +1014,11 @@ __device__ __forceinline__ void sepk_build_round(
 	const unsigned long long home = __ballot(rule >= 0);
 	// original index of a home-cell candidate, for the GT / LT rules
 	const int oj = !SHIFT && rule >= SEPDEV_RULE_GT ? s.orig[j] : 0;
-	uint2 cq = make_uint2(0u, 0u);
-	double px = 0.0, py = 0.0, pz = 0.0;
-	if (QNT) {
-		cq = L.cq[q];
-	} else {
-		px = L.cx[q];
-		py = L.cy[q];
-		pz = L.cz[q];
-	}
-	int lo2 = valid ? qt.lo2 : INT_MIN, hi2 = valid ? qt.hi2 : -1;
-	double rl2 = valid ? g.rlist2 : -1.0;
-	// the home atom i's own candidate is the one with j - tbase == i
-	int jrel = j - (int)tbase;
-	// held in registers as they are: the compiler would otherwise fold the
-	// selects back into every test of the loop below
-	asm volatile("" : "+v"(lo2), "+v"(hi2), "+v"(rl2), "+v"(jrel));
+	const double px = L.cx[q], py = L.cy[q], pz = L.cz[q];
+	const double rl2 = valid ? g.rlist2 : -1.0;
+	const int jrel = j - (int)tbase; // the home atom i's own candidate has jrel == i
 	double sx = 0.0, sy = 0.0, sz = 0.0;
-	if (SH && !QNT) {
+	if (SH) {
 		sx = L.segsh[o][0];
 		sy = L.segsh[o][1];
 		sz = L.segsh[o][2];
@@ -651,38 +1027,23 @@ __device__ __forceinline__ void sepk_build_round(
 	for (int i = wid; i < hn; i += SEPK_BT / 64, kk++) {
 		const long t = tbase + i;
 		const int t32 = (int)t;
-		unsigned long long take;
-		if (QNT) {
-			const int r2q = sepk_r2q(L.hq[i], cq);
-			take = __ballot(r2q < lo2);
-			const unsigned long long near = __ballot(r2q <= hi2) & ~take;
-			if (near) {
-				// the reference's FP64 test, with the target cell's shift
-				const double dx = L.hx[i] - L.cx[q] + L.segsh[o][0];
-				const double dy = L.hy[i] - L.cy[q] + L.segsh[o][1];
-				const double dz = L.hz[i] - L.cz[q] + L.segsh[o][2];
-				const double r2 = dx * dx + dy * dy + dz * dz;
-				take |= __ballot(r2 < g.rlist2) & near;
+		double dx, dy, dz;
+		if (SHIFT) {
+			dx = L.hx[i] - px;
+			dy = L.hy[i] - py;
+			dz = L.hz[i] - pz;
+			if (SH) {
+				dx += sx;
+				dy += sy;
+				dz += sz;
 			}
 		} else {
-			double dx, dy, dz;
-			if (SHIFT) {
-				dx = L.hx[i] - px;
-				dy = L.hy[i] - py;
-				dz = L.hz[i] - pz;
-				if (SH) {
-					dx += sx;
-					dy += sy;
-					dz += sz;
-				}
-			} else {
-				dx = sepk_wrap(L.hx[i] - px, g.L[0]);
-				dy = sepk_wrap(L.hy[i] - py, g.L[1]);
-				dz = sepk_wrap(L.hz[i] - pz, g.L[2]);
-			}
-			const double r2 = dx * dx + dy * dy + dz * dz;
-			take = __ballot(r2 < rl2);
+			dx = sepk_wrap(L.hx[i] - px, g.L[0]);
+			dy = sepk_wrap(L.hy[i] - py, g.L[1]);
+			dz = sepk_wrap(L.hz[i] - pz, g.L[2]);
 		}
+		const double r2 = dx * dx + dy * dy + dz * dz;
+		unsigned long long take = __ballot(r2 < rl2);
 		if (SHIFT) {
 			// the 27-cell stencil reaches the home cell only through
 			// offset 0: drop the atom itself
@@ -701,48 +1062,30 @@ __device__ __forceinline__ void sepk_build_round(
 		}
 		if (EXCL == 2 /* SEP_EXCL_BONDED */ && take) {
 			bool ok = false;
-			if (__builtin_amdgcn_inverse_ballot_w64(take)) {
-				const int oi = L.horig[i];
-				const int oj2 = s.orig[j];
-				int sh = sepk_share(s.partners, npad, t, j, 0, 10, oi, oj2);
-				if (g.bonded_all)
-					sh += sepk_share(s.partners, npad, t, j, 10, 10, oi, oj2) +
-					      sepk_share(s.partners, npad, t, j, 20, 20, oi, oj2);
-				// rule 2 is the Coulomb brute-force test of
-				// source/sepcoulomb.c:44, which excludes only when
-				// exactly one kind of partnership holds
-				ok = g.bonded_all == 2 ? sh != 1 : sh == 0;
-			}
+			if (__builtin_amdgcn_inverse_ballot_w64(take))
+				ok = sepk_keep_bonded(s, g, t, j, npad);
 			take = __ballot(ok);
 		}
 		if (take) {
 			const int e0 = __builtin_amdgcn_readlane(cnt, kk);
 			const int e = (int)__builtin_amdgcn_mbcnt_hi(
 				(unsigned)(take >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)take, (unsigned)e0));
-			if (__builtin_amdgcn_inverse_ballot_w64(take) && e < cap) {
-				if (NP32) {
-					// the atom's first slot as a scalar base, a 32-bit byte
-					// offset (sepk_entry)
-					const unsigned off = __umul24((unsigned)e / SEPK_PAD, npad16) +
-							     ((unsigned)e % SEPK_SUB) * SEPK_BATCH +
-							     ((unsigned)e / SEPK_SUB) % SEPK_BATCH;
-					*(int *)((char *)(nbr + (size_t)t * SEPK_PAD) + (size_t)(off * 4u)) = j;
-				} else {
-					nbr[sepk_entry(e, t, npad)] = j;
-				}
-			}
+			if (__builtin_amdgcn_inverse_ballot_w64(take) && e < cap)
+				nbr[sepk_entry(e, t, npad)] = j;
 			sepk_writelane(cnt, e0 + __popcll(take), kk);
 		}
 	}
 }
 
-// Slice `slice` of `nslice` of cell c: its home atoms
-// [h * slice / nslice, h * (slice + 1) / nslice), SEPK_BHOME at a time.
+// FP64 build: slice `slice` of `nslice` of cell c, its home atoms
+// [h * slice / nslice, h * (slice + 1) / nslice), SEPK_BHOME at a time.  The
+// stencil cells' segments are staged in LDS SEPK_BCHUNK candidates at a
+// time, the home atoms beside them; each wave owns every fourth home atom.
 template <bool SHIFT, int EXCL>
 __device__ __forceinline__ void sepk_build_cell(
 	sepk_build_lds &L, const sepk_state &s, long c, int slice, int nslice,
-	const int *start, const sepdev_grid &g, const sepk_qtest &qt, long npad, int cap,
-	int phantom, int *nbr, int *cnt, sepdev_sys *sys, int &mymax)
+	const int *start, const sepdev_grid &g, long npad, int cap, int phantom, int *nbr,
+	int *cnt, sepdev_sys *sys, int &mymax)
 {
 	const int lane = threadIdx.x & 63;
 	const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); // wave-uniform
@@ -754,8 +1097,9 @@ __device__ __forceinline__ void sepk_build_cell(
 		bool shifted = false;
 		if (lane < g.noff) {
 			const int o = lane;
-			const int cxi = (int)(c % n0), cyi = (int)((c / n0) % n1);
-			const int czi = (int)(c / ((long)n0 * n1));
+			const unsigned cu = (unsigned)c, zy = cu / (unsigned)n0;
+			const int cxi = (int)(cu - zy * (unsigned)n0), czi = (int)(zy / (unsigned)n1);
+			const int cyi = (int)zy - czi * n1;
 			const int ux = cxi + g.off[o][0], uy = cyi + g.off[o][1], uz = czi + g.off[o][2];
 			const int tx = sepk_mod(ux, n0), ty = sepk_mod(uy, n1), tz = sepk_mod(uz, n2);
 			const long c2 = tx + (long)ty * n0 + (long)tz * n0 * n1;
@@ -794,8 +1138,6 @@ __device__ __forceinline__ void sepk_build_cell(
 	// h < 2^24 atoms a cell and nslice <= 64: 32-bit products
 	const int hbeg = nslice == 1 ? 0 : (int)((unsigned)(h * slice) / (unsigned)nslice);
 	const int hend = nslice == 1 ? h : (int)((unsigned)(h * (slice + 1)) / (unsigned)nslice);
-	const bool qnt = SHIFT && qt.on;
-	const bool np32 = sepk_np32(npad, cap);
 	for (int hb = hbeg; hb < hend; hb += SEPK_BHOME) {
 		const int hn = min(hend - hb, SEPK_BHOME);
 		int len = 0; // lane kk: list length of the wave's kk-th home atom
@@ -814,7 +1156,7 @@ __device__ __forceinline__ void sepk_build_cell(
 				const int k = k0 + q;
 				int o = 0; // the last segment starting at or before k
 #pragma unroll
-				for (int step = 32; step > 0; step >>= 1)
+				for (int step = 16; step > 0; step >>= 1)
 					if (o + step < g.noff && L.segpre[o + step] <= k)
 						o += step;
 				oq[r] = q < kn && q < SEPK_BCHUNK ? o : -1;
@@ -837,8 +1179,6 @@ __device__ __forceinline__ void sepk_build_cell(
 					L.cx[q] = pq[r].x;
 					L.cy[q] = pq[r].y;
 					L.cz[q] = pq[r].z;
-					if (qnt)
-						L.cq[q] = sepk_quantize(pq[r], qt.scale);
 					L.cj[q] = jq[r];
 					L.co[q] = (unsigned char)oq[r];
 					if (EXCL == 3)
@@ -852,26 +1192,18 @@ __device__ __forceinline__ void sepk_build_cell(
 					L.hx[i] = p.x;
 					L.hy[i] = p.y;
 					L.hz[i] = p.z;
-					if (qnt)
-						L.hq[i] = sepk_quantize(p, qt.scale);
 					L.horig[i] = sepk_at(s.orig, t);
 					L.hmol[i] = EXCL == 3 ? sepk_at(s.mol, t) : -1;
 				}
 			__syncthreads();
 			const long tb = hs + hb;
 			for (int q0 = 0; q0 < kn; q0 += 64) {
-				if (qnt && np32)
-					sepk_build_round<true, false, EXCL, true, true>(L, s, g, qt, q0, kn, tb,
-											hn, npad, cap, nbr, len);
-				else if (qnt)
-					sepk_build_round<true, false, EXCL, true, false>(L, s, g, qt, q0, kn, tb,
-											 hn, npad, cap, nbr, len);
-				else if (SHIFT && anyshift)
-					sepk_build_round<SHIFT, true, EXCL, false, false>(L, s, g, qt, q0, kn, tb,
-											  hn, npad, cap, nbr, len);
+				if (SHIFT && anyshift)
+					sepk_build_round<SHIFT, true, EXCL>(L, s, g, q0, kn, tb, hn, npad, cap,
+									    nbr, len);
 				else
-					sepk_build_round<SHIFT, false, EXCL, false, false>(L, s, g, qt, q0, kn, tb,
-											   hn, npad, cap, nbr, len);
+					sepk_build_round<SHIFT, false, EXCL>(L, s, g, q0, kn, tb, hn, npad, cap,
+									     nbr, len);
 			}
 		}
 		// lane kk of each wave: its home atom's count and length bound
@@ -900,39 +1232,17 @@ __device__ __forceinline__ void sepk_build_cell(
 	}
 }
 
-// Persistent over (cell, slice) items, nslice per cell; the largest list
-// length goes to sys->max_full by an atomic maximum (order-independent, so
-// the result is deterministic).  The permuted state of the workgroup's cells
-// goes home at the end, in one batch, so its memory round trip is paid once.
-template <int EXCL>
-__global__ __launch_bounds__(SEPK_BT) __attribute__((amdgpu_waves_per_eu(EXCL == 2 ? 4 : 7))) void k_build(
-	sepk_state s, sepk_state home, const int *start, sepdev_grid g, long ncell, int nslice,
-	long n, long npad, int cap, int *nbr, int *cnt, sepdev_sys *sys, int conditional,
-	int has_partners)
+// End of a build kernel: the permuted state of the workgroup's share of the
+// cells goes home (in one batch, so its memory round trip is paid once; one
+// wave per cell, SEPK_BT / 64 cells at a time), and the largest list length to
+// sys->max_full by an atomic maximum (order-independent, so the result is
+// deterministic).
+__device__ __forceinline__ void sepk_build_end(const sepk_state &s, const sepk_state &home,
+					       const int *start, long ncell, long npad,
+					       int has_partners, int mymax, sepdev_sys *sys)
 {
-	if ((conditional && sys->neighb_flag == 0) || sys->frozen)
-		return;
-	__shared__ sepk_build_lds L;
-	const bool shift = g.shift_ok && sys->unclean == 0;
-	const sepk_qtest qt = sepk_qtest_of(g, shift);
 	const long per = gridDim.x / SEPK_NXCD;
 	const long xcd = blockIdx.x % SEPK_NXCD, k = blockIdx.x / SEPK_NXCD;
-	const long nitem = ncell * nslice;
-	const long iper = (nitem + SEPK_NXCD - 1) / SEPK_NXCD;
-	const long ilo = xcd * iper, ihi = min(ilo + iper, nitem);
-	int mymax = 0;
-	for (long it = ilo + k; it < ihi; it += per) {
-		// items < 2^31 (the host bounds nslice by the atoms a cell)
-		const long c = nslice == 1 ? it : (long)((unsigned)it / (unsigned)nslice);
-		const int sl = (int)(it - c * nslice);
-		if (shift)
-			sepk_build_cell<true, EXCL>(L, s, c, sl, nslice, start, g, qt, npad, cap,
-						    (int)n, nbr, cnt, sys, mymax);
-		else
-			sepk_build_cell<false, EXCL>(L, s, c, sl, nslice, start, g, qt, npad, cap,
-						     (int)n, nbr, cnt, sys, mymax);
-	}
-	// one wave per cell, SEPK_BT / 64 cells at a time
 	const long cper = (ncell + SEPK_NXCD - 1) / SEPK_NXCD;
 	const long lo = xcd * cper, hi = min(lo + cper, ncell);
 	const int wv = threadIdx.x >> 6, ln = threadIdx.x & 63;
@@ -947,11 +1257,138 @@ __global__ __launch_bounds__(SEPK_BT) __attribute__((amdgpu_waves_per_eu(EXCL ==
 	if (threadIdx.x == 0)
 		bmax = 0;
 	__syncthreads();
-	if ((threadIdx.x & 63) == 0)
+	if (ln == 0)
 		atomicMax(&bmax, mymax);
 	__syncthreads();
 	if (threadIdx.x == 0 && bmax > 0)
 		atomicMax(&sys->max_full, bmax);
+}
+
+// Quantized build, persistent over (cell, slice) items, a wave an item
+// (nslice per cell): no wave waits for another, so the memory round trips of
+// one (cell starts, candidates) hide behind the tests of the others.  A slice
+// takes the cell's atoms by their rank in x: a slab whose bounding box only
+// about 45 % of the stencil's candidates come near (two slabs a cell; a third
+// with four, but the walk over the candidates is then shared by too few).
+// Neither the order of the atoms nor that of the lists depends on the slices.
+//
+// What bounds the build is instruction issue and latency; its bytes are few.
+// N = 256000, per rebuild: 190 us with a workgroup a cell, candidates shared
+// through LDS, every one tested and each round's handful of accepted ones
+// stored at once (a partly filled store and 9 address instructions a round);
+// 143 with the accepted ones collected in an LDS row; 138 with the bounding
+// box; 130 with a wave an item and slabs of about 11 atoms (a few us more with 6
+// and with the whole cell).
+template <int EXCL>
+__global__ __launch_bounds__(SEPK_BT) __attribute__((amdgpu_waves_per_eu(EXCL == 2 ? 4 : 7))) void k_build_q(
+	sepk_state s, sepk_state home, const int *start, sepdev_grid g, sepk_qtest qt, long ncell,
+	int nslice, long n, long npad, int cap, int *nbr, int *cnt, sepdev_sys *sys,
+	int conditional, int has_partners)
+{
+	if ((conditional && sys->neighb_flag == 0) || sys->frozen)
+		return;
+	__shared__ sepk_qwave<EXCL> WV[SEPK_BT / 64];
+	const int lane = threadIdx.x & 63;
+	const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); // wave-uniform
+	sepk_qwave<EXCL> &W = WV[wid];
+	const bool clean = sys->unclean == 0;
+	// items < 2^31 (the host bounds nslice by the atoms a cell)
+	const unsigned per = gridDim.x / SEPK_NXCD;
+	const unsigned xcd = blockIdx.x % SEPK_NXCD, k = blockIdx.x / SEPK_NXCD;
+	const unsigned nitem = (unsigned)ncell * (unsigned)nslice;
+	const unsigned iper = (nitem + SEPK_NXCD - 1) / SEPK_NXCD;
+	const unsigned ilo = xcd * iper, ihi = min(ilo + iper, nitem);
+	int mymax = 0;
+	for (unsigned it = ilo + k * (SEPK_BT / 64) + wid; it < ihi; it += per * (SEPK_BT / 64)) {
+		const int c = sepk_quotient((int)it, qt.islice);
+		const int sl = (int)it - c * nslice;
+		int js, len;
+		sepk_build_segment(g, qt, c, start, js, len);
+		const int hs = __builtin_amdgcn_readlane(js, 18), h = __builtin_amdgcn_readlane(len, 18);
+		if (h == 0)
+			continue;
+		int x = lane < 18 ? len : 0; // inclusive scan over the segments
+		for (int d = 1; d < 32; d <<= 1) {
+			const int y = __shfl_up(x, d, 64);
+			if (lane >= d)
+				x += y;
+		}
+		const unsigned used = (unsigned)__ballot(lane < 18 && len > 0);
+		const int T = __builtin_amdgcn_readlane(x, 17);
+		// the cell's atoms in nb batches of at most 64 (one, unless it is
+		// very full), the cell's slices shared out among the batches: this
+		// one is slab `sub` of `nsub` of its batch (or whole batches, every
+		// nslice-th, where there are more batches than slices)
+		const int nb = (h + SEPK_BHOME - 1) / SEPK_BHOME;
+		const bool shared = nb <= nslice;
+		int b = shared ? (int)((unsigned)(sl * nb) / (unsigned)nslice) : sl;
+		for (; b < nb; b += shared ? nb : nslice) {
+			const int s0 = shared ? (b * nslice + nb - 1) / nb : sl;
+			const int s1 = shared ? ((b + 1) * nslice + nb - 1) / nb : sl + 1;
+			const int sub = sl - s0, nsub = s1 - s0;
+			const int ha = (int)((unsigned long)h * b / nb);
+			const int hn = (int)((unsigned long)h * (b + 1) / nb) - ha, tb = hs + ha;
+			const unsigned ti = (unsigned)(tb + min(lane, hn - 1));
+			const uint2 hq = sepk_quant21(sepk_at(s.qpos, ti));
+			const int hm = EXCL == 3 ? sepk_at(s.mol, ti) : -1;
+			unsigned long long mine = hn < 64 ? ~(~0ull << hn) : ~0ull;
+			if (nsub > 1) {
+				// the slab's atoms by their rank in x
+				const int key = (int)((hq.x & 0xffffu) << 6) | lane;
+				int rank = 0;
+				for (int j = 0; j < hn; j++)
+					rank += __builtin_amdgcn_readlane(key, j) < key;
+				mine &= __ballot(rank >= hn * sub / nsub && rank < hn * (sub + 1) / nsub);
+				if (!mine)
+					continue;
+			}
+			int m = 0; // lane i: list length of home atom i
+			if (clean)
+				sepk_build_home<EXCL>(W, used, x - len, js - (x - len), T, s, g, qt, tb, mine, hq,
+						      hm, npad, cap, (int)n, nbr, m);
+			else
+				sepk_build_outside<EXCL>(js, len, s, g, tb, mine, npad, cap, (int)n, nbr, m);
+			if (mine >> lane & 1ull) {
+				cnt[tb + lane] = m < cap ? m : cap;
+				if (m > cap)
+					sepk_set_error(sys, SEP_GPU_ENEIGHB);
+				mymax = max(mymax, m);
+			}
+		}
+	}
+	sepk_build_end(s, home, start, ncell, npad, has_partners, mymax, sys);
+}
+
+// FP64 build, persistent over (cell, slice) items, nslice per cell, a
+// workgroup an item.
+template <int EXCL>
+__global__ __launch_bounds__(SEPK_BT) __attribute__((amdgpu_waves_per_eu(EXCL == 2 ? 4 : 7))) void k_build(
+	sepk_state s, sepk_state home, const int *start, sepdev_grid g, sepk_qtest, long ncell,
+	int nslice, long n, long npad, int cap, int *nbr, int *cnt, sepdev_sys *sys,
+	int conditional, int has_partners)
+{
+	if ((conditional && sys->neighb_flag == 0) || sys->frozen)
+		return;
+	__shared__ sepk_build_lds L;
+	const bool shift = g.shift_ok && sys->unclean == 0;
+	const long per = gridDim.x / SEPK_NXCD;
+	const long xcd = blockIdx.x % SEPK_NXCD, k = blockIdx.x / SEPK_NXCD;
+	const long nitem = ncell * nslice;
+	const long iper = (nitem + SEPK_NXCD - 1) / SEPK_NXCD;
+	const long ilo = xcd * iper, ihi = min(ilo + iper, nitem);
+	int mymax = 0;
+	for (long it = ilo + k; it < ihi; it += per) {
+		// items < 2^31 (the host bounds nslice by the atoms a cell)
+		const long c = nslice == 1 ? it : (long)((unsigned)it / (unsigned)nslice);
+		const int sl = (int)(it - c * nslice);
+		if (shift)
+			sepk_build_cell<true, EXCL>(L, s, c, sl, nslice, start, g, npad, cap, (int)n, nbr,
+						    cnt, sys, mymax);
+		else
+			sepk_build_cell<false, EXCL>(L, s, c, sl, nslice, start, g, npad, cap, (int)n, nbr,
+						     cnt, sys, mymax);
+	}
+	sepk_build_end(s, home, start, ncell, npad, has_partners, mymax, sys);
 }
 
 // ---- host side --------------------------------------------------------------
@@ -1060,6 +1497,10 @@ extern "C" int sepdev_build_list(sepdev *d, const sepdev_grid *gp, int condition
 	}
 	if ((rc = sepk_claim_region(d, SEPK_R_BUILD)))
 		return rc;
+	sepk_qtest qt;
+	const bool qnt = sepk_qtest_of(g, qt);
+	if (qnt && (rc = sepk_fresh_qpos(d, g.L)))
+		return rc;
 
 	sepk_state &cur = d->s[0];   // current state, fixed addresses
 	sepk_state &spare = d->s[1]; // receives the permuted order
@@ -1095,27 +1536,36 @@ extern "C" int sepdev_build_list(sepdev *d, const sepdev_grid *gp, int condition
 		d->order_tmp, d->cell_start, cur, spare, d->iperm, ncell, d->npad,
 		d->sys, conditional, hp, d->cell_count);
 	SEPK_LAUNCH_CHECK();
-	// Home atoms of a cell split over nslice workgroups when the cells are
-	// few and full (small boxes, dense molecular systems): at least 16 home
-	// atoms a slice, at most SEPK_BHOME, about 1024 items where cells alone
-	// are fewer.  The lists do not depend on the split.
+	// A cell's atoms in nslice slices (the lists do not depend on the
+	// split).  FP64, a workgroup a slice: one, unless the cells are few and
+	// full: at least 16 atoms a slice, at most SEPK_BHOME, about 1024
+	// slices.  Quantized, a wave a slice: about SEPK_QSLICE atoms, fewer
+	// where there would not be 2048 slices (N = 27000: 37.5 us a step; 38.5
+	// with 4096 slices, 39.4 with a workgroup a cell).
 	const long avg = (d->n + ncell - 1) / ncell;
-	long nslice = (avg + 15) / 16;
-	const long fill = (1024 + ncell - 1) / ncell;
-	if (nslice > fill)
+	const long least = qnt ? (avg + 31) / 32 : (avg + SEPK_BHOME - 1) / SEPK_BHOME;
+	const long most = qnt ? avg : (avg + 15) / 16;
+	const long fill = ((qnt ? 2048 : 1024) + ncell - 1) / ncell;
+	long nslice = qnt ? (avg + SEPK_QSLICE / 2) / SEPK_QSLICE : 1;
+	if (nslice < fill)
 		nslice = fill;
-	if (nslice < (avg + SEPK_BHOME - 1) / SEPK_BHOME)
-		nslice = (avg + SEPK_BHOME - 1) / SEPK_BHOME;
+	if (nslice > most)
+		nslice = most;
+	if (nslice < least)
+		nslice = least;
 	if (nslice < 1)
 		nslice = 1;
 	if (nslice > 64)
 		nslice = 64;
-	long bb = (ncell * nslice + SEPK_NXCD - 1) / SEPK_NXCD * SEPK_NXCD;
+	qt.islice = 1.0 / (double)nslice;
+	const long wgs = qnt ? (ncell * nslice + SEPK_BT / 64 - 1) / (SEPK_BT / 64) : ncell * nslice;
+	long bb = (wgs + SEPK_NXCD - 1) / SEPK_NXCD * SEPK_NXCD;
 	if (bb > SEPK_BGRID)
 		bb = SEPK_BGRID;
-	auto kb = g.opt == 2 ? k_build<2> : g.opt == 3 ? k_build<3> : k_build<0>;
+	auto kb = qnt ? (g.opt == 2 ? k_build_q<2> : g.opt == 3 ? k_build_q<3> : k_build_q<0>)
+		      : (g.opt == 2 ? k_build<2> : g.opt == 3 ? k_build<3> : k_build<0>);
 	const int capb = d->cap_limit > 0 && d->cap_limit < d->cap ? d->cap_limit : d->cap;
-	kb<<<(unsigned)bb, SEPK_BT, 0, d->st>>>(spare, cur, d->cell_start, g, ncell, (int)nslice,
+	kb<<<(unsigned)bb, SEPK_BT, 0, d->st>>>(spare, cur, d->cell_start, g, qt, ncell, (int)nslice,
 						      d->n, d->npad, capb, d->nbr, d->nbr_count,
 						      d->sys, conditional, hp);
 	SEPK_LAUNCH_CHECK();
