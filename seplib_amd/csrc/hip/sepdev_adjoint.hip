@@ -109,12 +109,9 @@ __global__ __launch_bounds__(SEPK_BLOCK) void k_lj_table(
 			}
 		}
 	}
-#pragma unroll
-	for (int o = 1; o < SEPK_SUB; o <<= 1) {
-		fx += __shfl_xor(fx, o, SEPK_WAVE);
-		fy += __shfl_xor(fy, o, SEPK_WAVE);
-		fz += __shfl_xor(fz, o, SEPK_WAVE);
-	}
+	fx = sepk_atom_sum(fx);
+	fy = sepk_atom_sum(fy);
+	fz = sepk_atom_sum(fz);
 	// f stays as it is while the device error word is set
 	if (t < n && sub == 0 && !*s.err) {
 		if (OVERWRITE) {
@@ -127,7 +124,7 @@ __global__ __launch_bounds__(SEPK_BLOCK) void k_lj_table(
 			s.f[2 * npad + t] += fz;
 		}
 	}
-	sepk_block_partial<7>(acc, 0u, partial, lb, rows);
+	sepk_block_partial(acc, partial, lb, rows);
 }
 
 // The adjoint pass: g (3 x npad, device order) in, dL/dx (3 x npad) out, and
@@ -202,18 +199,15 @@ __global__ __launch_bounds__(SEPK_BLOCK) void k_lj_adjoint(
 			}
 		}
 	}
-#pragma unroll
-	for (int o = 1; o < SEPK_SUB; o <<= 1) {
-		hx += __shfl_xor(hx, o, SEPK_WAVE);
-		hy += __shfl_xor(hy, o, SEPK_WAVE);
-		hz += __shfl_xor(hz, o, SEPK_WAVE);
-	}
+	hx = sepk_atom_sum(hx);
+	hy = sepk_atom_sum(hy);
+	hz = sepk_atom_sum(hz);
 	if (t < n && sub == 0) {
 		dldx[t] = hx;
 		dldx[npad + t] = hy;
 		dldx[2 * npad + t] = hz;
 	}
-	sepk_block_partial<2 * SEPK_NPAIR>(gp, 0u, partial, lb, rows);
+	sepk_block_partial(gp, partial, lb, rows);
 }
 
 // One workgroup: column sums of the adjoint's partial rows, fixed order.

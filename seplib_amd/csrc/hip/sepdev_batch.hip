@@ -976,8 +976,14 @@ __global__ __launch_bounds__(SEPB_BLOCK) void k_bstep(sepb_view b, sepb_lj c, co
 				acc[15] = d2;
 			}
 		}
-		sepk_block_partial<SEPB_NV>(acc, 1u << 15, b.partial, td.z, b.prow);
-		__syncthreads(); // sepk_block_partial's LDS is reused by the next tile
+		double sums[SEPB_NV - 1];
+#pragma unroll
+		for (int k = 0; k < SEPB_NV - 1; k++)
+			sums[k] = acc[k];
+		sepk_block_reduce<true>(sums, acc[SEPB_NV - 1], [&](int i, double r) {
+			b.partial[(size_t)i * b.prow + td.z] = r;
+		});
+		__syncthreads(); // its LDS is reused by the next tile
 	}
 }
 

@@ -227,7 +227,7 @@ __global__ __launch_bounds__(SEPK_BLOCK) void k_bond(
 			contrib[3 * (2 * n + 1) + k] = -f[k];
 		}
 	}
-	sepk_block_partial<7>(acc, 0u, partial, blockIdx.x, rows);
+	sepk_block_partial(acc, partial, blockIdx.x, rows);
 }
 
 extern "C" int sepdev_bond(sepdev *d, int type, double lbond, double ks,
@@ -306,7 +306,7 @@ __global__ __launch_bounds__(SEPK_BLOCK) void k_angle(
 			contrib[3 * (3 * n + 2) + k] = fc[k];
 		}
 	}
-	sepk_block_partial<7>(acc, 0u, partial, blockIdx.x, rows);
+	sepk_block_partial(acc, partial, blockIdx.x, rows);
 }
 
 extern "C" int sepdev_angle(sepdev *d, int type, double angle0, double k, int cossq,
@@ -388,7 +388,7 @@ __global__ __launch_bounds__(SEPK_BLOCK) void k_torsion(
 			for (int k = 0; k < 3; k++)
 				contrib[3 * (4 * n + r) + k] = F[r][k];
 	}
-	sepk_block_partial<7>(acc, 0u, partial, blockIdx.x, rows);
+	sepk_block_partial(acc, partial, blockIdx.x, rows);
 }
 
 extern "C" int sepdev_torsion(sepdev *d, int type, const double *g, const double *L,

@@ -75,12 +75,9 @@ __device__ __forceinline__ void sepk_pair_epilogue(
 	double px, double py, double pz, double (&acc)[7], double *f, double *partial,
 	long row, long rows, bool frozen)
 {
-#pragma unroll
-	for (int o = 1; o < SEPK_SUB; o <<= 1) {
-		fx += __shfl_xor(fx, o, SEPK_WAVE);
-		fy += __shfl_xor(fy, o, SEPK_WAVE);
-		fz += __shfl_xor(fz, o, SEPK_WAVE);
-	}
+	fx = sepk_atom_sum(fx);
+	fy = sepk_atom_sum(fy);
+	fz = sepk_atom_sum(fz);
 	if (t < n && sub == 0 && !frozen) {
 		if (OVERWRITE) {
 			f[t] = fx;
@@ -101,7 +98,7 @@ __device__ __forceinline__ void sepk_pair_epilogue(
 		acc[5] = fma(gy, pz, acc[5]);
 		acc[6] = fma(gz, pz, acc[6]);
 	}
-	sepk_block_partial<7>(acc, 0u, partial, row, rows);
+	sepk_block_partial(acc, partial, row, rows);
 }
 
 // Minimum image of d, returning d - L k with the image count k in
@@ -931,12 +928,10 @@ __global__ __launch_bounds__(SEPK_BLOCK) void k_lj_coul(
 	}
 	// the two epilogues of sepk_pair_epilogue, the second adding to the first
 #pragma unroll
-	for (int o = 1; o < SEPK_SUB; o <<= 1)
-#pragma unroll
-		for (int k = 0; k < 3; k++) {
-			fl[k] += __shfl_xor(fl[k], o, SEPK_WAVE);
-			fc[k] += __shfl_xor(fc[k], o, SEPK_WAVE);
-		}
+	for (int k = 0; k < 3; k++) {
+		fl[k] = sepk_atom_sum(fl[k]);
+		fc[k] = sepk_atom_sum(fc[k]);
+	}
 	if (t < n && sub == 0 && !frozen) {
 		for (int k = 0; k < 3; k++) {
 			double v = OVERWRITE ? fl[k] : s.f[k * npad + t];
@@ -969,9 +964,15 @@ __global__ __launch_bounds__(SEPK_BLOCK) void k_lj_coul(
 		ac[5] = fma(gy, pz, ac[5]);
 		ac[6] = fma(gz, pz, ac[6]);
 	}
-	sepk_block_partial<7>(al, 0u, part_lj, lb, rows);
-	__syncthreads(); // the partial helper's LDS is reused
-	sepk_block_partial<7>(ac, 0u, part_c, lb, rows);
+	double v[14];
+#pragma unroll
+	for (int k = 0; k < 7; k++) {
+		v[k] = al[k];
+		v[7 + k] = ac[k];
+	}
+	sepk_block_reduce<false>(v, 0.0, [=](int i, double r) {
+		(i < 7 ? part_lj : part_c)[(size_t)(i < 7 ? i : i - 7) * rows + lb] = r;
+	});
 }
 
 // The recorded pair call and this Coulomb call as one k_lj_coul launch,
@@ -1107,7 +1108,7 @@ __global__ __launch_bounds__(SEPK_BLOCK) void k_nh_sum(sepk_state s, long n, lon
 		const double vx = s.v[t], vy = s.v[npad + t], vz = s.v[2 * npad + t];
 		acc[0] = (vx * vx * m + vy * vy * m) + vz * vz * m;
 	}
-	sepk_block_partial<1>(acc, 0u, partial, lb, rows);
+	sepk_block_partial(acc, partial, lb, rows);
 }
 
 __global__ void k_nh_apply(sepk_state s, long n, long npad, const double *alpha)
@@ -1183,7 +1184,7 @@ struct sepk_lfout {
 // (source/sepintgr.c:149-168, :42-88) from its force before the thermostat
 // term, spread over lanes 0..2 of the atom's SEPK_SUB lanes, one axis each
 // (lane k is given component k of the force as Fk).  Lane 0 gathers the
-// other axes' values by shuffles and forms the sums in axis order.  acc:
+// other axes' values by DPP moves and forms the sums in axis order.  acc:
 // m vh^2 summed, the six m vh (x) vh components, d^2 and m v^2.  Every lane
 // of the wave calls it.
 __device__ __forceinline__ void sepk_lf_atom_lanes(const sepk_state &s, const sepk_lfout &o,
@@ -1235,11 +1236,10 @@ __device__ __forceinline__ void sepk_lf_atom_lanes(const sepk_state &s, const se
 		o.cn[i] = cn;
 		o.cr[i] = cr;
 	}
-	const int base = (int)(threadIdx.x & (SEPK_WAVE - 1)) - sub;
-	const double x1 = __shfl(x, base + 1, SEPK_WAVE), x2 = __shfl(x, base + 2, SEPK_WAVE);
-	const double v1 = __shfl(v, base + 1, SEPK_WAVE), v2 = __shfl(v, base + 2, SEPK_WAVE);
-	const double h1 = __shfl(vh, base + 1, SEPK_WAVE), h2 = __shfl(vh, base + 2, SEPK_WAVE);
-	const double r1 = __shfl(dr, base + 1, SEPK_WAVE), r2 = __shfl(dr, base + 2, SEPK_WAVE);
+	const double x1 = sepk_dpp<SEPK_DPP_LANE1>(x), x2 = sepk_dpp<SEPK_DPP_LANE2>(x);
+	const double v1 = sepk_dpp<SEPK_DPP_LANE1>(v), v2 = sepk_dpp<SEPK_DPP_LANE2>(v);
+	const double h1 = sepk_dpp<SEPK_DPP_LANE1>(vh), h2 = sepk_dpp<SEPK_DPP_LANE2>(vh);
+	const double r1 = sepk_dpp<SEPK_DPP_LANE1>(dr), r2 = sepk_dpp<SEPK_DPP_LANE2>(dr);
 	if (act && sub == 0) {
 		acc[0] = (vh * vh * m + h1 * h1 * m) + h2 * h2 * m;
 		acc[8] = (v * v * m + v1 * v1 * m) + v2 * v2 * m;
@@ -1292,7 +1292,10 @@ __global__ __launch_bounds__(SEPK_BLOCK) void k_leapfrog(
 	const sepk_lfout o = {s.v, s.f, s.a, s.xn, s.cn, s.cr, s.pos, s.qpos};
 	sepk_lf_atom_lanes(s, o, t, npad, sub, act, Fk, Fk, Fk, dt, L0, L1, L2, nh, al, pending,
 			   qs0, qs1, qs2, acc);
-	sepk_block_partial<9>(acc, 1u << 7, partial, lb, rows);
+	const double v[8] = {acc[0], acc[1], acc[2], acc[3], acc[4], acc[5], acc[6], acc[8]};
+	sepk_block_reduce<true>(v, acc[7], [=](int i, double r) {
+		partial[(size_t)sepk_lf_col(i) * rows + lb] = r;
+	});
 }
 
 // Pair forces, Nose-Hoover and leapfrog in one launch (a step whose only
@@ -1324,12 +1327,9 @@ __global__ __launch_bounds__(SEPK_BLOCK) __attribute__((amdgpu_waves_per_eu(MIXE
 	double px = 0.0, py = 0.0, pz = 0.0;
 	sepk_lj_pairs<false, MIXED, FAST>(s, nbr, cnt, npad, c, t, sub, act, 0, fx, fy, fz, acc,
 					   px, py, pz);
-#pragma unroll
-	for (int m = 1; m < SEPK_SUB; m <<= 1) {
-		fx += __shfl_xor(fx, m, SEPK_WAVE);
-		fy += __shfl_xor(fy, m, SEPK_WAVE);
-		fz += __shfl_xor(fz, m, SEPK_WAVE);
-	}
+	fx = sepk_atom_sum(fx);
+	fy = sepk_atom_sum(fy);
+	fz = sepk_atom_sum(fz);
 	double lf[9] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
 	const int pending = sys->xn_pending;
 	double al = 0.0;
@@ -1347,8 +1347,16 @@ __global__ __launch_bounds__(SEPK_BLOCK) __attribute__((amdgpu_waves_per_eu(MIXE
 	}
 	sepk_lf_atom_lanes(s, o, t, npad, sub, act, fx, fy, fz, dt, c.L0, c.L1, c.L2, nh, al,
 			   pending, qs0, qs1, qs2, lf);
-	sepk_block_partial<7>(acc, 0u, ppart, lb, rows);
-	sepk_block_partial<9>(lf, 1u << 7, lpart, lb, rows);
+	double v[15];
+#pragma unroll
+	for (int k = 0; k < 7; k++) {
+		v[k] = acc[k];
+		v[7 + k] = lf[k];
+	}
+	v[14] = lf[8];
+	sepk_block_reduce<true>(v, lf[7], [=](int i, double r) {
+		(i < 7 ? ppart : lpart)[(size_t)(i < 7 ? i : sepk_lf_col(i - 7)) * rows + lb] = r;
+	});
 }
 
 // The leapfrog's finishing task (after the step's pair task, if fused).

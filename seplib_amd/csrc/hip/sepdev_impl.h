@@ -383,46 +383,170 @@ __device__ __forceinline__ int4 sepk_quant(const sepk_pos &p, double s0, double 
 			 (int)(unsigned)(long long)rint(p.z * s2), __float_as_int((float)p.q));
 }
 
-// Per-block reduction of NV values per thread into column-major partial
-// rows, partial[i*rows + row]:
-// columns whose bit is set in maxmask take the maximum, the others the sum,
-// in a fixed order (wave butterfly, then the block's waves in index order).
-// The finisher kernels (k_fin_rows, k_fin_apply) combine the rows
-// afterwards; the kernel boundary makes every row visible to them, so no
-// fences are needed.
-template <int NV>
-__device__ __forceinline__ void sepk_block_partial(double (&v)[NV], unsigned maxmask,
-						   double *partial, long row, long rows)
+// ---- reductions across a wave and a block ----------------------------------
+
+// x from another lane of the row of 16, by a DPP move (no LDS traffic).
+template <int CTRL>
+__device__ __forceinline__ double sepk_dpp(double x)
 {
-	__shared__ double sh[SEPK_BLOCK / SEPK_WAVE][NV];
-	const int lane = threadIdx.x & (SEPK_WAVE - 1), wid = threadIdx.x / SEPK_WAVE;
-	// butterfly step by step over all columns at once, so that each step's
-	// shuffles are in flight together (one wait a step, not one a column)
+	const long long b = __builtin_bit_cast(long long, x);
+	const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+	const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+	return __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
+}
+
+#define SEPK_DPP_XOR1 0xb1  // quad_perm [1,0,3,2]
+#define SEPK_DPP_XOR2 0x4e  // quad_perm [2,3,0,1]
+#define SEPK_DPP_LANE1 0x55 // quad_perm [1,1,1,1]
+#define SEPK_DPP_LANE2 0xaa // quad_perm [2,2,2,2]
+#define SEPK_DPP_FLIP4 0x1b // quad_perm [3,2,1,0]
+#define SEPK_DPP_FLIP8 0x141 // row_half_mirror: lane 7 - l of 8
+#define SEPK_DPP_ROR8 0x128 // lane l ^ 8 of 16
+
+// The value of lane l ^ 4: 7 - (l ^ 3) = l ^ 4 within 8 lanes.
+__device__ __forceinline__ double sepk_xor4(double x)
+{
+	return sepk_dpp<SEPK_DPP_FLIP4>(sepk_dpp<SEPK_DPP_FLIP8>(x));
+}
+
+// Sum over the SEPK_SUB lanes of an atom, in every one of them.
+__device__ __forceinline__ double sepk_atom_sum(double x)
+{
+	static_assert(SEPK_SUB == 4, "an atom's lanes are a quad");
+	x += sepk_dpp<SEPK_DPP_XOR1>(x);
+	return x + sepk_dpp<SEPK_DPP_XOR2>(x);
+}
+
+// Lanes l and l ^ W (W = 32 or 16) exchanged between two values: a keeps the
+// lower partner's of both, b the upper's.
+template <int W>
+__device__ __forceinline__ void sepk_swap(double &a, double &b)
+{
+	const unsigned long long x = __builtin_bit_cast(unsigned long long, a);
+	const unsigned long long y = __builtin_bit_cast(unsigned long long, b);
+	unsigned v[2][2];
 #pragma unroll
-	for (int o = SEPK_WAVE / 2; o > 0; o >>= 1) {
-		double y[NV];
-#pragma unroll
-		for (int i = 0; i < NV; i++)
-			y[i] = __shfl_xor(v[i], o, SEPK_WAVE);
-#pragma unroll
-		for (int i = 0; i < NV; i++)
-			v[i] = (maxmask >> i) & 1u ? fmax(v[i], y[i]) : v[i] + y[i];
+	for (int k = 0; k < 2; k++) {
+		const auto r = W == 32
+				       ? __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32 * k),
+									  (unsigned)(y >> 32 * k), false, false)
+				       : __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32 * k),
+									  (unsigned)(y >> 32 * k), false, false);
+		v[0][k] = r[0];
+		v[1][k] = r[1];
 	}
-	if (lane == 0) {
+	a = __builtin_bit_cast(double, (unsigned long long)v[0][1] << 32 | v[0][0]);
+	b = __builtin_bit_cast(double, (unsigned long long)v[1][1] << 32 | v[1][0]);
+}
+
+// One level of the wave reduction below, over partners l ^ W: N columns in,
+// (N + 1) / 2 out; while there is more than one, a lane keeps the first half
+// of them (bit W clear) or the second.
+template <int W, int N>
+__device__ __forceinline__ void sepk_wave_level(double *v)
+{
+	const bool up = threadIdx.x & W;
 #pragma unroll
-		for (int i = 0; i < NV; i++)
-			sh[wid][i] = v[i];
-	}
-	__syncthreads();
-	if (threadIdx.x < NV) {
-		const int i = threadIdx.x;
-		const bool mx = (maxmask >> i) & 1u;
-		double s = sh[0][i];
-		for (int w = 1; w < SEPK_BLOCK / SEPK_WAVE; w++)
-			s = mx ? fmax(s, sh[w][i]) : s + sh[w][i];
-		partial[(size_t)i * rows + row] = s;
+	for (int i = 0; i < (N + 1) / 2; i++) {
+		double a = v[i], b = v[N > 1 ? i + N / 2 : i];
+		if (W >= 16) {
+			sepk_swap < W >= 16 ? W : 16 > (a, b);
+		} else {
+			const double send = up ? a : b;
+			a = up ? b : a;
+			b = W == 8   ? sepk_dpp<SEPK_DPP_ROR8>(send)
+			    : W == 4 ? sepk_xor4(send)
+			    : W == 2 ? sepk_dpp<SEPK_DPP_XOR2>(send)
+				     : sepk_dpp<SEPK_DPP_XOR1>(send);
+		}
+		v[i] = a + b;
 	}
 }
+
+// Sums of NV values per lane over the wave: each column's is the butterfly's
+// tree (partners 32, 16, 8, 4, 2, 1 apart), but a level halves the columns a
+// lane carries instead of repeating all of them in every lane, and moves them
+// with lane swaps and DPP: 16 columns take about 65 vector instructions and no
+// LDS where 16 butterflies took 96 additions and 192 LDS permutes, a fifth of
+// the fused step kernel's instructions (the same bits; per step, N = 1000:
+// 31.5 -> 27.3 us, 256000 mixed: 91.3 -> 81.5, 500000: 181.5 -> 177.8, water
+// 96000: 197.9 -> 186).  Column c is left in lanes
+// SEPK_COL_LANES(NV) c and up.
+#define SEPK_COL_LANES(NV) ((NV) > 8 ? 4 : (NV) > 4 ? 8 : (NV) > 2 ? 16 : (NV) > 1 ? 32 : 64)
+template <int NV>
+__device__ __forceinline__ double sepk_wave_sums(const double (&in)[NV])
+{
+	constexpr int P = 64 / SEPK_COL_LANES(NV);
+	static_assert(NV <= 16, "at most 16 columns");
+	double v[P];
+#pragma unroll
+	for (int i = 0; i < P; i++)
+		v[i] = i < NV ? in[i < NV ? i : 0] : 0.0;
+	sepk_wave_level<32, P>(v);
+	sepk_wave_level<16, (P + 1) / 2>(v);
+	sepk_wave_level<8, (P + 3) / 4>(v);
+	sepk_wave_level<4, (P + 7) / 8>(v);
+	sepk_wave_level<2, 1>(v);
+	sepk_wave_level<1, 1>(v);
+	return v[0];
+}
+
+__device__ __forceinline__ double sepk_wave_max(double x)
+{
+	double y = x;
+	sepk_swap<32>(x, y);
+	x = y = fmax(x, y);
+	sepk_swap<16>(x, y);
+	x = fmax(x, y);
+	x = fmax(x, sepk_dpp<SEPK_DPP_ROR8>(x));
+	x = fmax(x, sepk_xor4(x));
+	x = fmax(x, sepk_dpp<SEPK_DPP_XOR2>(x));
+	return fmax(x, sepk_dpp<SEPK_DPP_XOR1>(x));
+}
+
+// Reduction over the block of NV sums per thread and, with MAX, one maximum,
+// in a fixed order (wave, then the block's waves in index order);
+// out(i, value) is called once for each column i, the maximum's is NV.
+// The finisher kernels (k_fin_rows, k_fin_apply) combine the blocks'
+// results afterwards; the kernel boundary makes them visible, so no fences
+// are needed.
+template <bool MAX, int NV, class OUT>
+__device__ __forceinline__ void sepk_block_reduce(const double (&v)[NV], double mx, OUT out)
+{
+	constexpr int NW = SEPK_BLOCK / SEPK_WAVE;
+	__shared__ double sh[NW][NV + 1];
+	const int lane = threadIdx.x & (SEPK_WAVE - 1), wid = threadIdx.x / SEPK_WAVE;
+	const double s = sepk_wave_sums(v);
+	const int c = lane / SEPK_COL_LANES(NV);
+	if (lane % SEPK_COL_LANES(NV) == 0 && c < NV)
+		sh[wid][c] = s;
+	if (MAX) {
+		const double m = sepk_wave_max(mx);
+		if (lane == 0)
+			sh[wid][NV] = m;
+	}
+	__syncthreads();
+	if (threadIdx.x < NV + (MAX ? 1 : 0)) {
+		const int i = threadIdx.x;
+		const bool top = MAX && i == NV;
+		double r = sh[0][i];
+		for (int w = 1; w < NW; w++)
+			r = top ? fmax(r, sh[w][i]) : r + sh[w][i];
+		out(i, r);
+	}
+}
+
+// The same into column-major partial rows, partial[i * rows + row].
+template <int NV>
+__device__ __forceinline__ void sepk_block_partial(const double (&v)[NV], double *partial, long row,
+						   long rows)
+{
+	sepk_block_reduce<false>(v, 0.0,
+				 [=](int i, double r) { partial[(size_t)i * rows + row] = r; });
+}
+
+// A leapfrog's columns (sepk_lf_atom_lanes): 0-6 and 8 sums, 7 the maximum.
+__device__ __forceinline__ int sepk_lf_col(int i) { return i < 7 ? i : 15 - i; }
 
 // Nose-Hoover friction update of source/sepintgr.c:151-162, from the sum of
 // m v^2 over all atoms: ekin = 0.5 sum / N, T = 0.666667 ekin,

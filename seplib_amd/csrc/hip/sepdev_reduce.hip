@@ -105,7 +105,7 @@ __device__ static void fin_sys(const sepk_task &k, const double *tot, double *al
 // queued task (at least two); wave w of every workgroup takes task w: a
 // contiguous chunk of its rows, one lane per row (SEPK_MAXNV columns loaded
 // at once with clamped addresses, all tasks' loads in flight together),
-// reduced in a fixed order -- lane-strided rows, then a wave butterfly --
+// reduced in a fixed order -- lane-strided rows, then the wave's tree --
 // to one value per column.  k_fin_apply, one workgroup, combines the
 // SEPK_FIN_BLOCKS values of each column in block order (wave w again for
 // task w) and applies the tasks in queue order: lane w of the first wave
@@ -118,6 +118,24 @@ __device__ static void fin_sys(const sepk_task &k, const double *tot, double *al
 __device__ static double fin_comb(bool mx, double a, double b)
 {
 	return mx ? fmax(a, b) : a + b;
+}
+
+// A task's columns over the wave, left as sepk_wave_sums leaves them; the
+// column whose bit is set in maxmask (at most one) takes the maximum.
+__device__ static double fin_wave(const sepk_task &k, const double (&v)[SEPK_MAXNV])
+{
+	double r = sepk_wave_sums(v);
+	if (k.maxmask) {
+		const int c = __builtin_ctz(k.maxmask);
+		double x = v[0];
+#pragma unroll
+		for (int i = 1; i < SEPK_MAXNV; i++)
+			x = i == c ? v[i] : x;
+		x = sepk_wave_max(x);
+		if ((int)(threadIdx.x & 63) / SEPK_COL_LANES(SEPK_MAXNV) == c)
+			r = x;
+	}
+	return r;
 }
 
 static_assert(FIN_THREADS == 64 * SEPK_MAXTASK, "one finisher wave per task");
@@ -147,21 +165,10 @@ __global__ __launch_bounds__(FIN_THREADS) void k_fin_rows(const double *partials
 			for (int i = 0; i < SEPK_MAXNV; i++)
 				a[i] = fin_comb((k.maxmask >> i) & 1u, a[i], v[i]);
 		}
-		// butterfly step by step over all columns at once (one wait a step)
-#pragma unroll
-		for (int o = 32; o > 0; o >>= 1) {
-			double y[SEPK_MAXNV];
-#pragma unroll
-			for (int i = 0; i < SEPK_MAXNV; i++)
-				y[i] = __shfl_xor(a[i], o, 64);
-#pragma unroll
-			for (int i = 0; i < SEPK_MAXNV; i++)
-				a[i] = fin_comb((k.maxmask >> i) & 1u, a[i], y[i]);
-		}
-#pragma unroll
-		for (int i = 0; i < SEPK_MAXNV; i++)
-			if (lane == 0 && i < k.nv)
-				f.l2[((size_t)ti * SEPK_MAXNV + i) * G + blockIdx.x] = a[i];
+		const double r = fin_wave(k, a);
+		const int c = lane / SEPK_COL_LANES(SEPK_MAXNV);
+		if (lane % SEPK_COL_LANES(SEPK_MAXNV) == 0 && c < k.nv)
+			f.l2[((size_t)ti * SEPK_MAXNV + c) * G + blockIdx.x] = r;
 	}
 }
 
@@ -198,20 +205,10 @@ __global__ __launch_bounds__(FIN_THREADS) void k_fin_apply(sepk_fin f, int G)
 			const double *col = f.l2 + ((size_t)ti * SEPK_MAXNV + (i < k.nv ? i : 0)) * G;
 			x[i] = lane < G ? col[lane] : 0.0;
 		}
-#pragma unroll
-		for (int o = 32; o > 0; o >>= 1) {
-			double y[SEPK_MAXNV];
-#pragma unroll
-			for (int i = 0; i < SEPK_MAXNV; i++)
-				y[i] = __shfl_xor(x[i], o, 64);
-#pragma unroll
-			for (int i = 0; i < SEPK_MAXNV; i++)
-				x[i] = fin_comb((k.maxmask >> i) & 1u, x[i], y[i]);
-		}
-#pragma unroll
-		for (int i = 0; i < SEPK_MAXNV; i++)
-			if (lane == 0)
-				tot[ti][i] = x[i];
+		const double r = fin_wave(k, x);
+		const int c = lane / SEPK_COL_LANES(SEPK_MAXNV);
+		if (lane % SEPK_COL_LANES(SEPK_MAXNV) == 0 && c < SEPK_MAXNV)
+			tot[ti][c] = r;
 	}
 	__syncthreads();
 	// after a device error the step changed nothing, and neither does this
