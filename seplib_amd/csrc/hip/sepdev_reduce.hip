@@ -172,31 +172,88 @@ __global__ __launch_bounds__(FIN_THREADS) void k_fin_rows(const double *partials
 	}
 }
 
-__global__ __launch_bounds__(FIN_THREADS) void k_fin_apply(sepk_fin f, int G)
+// The words the tasks work on, in the applying workgroup's LDS.
+struct fin_lds {
+	double tot[SEPK_MAXTASK][SEPK_MAXNV];
+	double sret[SEPK_MAXTASK][SEPDEV_RET_WORDS];
+	double salpha[SEPK_MAXTASK];
+	sepdev_sys ssys;
+};
+
+// The tasks read and update the system scalars, their return slots and
+// thermostat variables: one parallel load of each into LDS (issued with the
+// loads of the row results), the tasks applied there in queue order, one
+// parallel store back.  Returns the step record's count to the first wave.
+__device__ __forceinline__ unsigned long long fin_load(const sepk_fin &f, fin_lds &L)
 {
-	__shared__ double tot[SEPK_MAXTASK][SEPK_MAXNV];
-	__shared__ double sret[SEPK_MAXTASK][SEPDEV_RET_WORDS];
-	__shared__ double salpha[SEPK_MAXTASK];
-	__shared__ sepdev_sys ssys;
-	const int lane = threadIdx.x & 63;
-	const int ti = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); // this wave's task
-	// The tasks read and update the system scalars, their return slots and
-	// thermostat variables: one parallel load of each into LDS (issued with
-	// the loads of the row results), the tasks applied there in queue order,
-	// one parallel store back.
 	const signed char *rmap = f.rmap, *amap = f.amap; // first task sharing the pointer
 	const int nsys = (int)(sizeof(sepdev_sys) / sizeof(int));
 	for (int w = threadIdx.x; w < f.ntask * SEPDEV_RET_WORDS; w += blockDim.x) {
 		const int u = w / SEPDEV_RET_WORDS, word = w % SEPDEV_RET_WORDS;
 		if (rmap[u] == u)
-			sret[u][word] = f.t[u].ret[word];
+			L.sret[u][word] = f.t[u].ret[word];
 	}
 	if (threadIdx.x < f.ntask && amap[threadIdx.x] == (int)threadIdx.x)
-		salpha[threadIdx.x] = *f.t[threadIdx.x].alpha;
+		L.salpha[threadIdx.x] = *f.t[threadIdx.x].alpha;
 	if (threadIdx.x >= 64 && threadIdx.x < 64 + nsys)
-		((int *)&ssys)[threadIdx.x - 64] = ((const int *)f.sys)[threadIdx.x - 64];
-	const unsigned long long ring_at =
-		f.ring_task >= 0 && ti == 0 ? *f.t[f.ring_task].ring_n : 0ull;
+		((int *)&L.ssys)[threadIdx.x - 64] = ((const int *)f.sys)[threadIdx.x - 64];
+	return f.ring_task >= 0 && threadIdx.x < 64 ? *f.t[f.ring_task].ring_n : 0ull;
+}
+
+// Applies the tasks from their totals and stores what they changed.
+__device__ __forceinline__ void fin_finish(const sepk_fin &f, fin_lds &L, unsigned long long ring_at)
+{
+	const signed char *rmap = f.rmap, *amap = f.amap;
+	const int nsys = (int)(sizeof(sepdev_sys) / sizeof(int));
+	__syncthreads();
+	// after a device error the step changed nothing, and neither does this
+	const bool frozen = L.ssys.error != 0;
+	if (threadIdx.x < SEPDEV_RET_WORDS && !frozen) {
+		for (int u = 0; u < f.ntask; u++)
+			if (rmap[u] >= 0)
+				L.sret[rmap[u]][threadIdx.x] =
+					fin_word(f.t[u], L.tot[u], threadIdx.x, L.sret[rmap[u]][threadIdx.x]);
+	} else if (threadIdx.x == 64 && !frozen) {
+		for (int u = 0; u < f.ntask; u++) {
+			const sepk_task &k = f.t[u];
+			// a conditional build that did not run leaves nothing to finish
+			if (k.mode == SEPK_FIN_BUILD && k.conditional && L.ssys.neighb_flag == 0)
+				continue;
+			fin_sys(k, L.tot[u], amap[u] >= 0 ? &L.salpha[amap[u]] : nullptr, &L.ssys);
+		}
+	}
+	__syncthreads();
+	for (int w = threadIdx.x; w < f.ntask * SEPDEV_RET_WORDS; w += blockDim.x) {
+		const int u = w / SEPDEV_RET_WORDS, word = w % SEPDEV_RET_WORDS;
+		if (rmap[u] == u)
+			f.t[u].ret[word] = L.sret[u][word];
+	}
+	// the per-step record: the leapfrog's return slot and the new tnow; the
+	// count was read at the start by this same wave, which alone stores it
+	if (f.ring_task >= 0 && !frozen && threadIdx.x <= SEPDEV_RET_WORDS) {
+		const sepk_task &k = f.t[f.ring_task];
+		double *rec = k.ring + (size_t)(ring_at % (unsigned long long)k.ring_cap) * SEPDEV_RING_WORDS;
+		rec[threadIdx.x] = threadIdx.x < SEPDEV_RET_WORDS ? L.sret[rmap[f.ring_task]][threadIdx.x]
+								  : L.ssys.tnow;
+		if (threadIdx.x == 0)
+			*k.ring_n = ring_at + 1;
+	}
+	if (threadIdx.x < f.ntask && amap[threadIdx.x] == (int)threadIdx.x)
+		*f.t[threadIdx.x].alpha = L.salpha[threadIdx.x];
+	if (threadIdx.x >= 64 && threadIdx.x < 64 + nsys)
+		((int *)f.sys)[threadIdx.x - 64] = ((const int *)&L.ssys)[threadIdx.x - 64];
+}
+
+// A region's rows combined in k_fin_rows's groups by the workgroup itself.
+#define FIN_ONE_ROWS 512
+#define FIN_ONE_THREADS 1024
+
+__global__ __launch_bounds__(FIN_THREADS) void k_fin_apply(sepk_fin f, int G)
+{
+	__shared__ fin_lds L;
+	const int lane = threadIdx.x & 63;
+	const int ti = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); // this wave's task
+	const unsigned long long ring_at = fin_load(f, L);
 	if (ti < f.ntask) {
 		const sepk_task &k = f.t[ti];
 		double x[SEPK_MAXNV];
@@ -208,45 +265,50 @@ __global__ __launch_bounds__(FIN_THREADS) void k_fin_apply(sepk_fin f, int G)
 		const double r = fin_wave(k, x);
 		const int c = lane / SEPK_COL_LANES(SEPK_MAXNV);
 		if (lane % SEPK_COL_LANES(SEPK_MAXNV) == 0 && c < SEPK_MAXNV)
-			tot[ti][c] = r;
+			L.tot[ti][c] = r;
 	}
-	__syncthreads();
-	// after a device error the step changed nothing, and neither does this
-	const bool frozen = ssys.error != 0;
-	if (threadIdx.x < SEPDEV_RET_WORDS && !frozen) {
-		for (int u = 0; u < f.ntask; u++)
-			if (rmap[u] >= 0)
-				sret[rmap[u]][threadIdx.x] =
-					fin_word(f.t[u], tot[u], threadIdx.x, sret[rmap[u]][threadIdx.x]);
-	} else if (threadIdx.x == 64 && !frozen) {
-		for (int u = 0; u < f.ntask; u++) {
-			const sepk_task &k = f.t[u];
-			// a conditional build that did not run leaves nothing to finish
-			if (k.mode == SEPK_FIN_BUILD && k.conditional && ssys.neighb_flag == 0)
-				continue;
-			fin_sys(k, tot[u], amap[u] >= 0 ? &salpha[amap[u]] : nullptr, &ssys);
+	fin_finish(f, L, ring_at);
+}
+
+// The whole finisher in one workgroup, for tasks of at most FIN_ONE_ROWS rows
+// (32768 atoms): one launch instead of two.  The waves take the (task, column)
+// pairs in turn; lane g combines the rows that k_fin_rows's workgroup g would
+// (at most 8, loaded together) in that workgroup's tree -- its lanes' partners
+// 4, 2, 1 apart, the others zero -- and the wave the 64 groups as k_fin_apply
+// does, so both give the same bits.  Per step: N = 1000 27.1 -> 23.8 us, 27000
+// 32.1 -> 28.7, water 6000 100.9 -> 98.
+__global__ __launch_bounds__(FIN_ONE_THREADS) void k_fin_one(const double *partials, sepk_fin f)
+{
+	__shared__ fin_lds L;
+	const int lane = threadIdx.x & 63;
+	const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	const unsigned long long ring_at = fin_load(f, L);
+	for (int u = 0, q = wid; u < f.ntask; u++) {
+		const sepk_task &k = f.t[u];
+		const double *p = partials + (size_t)k.region * f.region_words;
+		const int chunk = (k.nblk + 63) / 64, r0 = lane * chunk;
+		for (; q < k.nv; q += FIN_ONE_THREADS / 64) {
+			const bool mx = (k.maxmask >> q) & 1u;
+			double v[FIN_ONE_ROWS / 64];
+#pragma unroll
+			for (int i = 0; i < FIN_ONE_ROWS / 64; i++)
+				v[i] = i < chunk && r0 + i < k.nblk ? p[(size_t)q * f.region_rows + r0 + i] : 0.0;
+#pragma unroll
+			for (int i = 0; i < FIN_ONE_ROWS / 64; i++)
+				v[i] = fin_comb(mx, 0.0, v[i]);
+#pragma unroll
+			for (int o = FIN_ONE_ROWS / 128; o > 0; o >>= 1)
+#pragma unroll
+				for (int i = 0; i < o; i++)
+					v[i] = fin_comb(mx, v[i], v[i + o]);
+			const double one[1] = {v[0]};
+			const double r = mx ? sepk_wave_max(v[0]) : sepk_wave_sums(one);
+			if (lane == 0)
+				L.tot[u][q] = r;
 		}
+		q -= k.nv;
 	}
-	__syncthreads();
-	for (int w = threadIdx.x; w < f.ntask * SEPDEV_RET_WORDS; w += blockDim.x) {
-		const int u = w / SEPDEV_RET_WORDS, word = w % SEPDEV_RET_WORDS;
-		if (rmap[u] == u)
-			f.t[u].ret[word] = sret[u][word];
-	}
-	// the per-step record: the leapfrog's return slot and the new tnow; the
-	// count was read at the start by this same wave, which alone stores it
-	if (f.ring_task >= 0 && !frozen && threadIdx.x <= SEPDEV_RET_WORDS) {
-		const sepk_task &k = f.t[f.ring_task];
-		double *rec = k.ring + (size_t)(ring_at % (unsigned long long)k.ring_cap) * SEPDEV_RING_WORDS;
-		rec[threadIdx.x] = threadIdx.x < SEPDEV_RET_WORDS ? sret[rmap[f.ring_task]][threadIdx.x]
-								  : ssys.tnow;
-		if (threadIdx.x == 0)
-			*k.ring_n = ring_at + 1;
-	}
-	if (threadIdx.x < f.ntask && amap[threadIdx.x] == (int)threadIdx.x)
-		*f.t[threadIdx.x].alpha = salpha[threadIdx.x];
-	if (threadIdx.x >= 64 && threadIdx.x < 64 + nsys)
-		((int *)f.sys)[threadIdx.x - 64] = ((const int *)&ssys)[threadIdx.x - 64];
+	fin_finish(f, L, ring_at);
 }
 
 double *sepk_region(sepdev *d, int region)
@@ -287,6 +349,14 @@ int sepk_flush_tasks(sepdev *d)
 		if (f.t[u].mode == SEPK_FIN_LF && f.t[u].ring && f.rmap[u] >= 0)
 			f.ring_task = u;
 	d->npending = 0;
+	bool one = true;
+	for (int u = 0; u < f.ntask; u++)
+		one = one && f.t[u].nblk <= FIN_ONE_ROWS;
+	if (one) {
+		k_fin_one<<<1, FIN_ONE_THREADS, 0, d->st>>>(d->partials, f);
+		SEPK_LAUNCH_CHECK();
+		return 0;
+	}
 	// one wave per task, at least two (the system scalars are copied by the
 	// second wave)
 	const unsigned threads = 64u * (unsigned)(f.ntask > 2 ? f.ntask : 2);
