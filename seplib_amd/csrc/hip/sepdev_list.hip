@@ -13,6 +13,8 @@
 //                  index (so the device order and every list are independent
 //                  of atomic timing) and move each member's state to its new
 //                  cell-sorted index in the spare copy
+//                  (k_order: all of these in one launch, for systems of up to
+//                  32768 atoms)
 //   k_build_q      a wave per slab of a cell's atoms (k_build: a workgroup per
 //                  cell, for boxes that are not cubic): the stencil's atoms
 //                  within the list cutoff, 64 candidates at a time; then copy
@@ -457,6 +459,165 @@ __global__ __launch_bounds__(SEPK_BLOCK) void k_sort_permute_wg(
 			if (has_partners)
 				sepk_copy_partners(src, dst, o, t, npad);
 		}
+	}
+}
+
+// Binning, scan, sort and permutation in one launch, for systems of up to
+// SEPK_ORDER_ATOMS atoms and SEPK_ORDER_CELLS cells: every workgroup bins all
+// atoms and scans the cell counts in its LDS, and permutes the cells of its
+// own share, so that no workgroup waits for another and the three launches of
+// a larger system (k_bin, k_scan_scatter, k_sort_permute) are one.  Reading
+// every position in each of 64 workgroups costs a few us a rebuild up to this
+// size; what it saves is two launches in every step, rebuilt or not, and the
+// chain of three kernels' memory round trips in a rebuild.  Per step: N = 1000
+// 23.8 -> 20.3 us, 27000 28.7 -> 27.5, water 6000 98 -> 96.1 (at 27000 a rebuild
+// already spends more on the binning; larger systems gain nothing).
+#define SEPK_ORDER_ATOMS 32768
+#define SEPK_ORDER_CELLS 4096
+#define SEPK_ORDER_GRID 64
+#define SEPK_ORDER_KEYS 2048
+
+// Whether q = p / l, from the product with 1 / l, is far enough from a whole
+// number and inside the grid for its truncation to be that of the division.
+__device__ __forceinline__ bool sepk_plain_cell(double q, int n, int &c)
+{
+	c = (int)q;
+	const double r = q - (double)c;
+	return q > 1e-6 && r > 1e-9 && r < 1.0 - 1e-9 && c < n;
+}
+
+template <int NMAX>
+__global__ __launch_bounds__(1024) void k_order(sepk_state src, sepk_state dst, long nl, long npad,
+						sepdev_grid g, int ncell, int *start, int *iperm,
+						sepdev_sys *sys, int conditional, int has_partners)
+{
+	if (conditional && sys->neighb_flag == 0)
+		return;
+	__shared__ unsigned short cid[NMAX], mem[NMAX];
+	__shared__ int sstart[SEPK_ORDER_CELLS + 4], keys[SEPK_ORDER_KEYS];
+	__shared__ int fill[SEPK_ORDER_CELLS / SEPK_ORDER_GRID + 1];
+	__shared__ int wsum[16], failed, bad;
+	const int n = (int)nl, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+	const int pending = sys->xn_pending;
+	for (int c = tid; c < ncell; c += 1024)
+		sstart[c] = 0;
+	// an error set while this runs is an atom outside the grid, which every
+	// workgroup finds by itself; one set before is looked at once
+	if (tid == 0)
+		failed = bad = sys->error != 0;
+	if (blockIdx.x == 0 && tid == 0)
+		sys->max_full = 0; // the build's atomic maximum starts here
+	__syncthreads();
+	const double il0 = 1.0 / g.l[0], il1 = 1.0 / g.l[1], il2 = 1.0 / g.l[2];
+	// whole waves iterate together
+	for (int t0 = 0; t0 < n && !failed; t0 += 1024) {
+		const int t = t0 + tid;
+		int c = -1;
+		if (t < n) {
+			const sepk_pos p = sepk_at(src.pos, (unsigned)t);
+			int cx, cy, cz;
+			const bool fx = sepk_plain_cell(p.x * il0, g.n[0], cx),
+				   fy = sepk_plain_cell(p.y * il1, g.n[1], cy),
+				   fz = sepk_plain_cell(p.z * il2, g.n[2], cz);
+			c = cx + (cy + cz * g.n[1]) * g.n[0];
+			if (!(fx && fy && fz)) {
+				c = (int)sepk_cell_of(p, g);
+				if (c < 0) {
+					sepk_set_error(sys, SEP_GPU_ECELL);
+					bad = 1;
+					c = 0;
+				}
+				// an atom outside [0, n*l) on some axis, as in k_bin
+				const double q[3] = {p.x / g.l[0], p.y / g.l[1], p.z / g.l[2]};
+				if (!(q[0] >= 0.0 && q[0] < g.n[0] && q[1] >= 0.0 && q[1] < g.n[1] &&
+				      q[2] >= 0.0 && q[2] < g.n[2]))
+					sys->unclean = 1;
+			}
+			cid[t] = (unsigned short)c;
+		}
+		// one LDS atomic per run of lanes in one cell (the atoms arrive in
+		// the last build's cell order)
+		const int before = __shfl_up(c, 1, 64);
+		const unsigned long long head = __ballot(lane == 0 || c != before);
+		if (c >= 0 && (head >> lane & 1ull)) {
+			const unsigned long long rest = lane == 63 ? 0ull : head >> (lane + 1);
+			atomicAdd(&sstart[c], rest ? __builtin_ctzll(rest) + 1 : min(64 - lane, n - t));
+		}
+	}
+	__syncthreads();
+	const bool frozen = bad != 0;
+	if (blockIdx.x == 0 && tid == 0)
+		sys->frozen = frozen;
+	if (frozen)
+		return; // the build skips as well
+	// exclusive scan of the counts, four cells a thread
+	{
+		static_assert(SEPK_ORDER_CELLS == 4 * 1024, "one pass");
+		int v[4], tot = 0;
+#pragma unroll
+		for (int k = 0; k < 4; k++) {
+			v[k] = 4 * tid + k < ncell ? sstart[4 * tid + k] : 0;
+			tot += v[k];
+		}
+		int x = tot; // inclusive wave scan of the thread totals
+		for (int o = 1; o < 64; o <<= 1) {
+			const int y = __shfl_up(x, o, 64);
+			if (lane >= o)
+				x += y;
+		}
+		if (lane == 63)
+			wsum[wid] = x;
+		__syncthreads();
+		int off = x - tot;
+		for (int w = 0; w < wid; w++)
+			off += wsum[w];
+#pragma unroll
+		for (int k = 0; k < 4; k++) {
+			if (4 * tid + k < ncell)
+				sstart[4 * tid + k] = off;
+			off += v[k];
+		}
+		if (tid == 0)
+			sstart[ncell] = n;
+	}
+	// this workgroup's cells [c0, c1): their members, in any order
+	const int per = (ncell + (int)gridDim.x - 1) / (int)gridDim.x;
+	const int c0 = min((int)blockIdx.x * per, ncell), c1 = min(c0 + per, ncell);
+	for (int k = tid; k < per; k += 1024)
+		fill[k] = 0;
+	__syncthreads();
+	if (c0 == c1)
+		return;
+	const int base = sstart[c0], m = sstart[c1] - base;
+	for (int c = c0 + tid; c < c1 + (c1 == ncell ? 1 : 0); c += 1024)
+		start[c] = sstart[c];
+	for (int t = tid; t < n; t += 1024) {
+		const int c = cid[t];
+		if (c >= c0 && c < c1)
+			mem[sstart[c] - base + atomicAdd(&fill[c - c0], 1)] = (unsigned short)t;
+	}
+	__syncthreads();
+	const bool small = m <= SEPK_ORDER_KEYS;
+	for (int i = tid; i < m && small; i += 1024)
+		keys[i] = sepk_at(src.orig, (unsigned)mem[i]);
+	__syncthreads();
+	// each member ranked by its original index within its cell and moved
+	for (int i = tid; i < m; i += 1024) {
+		const int o = mem[i], c = cid[o];
+		const int a = sstart[c] - base, b = sstart[c + 1] - base;
+		const int key = small ? keys[i] : sepk_at(src.orig, (unsigned)o);
+		int rank = 0;
+		if (small)
+			for (int j = a; j < b; j++)
+				rank += keys[j] < key;
+		else
+			for (int j = a; j < b; j++)
+				rank += sepk_at(src.orig, (unsigned)mem[j]) < key;
+		const int t = sstart[c] + rank;
+		sepk_move_atom(src, o, dst, t, npad, pending);
+		sepk_at(iperm, (unsigned)key) = t;
+		if (has_partners)
+			sepk_copy_partners(src, dst, o, t, npad);
 	}
 }
 
@@ -1505,36 +1666,43 @@ extern "C" int sepdev_build_list(sepdev *d, const sepdev_grid *gp, int condition
 	sepk_state &cur = d->s[0];   // current state, fixed addresses
 	sepk_state &spare = d->s[1]; // receives the permuted order
 	const int hp = cur.partners != nullptr;
-	unsigned nb = sepk_blocks(d->n);
-	if (nb > SEPK_GRID_CAP)
-		nb = SEPK_GRID_CAP;
-	// half a wave per cell when the cells hold 32 atoms or fewer on
-	// average, a wave up to 64, a workgroup beyond
-	const bool half = d->n <= 32 * ncell, wg = d->n > 64 * ncell;
-	long sb = wg ? ncell : (ncell * (half ? 32 : 64) + SEPK_BLOCK - 1) / SEPK_BLOCK;
-	if (sb > SEPK_GRID_CAP)
-		sb = SEPK_GRID_CAP;
-	k_bin<<<nb, SEPK_BLOCK, 0, d->st>>>(cur.pos, d->n, g, d->cellid_old, d->cell_slot,
-					    d->cell_count, d->sys,
-					    conditional);
-	if (ncell <= SEPK_PLACE_CELLS) {
-		// one launch: each workgroup scans the counts itself
-		long pb = (d->n + 1023) / 1024;
-		if (pb > 256)
-			pb = 256;
-		k_scan_scatter<<<(unsigned)pb, 1024, 0, d->st>>>(
-			d->cell_count, d->cell_start, d->cellid_old, d->cell_slot, d->order_tmp, ncell,
-			d->n, d->sys, conditional);
+	if (d->n <= SEPK_ORDER_ATOMS && ncell <= SEPK_ORDER_CELLS) {
+		const unsigned ob = (unsigned)(ncell < SEPK_ORDER_GRID ? ncell : SEPK_ORDER_GRID);
+		(d->n <= SEPK_ORDER_ATOMS / 8 ? k_order<SEPK_ORDER_ATOMS / 8> : k_order<SEPK_ORDER_ATOMS>)<<<ob, 1024, 0, d->st>>>(
+			cur, spare, d->n, d->npad, g, (int)ncell, d->cell_start, d->iperm, d->sys,
+			conditional, hp);
 	} else {
-		k_scan<<<1, 1024, 0, d->st>>>(d->cell_count, d->cell_start, ncell, d->sys,
-					      conditional);
-		k_scatter<<<nb, SEPK_BLOCK, 0, d->st>>>(d->cellid_old, d->cell_slot,
-							d->cell_start, d->order_tmp, d->n, d->sys,
-							conditional);
+		unsigned nb = sepk_blocks(d->n);
+		if (nb > SEPK_GRID_CAP)
+			nb = SEPK_GRID_CAP;
+		// half a wave per cell when the cells hold 32 atoms or fewer on
+		// average, a wave up to 64, a workgroup beyond
+		const bool half = d->n <= 32 * ncell, wg = d->n > 64 * ncell;
+		long sb = wg ? ncell : (ncell * (half ? 32 : 64) + SEPK_BLOCK - 1) / SEPK_BLOCK;
+		if (sb > SEPK_GRID_CAP)
+			sb = SEPK_GRID_CAP;
+		k_bin<<<nb, SEPK_BLOCK, 0, d->st>>>(cur.pos, d->n, g, d->cellid_old, d->cell_slot,
+						    d->cell_count, d->sys,
+						    conditional);
+		if (ncell <= SEPK_PLACE_CELLS) {
+			// one launch: each workgroup scans the counts itself
+			long pb = (d->n + 1023) / 1024;
+			if (pb > 256)
+				pb = 256;
+			k_scan_scatter<<<(unsigned)pb, 1024, 0, d->st>>>(
+				d->cell_count, d->cell_start, d->cellid_old, d->cell_slot, d->order_tmp, ncell,
+				d->n, d->sys, conditional);
+		} else {
+			k_scan<<<1, 1024, 0, d->st>>>(d->cell_count, d->cell_start, ncell, d->sys,
+						      conditional);
+			k_scatter<<<nb, SEPK_BLOCK, 0, d->st>>>(d->cellid_old, d->cell_slot,
+								d->cell_start, d->order_tmp, d->n, d->sys,
+								conditional);
+		}
+		(wg ? k_sort_permute_wg : half ? k_sort_permute<32> : k_sort_permute<64>)<<<(unsigned)sb, SEPK_BLOCK, 0, d->st>>>(
+			d->order_tmp, d->cell_start, cur, spare, d->iperm, ncell, d->npad,
+			d->sys, conditional, hp, d->cell_count);
 	}
-	(wg ? k_sort_permute_wg : half ? k_sort_permute<32> : k_sort_permute<64>)<<<(unsigned)sb, SEPK_BLOCK, 0, d->st>>>(
-		d->order_tmp, d->cell_start, cur, spare, d->iperm, ncell, d->npad,
-		d->sys, conditional, hp, d->cell_count);
 	SEPK_LAUNCH_CHECK();
 	// A cell's atoms in nslice slices (the lists do not depend on the
 	// split).  FP64, a workgroup a slice: one, unless the cells are few and

@@ -112,3 +112,52 @@ def test_faces(product, oracle, opt, where):
 def test_box_not_cubic(product, oracle, shape):
     L = np.array([RL * k * 1.01 for k in shape])
     _check(product, oracle, _workload(_points(1500, L, 13), L))
+
+
+@pytest.mark.parametrize("n,clump", [(4096, 0), (4097, 2500), (9000, 2100), (32768, 0), (32769, 0)])
+def test_wide_cells(product, oracle, n, clump):
+    """Cells much wider than the list cutoff: more members in one than the
+    one-launch ordering ranks in LDS, and its largest and the next system."""
+    L = 30.0
+    x = W.uniform(17, 3 * n).reshape(n, 3) * L
+    x[:clump] = 10.1 + W.uniform(18, 3 * clump).reshape(clump, 3) * 9.8
+    w = _workload(x, [L] * 3)
+    pairs = []
+    for api in (product, oracle):
+        s = SepSystem.from_workload(api, w, cf=1.0, dt=0.005, skin=0.2, nneighb=100,
+                                    nsubbox=(3, 3, 3))
+        try:
+            s.reset_retval()
+            s.reset_force()
+            s.force_pairs("AA", 1.0, "sep_lj", S.SEP_ALL)
+            pairs.append(s.half_pairs())
+        finally:
+            s.close()
+    assert len(pairs[1]) > 0
+    assert np.array_equal(*pairs)
+
+
+@pytest.mark.parametrize("n", [2, 63, 65, 4096, 4097, 32767, 32768, 32769])
+def test_sums_over_blocks(product, oracle, n):
+    """Energies and stress where the number of partial rows crosses the
+    finisher's limits: sums of n terms in another order than the oracle's,
+    each within n roundings, so 1e-12 relative holds with room to spare."""
+    w = W.random_packed(n, 0.8442, 1.0, seed=23)
+    if n < 1000:  # the box holds three cells an axis
+        w["L"] = np.maximum(w["L"], 3.1 * RL)
+    out = []
+    for api in (product, oracle):
+        s = SepSystem.from_workload(api, w, cf=CF, dt=0.005, skin=SKIN, nneighb=128,
+                                    nsubbox=[int(l / RL) for l in w["L"]])
+        try:
+            s.reset_retval()
+            s.reset_force()
+            s.force_pairs("AA", CF, "sep_lj_shift", S.SEP_ALL)
+            s.leapfrog()
+            out.append((s.ret.epot, s.ret.ekin, S.mat(s.ret.pot_P), S.mat(s.ret.kin_P),
+                        s.sys.max_dist2))
+        finally:
+            s.close()
+    for a, b in zip(*out):
+        scale = np.abs(b).max()
+        assert np.abs(np.asarray(a) - b).max() <= 1e-12 * scale, (a, b)
