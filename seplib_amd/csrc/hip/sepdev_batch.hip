@@ -51,6 +51,7 @@
 #define SEPB_BLOCK 256
 #define SEPB_NV 16
 #define SEPB_BATCH 4
+#define SEPB_REC_ATOMS 64 // atoms per workgroup of a download
 
 // One system on the device.  Read by every kernel; written only by the
 // finishing tile of k_bstep, the last cell of k_bbuild and the host.
@@ -126,6 +127,9 @@ struct sepdev_batch {
 	hipGraph_t graph;
 	hipGraphExec_t exec;
 	int graph_mixed, graph_steps;
+	int *hrec; // pinned records of a download
+	hipEvent_t chunk_ev[SEPK_CHUNKS];
+	int chunk_sys[SEPK_CHUNKS]; // first system past each chunk
 };
 
 __device__ __forceinline__ int sepb_mod(int a, int n)
@@ -1117,6 +1121,11 @@ extern "C" void sepdev_batch_destroy(sepdev_batch *b)
 	(void)hipFree(b->partial);
 	(void)hipFree(b->tiles);
 	(void)hipFree(b->sub_tiles);
+	if (b->hrec)
+		(void)hipHostFree(b->hrec);
+	for (hipEvent_t ev : b->chunk_ev)
+		if (ev)
+			(void)hipEventDestroy(ev);
 	if (b->st)
 		(void)hipStreamDestroy(b->st);
 	free(b->hsys);
@@ -1289,6 +1298,12 @@ extern "C" sepdev_batch *sepdev_batch_create(int nsys, const sepdev_batch_sys *i
 	rc |= balloc(&b->partial, (size_t)b->prow * SEPB_NV);
 	rc |= balloc(&b->tiles, b->prow);
 	rc |= balloc(&b->sub_tiles, b->prow);
+	if (hipHostMalloc((void **)&b->hrec, (size_t)slots * SEPDEV_BATCH_WORDS * sizeof(int),
+			  hipHostMallocDefault) != hipSuccess)
+		rc |= sepk_fail(SEP_GPU_EDEVICE, "batch: hipHostMalloc failed");
+	for (hipEvent_t &ev : b->chunk_ev)
+		if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess)
+			rc |= sepk_fail(SEP_GPU_EDEVICE, "batch: hipEventCreate failed");
 	if (rc) {
 		*err = rc;
 		sepdev_batch_destroy(b);
@@ -1521,68 +1536,103 @@ extern "C" int sepdev_batch_synchronize(sepdev_batch *b)
 // State of system s in its original atom order (3n interleaved vectors;
 // any pointer may be null), its return slot (SEPDEV_RET_WORDS) and scalars
 // {alpha, max_dist2, tnow, nupdate, neighb_flag, max_full, error, sumv2}.
-extern "C" int sepdev_batch_get(sepdev_batch *b, int s, double *x, double *v, double *f,
-				double *a, int *cr, double *ret, double *scal)
+// Records of the systems s0 + blockIdx.y: x, v, f, a (3 doubles each), the
+// crossings and one word of padding per atom, in original order, written to
+// pinned host memory (system s's from record sys[s].off on).  A record is 112
+// contiguous bytes, so the link sees whole accesses although the atoms arrive
+// in cell order.
+__global__ void k_bgather(const sepb_sys *sys, const sepb_state *st, long slots, int s0, int *rec)
+{
+	const sepb_sys &y = sys[s0 + blockIdx.y];
+	const sepb_state &S = st[y.cur];
+	const int *const x = (const int *)S.pos[y.p];
+	for (int j = threadIdx.x; j < SEPB_REC_ATOMS * SEPDEV_BATCH_WORDS; j += SEPB_BLOCK) {
+		const int a = j / SEPDEV_BATCH_WORDS, w = j - a * SEPDEV_BATCH_WORDS;
+		const int t = blockIdx.x * SEPB_REC_ATOMS + a;
+		if (t >= y.n)
+			return;
+		const size_t g = y.off + t;
+		int v = 0;
+		if (w < 6) {
+			v = x[g * (sizeof(sepk_pos) / 4) + w];
+		} else if (w < 24) {
+			const int q = w / 6, e = w - 6 * q;
+			const double *blk = q == 1 ? S.v : q == 2 ? S.f : S.a;
+			v = ((const int *)(blk + (e / 2) * slots + g))[e & 1];
+		} else if (w < 27) {
+			v = S.cr[(w - 24) * slots + g];
+		}
+		rec[(y.off + S.orig[g]) * SEPDEV_BATCH_WORDS + w] = v;
+	}
+}
+
+// Starts the download of the first nsys systems' records in *nchunk chunks
+// of whole systems.  Per-system results (and errors) come from
+// sepdev_batch_scalars before it.
+extern "C" int sepdev_batch_get_open(sepdev_batch *b, int nsys, int *nchunk)
+{
+	int k = 0, s = 0;
+	long left = 0;
+	for (int i = 0; i < nsys; i++)
+		left += b->hsys[i].npad;
+	while (s < nsys) {
+		// equal shares of what is left, by atoms
+		const long share = k + 1 < SEPK_CHUNKS ? left / (SEPK_CHUNKS - k) : left;
+		const int s0 = s;
+		long atoms = 0;
+		int widest = 0;
+		while (s < nsys && (s == s0 || atoms + b->hsys[s].npad <= share ||
+				    atoms + b->hsys[s].npad <= SEPK_CHUNK_ATOMS ||
+				    k + 1 == SEPK_CHUNKS)) {
+			atoms += b->hsys[s].npad;
+			if (b->hsys[s].n > widest)
+				widest = b->hsys[s].n;
+			s++;
+		}
+		left -= atoms;
+		for (int q = s0; q < s; q += 32768) // grid.y limit
+			k_bgather<<<dim3((widest + SEPB_REC_ATOMS - 1) / SEPB_REC_ATOMS,
+					 s - q < 32768 ? s - q : 32768),
+				    SEPB_BLOCK, 0, b->st>>>(b->dsys, b->dS, b->slots, q, b->hrec);
+		SEPK_LAUNCH_CHECK();
+		SEPK_CHECK(hipEventRecord(b->chunk_ev[k], b->st));
+		b->chunk_sys[k++] = s;
+	}
+	*nchunk = k;
+	return 0;
+}
+
+// Waits for chunk k and gives its systems [*s0, *s1); any thread may call it.
+extern "C" int sepdev_batch_get_chunk(sepdev_batch *b, int k, int *s0, int *s1)
+{
+	*s0 = k ? b->chunk_sys[k - 1] : 0;
+	*s1 = b->chunk_sys[k];
+	return (int)hipEventSynchronize(b->chunk_ev[k]);
+}
+
+extern "C" const char *sepdev_batch_records(const sepdev_batch *b, int s)
+{
+	return (const char *)(b->hrec + (size_t)b->hsys[s].off * SEPDEV_BATCH_WORDS);
+}
+
+// Waits for the batch and reads every system's descriptor.
+extern "C" int sepdev_batch_fetch(sepdev_batch *b)
+{
+	return get_sys(b);
+}
+
+// The results of system s as last fetched; its device error, if any.
+extern "C" int sepdev_batch_scalars(sepdev_batch *b, int s, double *ret, double *scal)
 {
 	if (s < 0 || s >= b->nsys)
 		return sepk_fail(SEP_GPU_EARG, "batch: system %d", s);
-	int rc = get_sys(b);
-	if (rc)
-		return rc;
 	const sepb_sys &y = b->hsys[s];
-	const sepb_state &S = b->S[y.cur];
-	const long n = y.n, slots = b->slots;
-	sepk_pos *hp = (sepk_pos *)malloc(n * sizeof(sepk_pos));
-	double *hv = (double *)malloc(3 * n * sizeof(double));
-	int *ho = (int *)malloc(n * sizeof(int));
-	int *hi = (int *)malloc(3 * n * sizeof(int));
-	hipError_t e = hipMemcpy(ho, S.orig + y.off, n * sizeof(int), hipMemcpyDeviceToHost);
-	if (e == hipSuccess && x) {
-		e = hipMemcpy(hp, S.pos[y.p] + y.off, n * sizeof(sepk_pos), hipMemcpyDeviceToHost);
-		for (long t = 0; t < n && e == hipSuccess; t++) {
-			x[3 * ho[t]] = hp[t].x;
-			x[3 * ho[t] + 1] = hp[t].y;
-			x[3 * ho[t] + 2] = hp[t].z;
-		}
-	}
-	double *fields[3] = {v, f, a};
-	double *src[3] = {S.v, S.f, S.a};
-	for (int q = 0; q < 3 && e == hipSuccess; q++) {
-		if (!fields[q])
-			continue;
-		for (int k = 0; k < 3 && e == hipSuccess; k++)
-			e = hipMemcpy(hv + k * n, src[q] + k * slots + y.off, n * sizeof(double),
-				      hipMemcpyDeviceToHost);
-		for (long t = 0; t < n && e == hipSuccess; t++)
-			for (int k = 0; k < 3; k++)
-				fields[q][3 * ho[t] + k] = hv[k * n + t];
-	}
-	if (cr && e == hipSuccess) {
-		for (int k = 0; k < 3 && e == hipSuccess; k++)
-			e = hipMemcpy(hi + k * n, S.cr + k * slots + y.off, n * sizeof(int),
-				      hipMemcpyDeviceToHost);
-		for (long t = 0; t < n && e == hipSuccess; t++)
-			for (int k = 0; k < 3; k++)
-				cr[3 * ho[t] + k] = hi[k * n + t];
-	}
-	free(hp);
-	free(hv);
-	free(ho);
-	free(hi);
-	if (e != hipSuccess)
-		return sepk_fail(SEP_GPU_EDEVICE, "batch: download: %s", hipGetErrorString(e));
-	if (ret)
-		memcpy(ret, y.ret, SEPDEV_RET_WORDS * sizeof(double));
-	if (scal) {
-		scal[0] = y.alpha;
-		scal[1] = y.max_dist2;
-		scal[2] = y.tnow;
-		scal[3] = y.nupdate;
-		scal[4] = y.neighb_flag;
-		scal[5] = y.max_full;
-		scal[6] = y.error;
-		scal[7] = y.sumv2;
-	}
+	memcpy(ret, y.ret, SEPDEV_RET_WORDS * sizeof(double));
+	scal[0] = y.alpha;
+	scal[1] = y.max_dist2;
+	scal[2] = y.tnow;
+	scal[3] = y.nupdate;
+	scal[4] = y.neighb_flag;
 	if (y.error)
 		return sepk_fail(y.error, "batch: system %d: device error %d%s", s, y.error,
 				 y.error == SEP_GPU_ENEIGHB ? " (neighbour list overflow)" : "");

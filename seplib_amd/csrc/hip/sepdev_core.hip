@@ -158,12 +158,14 @@ extern "C" sepdev *sepdev_create(long npart, int *err)
 	d->ret_zero = (unsigned char *)calloc(d->ret_cap, 1);
 	d->scal_cap = 16;
 	rc |= dalloc(&d->scal, d->scal_cap);
-	d->stage_bytes = (size_t)d->npad * 40 * sizeof(int);
-	if (d->stage_bytes < (size_t)d->npad * 3 * sizeof(double))
-		d->stage_bytes = (size_t)d->npad * 3 * sizeof(double);
-	if (hipHostMalloc(&d->hstage, d->stage_bytes, hipHostMallocDefault) != hipSuccess)
+	if (hipHostMalloc(&d->hstage,
+			  SEPK_HEAD_BYTES + (size_t)d->npad * SEPK_REC_WORDS * sizeof(int),
+			  hipHostMallocDefault) != hipSuccess)
 		rc |= sepk_fail(SEP_GPU_EDEVICE, "hipHostMalloc staging failed");
-	rc |= dalloc((char **)&d->dstage, d->stage_bytes);
+	d->hrec = (char *)d->hstage + SEPK_HEAD_BYTES;
+	for (hipEvent_t &ev : d->chunk_ev)
+		if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess)
+			rc |= sepk_fail(SEP_GPU_EDEVICE, "hipEventCreate failed");
 	if (rc) {
 		*err = rc;
 		sepdev_destroy(d);
@@ -200,7 +202,7 @@ extern "C" void sepdev_destroy(sepdev *d)
 	void *ptrs[] = {d->iperm, d->cell_count, d->cell_start,
 			d->cellid_old, d->order_tmp, d->cell_slot,
 			d->nbr, d->nbr_count, d->partials, d->fin_l2, d->ring, d->ring_n, d->ret,
-			d->scal, d->sys, d->dstage, d->blist, d->alist, d->dlist,
+			d->scal, d->sys, d->blist, d->alist, d->dlist,
 			d->bcontrib, d->acontrib, d->dcontrib, d->bcsr_off,
 			d->bcsr_idx, d->acsr_off, d->acsr_idx, d->dcsr_off,
 			d->dcsr_idx, d->blen, d->aval, d->dval};
@@ -209,6 +211,9 @@ extern "C" void sepdev_destroy(sepdev *d)
 			(void)hipFree(p);
 	if (d->hstage)
 		(void)hipHostFree(d->hstage);
+	for (hipEvent_t ev : d->chunk_ev)
+		if (ev)
+			(void)hipEventDestroy(ev);
 	free(d->ret_zero);
 	free(d->last_lj);
 	(void)hipFree(d->pos_alt);
@@ -237,79 +242,115 @@ extern "C" void sepdev_destroy(sepdev *d)
 
 // ---- transfers ----------------------------------------------------------------
 
-// dst block (3 x npad, device order) <- src (3n interleaved, original order)
-__global__ void k_scatter_vec(double *dst, const double *src, const int *iperm,
-			      long n, long npad)
+// Atoms cross the host link as records: the 4-byte words of the chosen
+// fields of one atom, side by side, atoms in original order, in pinned host
+// memory that the kernels read and write themselves.  One call of the API
+// moves all of its fields with one launch and the host layer packs or unpacks
+// an atom's fields in one visit.  With a launch, a copy through a staging
+// array and a pass over the atoms per field, a resident system took 0.19, 0.53,
+// 9.8 and 18.6 ms to synchronise at 1000, 27000, 256000 and 500000 atoms; it
+// takes 0.07, 0.25, 1.6 and 3.0 ms (4.4 and 9.0 ms where one host thread
+// unpacks).
+// Consecutive lanes take consecutive words, so the link sees whole 64-byte
+// accesses whatever order the device keeps the atoms in.
+struct sepk_rec {
+	int nw;                     // words per record
+	int byte;                   // the word that is a single byte on the device, or -1
+	int stride[SEPK_REC_WORDS]; // words (bytes for `byte`) between two atoms
+	char *base[SEPK_REC_WORDS]; // the word of device atom 0
+};
+
+#define SEPK_REC_ATOMS 64 // atoms per workgroup
+
+static void rec_add(sepk_rec &r, void *base, int words, int stride)
 {
-	long o = (long)blockIdx.x * blockDim.x + threadIdx.x;
-	if (o >= n)
-		return;
-	const long t = iperm[o];
-	dst[t] = src[3 * o];
-	dst[npad + t] = src[3 * o + 1];
-	dst[2 * npad + t] = src[3 * o + 2];
+	for (int h = 0; h < words; h++) {
+		r.stride[r.nw] = stride;
+		r.base[r.nw++] = (char *)base + 4 * h;
+	}
 }
 
-__global__ void k_scatter_pos(sepk_pos *pos, const double *src, const int *iperm,
-			      long n)
+// x, y, z blocks of npad elements of `words` words
+static void rec_add3(sepk_rec &r, void *blocks, long npad, int words)
 {
-	long o = (long)blockIdx.x * blockDim.x + threadIdx.x;
-	if (o >= n)
-		return;
-	const long t = iperm[o];
-	sepk_pos p = pos[t];
-	p.x = src[3 * o];
-	p.y = src[3 * o + 1];
-	p.z = src[3 * o + 2];
-	pos[t] = p;
+	for (int k = 0; k < 3; k++)
+		rec_add(r, (char *)blocks + (size_t)k * npad * words * 4, words, words);
 }
 
-__global__ void k_gather_vec(double *dst, const double *src, const int *iperm,
-			     long n, long npad)
+// The record of a field mask; the order is the one sepdev.h states.
+static sepk_rec rec_of(const sepdev *d, unsigned mask)
 {
-	long o = (long)blockIdx.x * blockDim.x + threadIdx.x;
-	if (o >= n)
-		return;
-	const long t = iperm[o];
-	dst[3 * o] = src[t];
-	dst[3 * o + 1] = src[npad + t];
-	dst[3 * o + 2] = src[2 * npad + t];
+	sepk_rec r;
+	r.nw = 0;
+	r.byte = -1;
+	const sepk_state &s = d->s[0];
+	if (mask & SEPDEV_X)
+		rec_add(r, s.pos, 6, sizeof(sepk_pos) / 4);
+	if (mask & SEPDEV_V)
+		rec_add3(r, s.v, d->npad, 2);
+	if (mask & SEPDEV_F)
+		rec_add3(r, s.f, d->npad, 2);
+	if (mask & SEPDEV_A)
+		rec_add3(r, s.a, d->npad, 2);
+	if (mask & SEPDEV_XN)
+		rec_add3(r, s.xn, d->npad, 2);
+	if (mask & SEPDEV_SCALARS) {
+		rec_add(r, s.m, 2, 2);
+		rec_add(r, &s.pos->q, 2, sizeof(sepk_pos) / 4);
+	}
+	if (mask & SEPDEV_CROSS_NB)
+		rec_add3(r, s.cn, d->npad, 1);
+	if (mask & SEPDEV_CROSS)
+		rec_add3(r, s.cr, d->npad, 1);
+	if (mask & SEPDEV_SCALARS) {
+		rec_add(r, s.mol, 1, 1);
+		r.byte = r.nw;
+		rec_add(r, s.type, 1, 1);
+	}
+	return r;
 }
 
-__global__ void k_gather_pos(double *dst, const sepk_pos *pos, const int *iperm,
-			     long n)
+// records [o0, n) of the host buffer -> device fields
+__global__ void k_scatter_records(sepk_rec r, const int *rec, const int *iperm, long n)
 {
-	long o = (long)blockIdx.x * blockDim.x + threadIdx.x;
-	if (o >= n)
-		return;
-	const sepk_pos p = pos[iperm[o]];
-	dst[3 * o] = p.x;
-	dst[3 * o + 1] = p.y;
-	dst[3 * o + 2] = p.z;
+	const long o0 = (long)blockIdx.x * SEPK_REC_ATOMS;
+	for (int j = threadIdx.x; j < SEPK_REC_ATOMS * r.nw; j += SEPK_BLOCK) {
+		const int a = j / r.nw, w = j - a * r.nw;
+		if (o0 + a >= n)
+			return;
+		const int v = rec[(size_t)o0 * r.nw + j];
+		const size_t t = (size_t)iperm[o0 + a] * r.stride[w];
+		if (w == r.byte)
+			((signed char *)r.base[w])[t] = (signed char)v;
+		else
+			((int *)r.base[w])[t] = v;
+	}
 }
 
-__global__ void k_scatter_ivec(int *dst, const int *src, const int *iperm,
-			       long n, long npad)
+// device fields -> records [o0, o1) of the host buffer
+__global__ void k_gather_records(sepk_rec r, int *rec, const int *iperm, long o0, long o1)
 {
-	long o = (long)blockIdx.x * blockDim.x + threadIdx.x;
-	if (o >= n)
-		return;
-	const long t = iperm[o];
-	dst[t] = src[3 * o];
-	dst[npad + t] = src[3 * o + 1];
-	dst[2 * npad + t] = src[3 * o + 2];
+	const long b0 = o0 + (long)blockIdx.x * SEPK_REC_ATOMS;
+	for (int j = threadIdx.x; j < SEPK_REC_ATOMS * r.nw; j += SEPK_BLOCK) {
+		const int a = j / r.nw, w = j - a * r.nw;
+		if (b0 + a >= o1)
+			return;
+		rec[(size_t)b0 * r.nw + j] =
+			((const int *)r.base[w])[(size_t)iperm[b0 + a] * r.stride[w]];
+	}
 }
 
-__global__ void k_gather_ivec(int *dst, const int *src, const int *iperm,
-			      long n, long npad)
+static unsigned rec_blocks(long atoms)
 {
-	long o = (long)blockIdx.x * blockDim.x + threadIdx.x;
-	if (o >= n)
-		return;
-	const long t = iperm[o];
-	dst[3 * o] = src[t];
-	dst[3 * o + 1] = src[npad + t];
-	dst[3 * o + 2] = src[2 * npad + t];
+	return (unsigned)((atoms + SEPK_REC_ATOMS - 1) / SEPK_REC_ATOMS);
+}
+
+static int scatter_records(sepdev *d, const sepk_rec &r)
+{
+	k_scatter_records<<<rec_blocks(d->n), SEPK_BLOCK, 0, d->st>>>(r, (const int *)d->hrec,
+								      d->iperm, d->n);
+	SEPK_LAUNCH_CHECK();
+	return 0;
 }
 
 __global__ void k_zero_blocks(double *p, long count)
@@ -319,38 +360,66 @@ __global__ void k_zero_blocks(double *p, long count)
 		p[t] = 0.0;
 }
 
-static int stage_in(sepdev *d, const void *src, size_t bytes)
+// A few words between the host and the device: the kernel writes pinned
+// memory, or carries the words in its arguments, where a copy of its own would
+// go through the copy queue and, on the way in, have to be waited for.
+#define SEPK_SMALL_WORDS 64
+struct sepk_words {
+	int w[SEPK_SMALL_WORDS];
+};
+
+__global__ void k_fetch_words(int *dst, const int *src, int n)
 {
-	if (bytes > d->stage_bytes)
-		return sepk_fail(SEP_GPU_EARG, "staging overflow (%zu bytes)", bytes);
-	// the pinned buffer may still feed an earlier copy
-	SEPK_CHECK(hipStreamSynchronize(d->st));
-	memcpy(d->hstage, src, bytes);
-	SEPK_CHECK(hipMemcpyAsync(d->dstage, d->hstage, bytes, hipMemcpyHostToDevice, d->st));
-	return 0;
+	if ((int)threadIdx.x < n)
+		dst[threadIdx.x] = src[threadIdx.x];
 }
 
-static int stage_out(sepdev *d, void *dst, size_t bytes)
+__global__ void k_store_words(int *dst, sepk_words w, int n)
 {
-	SEPK_CHECK(hipMemcpyAsync(d->hstage, d->dstage, bytes, hipMemcpyDeviceToHost, d->st));
+	if ((int)threadIdx.x < n)
+		dst[threadIdx.x] = w.w[threadIdx.x];
+}
+
+static int fetch_words(sepdev *d, void *dst, const void *src, size_t bytes)
+{
+	if (d->capturing)
+		return sepk_fail(SEP_GPU_ESTATE, "transfer during graph capture");
+	if (bytes > sizeof(sepk_words) || bytes % 4)
+		return sepk_fail(SEP_GPU_EARG, "fetch of %zu bytes", bytes);
+	k_fetch_words<<<1, SEPK_SMALL_WORDS, 0, d->st>>>((int *)d->hstage, (const int *)src,
+							 (int)(bytes / 4));
+	SEPK_LAUNCH_CHECK();
 	SEPK_CHECK(hipStreamSynchronize(d->st));
 	memcpy(dst, d->hstage, bytes);
 	return 0;
 }
 
-static double *vec_field(sepdev *d, int which)
+static int store_words(sepdev *d, void *dst, const void *src, size_t bytes)
 {
-	sepk_state &s = d->s[0];
-	switch (which) {
-	case SEPDEV_V: return s.v;
-	case SEPDEV_F: return s.f;
-	case SEPDEV_A: return s.a;
-	case SEPDEV_XN: return s.xn;
-	}
-	return nullptr;
+	if (d->capturing)
+		return sepk_fail(SEP_GPU_ESTATE, "transfer during graph capture");
+	if (bytes > sizeof(sepk_words) || bytes % 4)
+		return sepk_fail(SEP_GPU_EARG, "store of %zu bytes", bytes);
+	sepk_words w;
+	memset(&w, 0, sizeof w);
+	memcpy(&w, src, bytes);
+	k_store_words<<<1, SEPK_SMALL_WORDS, 0, d->st>>>((int *)dst, w, (int)(bytes / 4));
+	SEPK_LAUNCH_CHECK();
+	return 0;
 }
 
-extern "C" int sepdev_put_vec(sepdev *d, int which, const double *src3n)
+extern "C" int sepdev_record_bytes(unsigned mask)
+{
+	int w = 0;
+	for (unsigned f = SEPDEV_X; f <= SEPDEV_XN; f <<= 1)
+		w += mask & f ? 6 : 0;
+	w += mask & SEPDEV_SCALARS ? 6 : 0;
+	w += mask & SEPDEV_CROSS_NB ? 3 : 0;
+	w += mask & SEPDEV_CROSS ? 3 : 0;
+	return 4 * w;
+}
+
+extern "C" int sepdev_put_open(sepdev *d, char **rec)
 {
 	if (d->capturing)
 		return sepk_fail(SEP_GPU_ESTATE, "transfer during graph capture");
@@ -358,158 +427,96 @@ extern "C" int sepdev_put_vec(sepdev *d, int which, const double *src3n)
 	int rc = sepk_flush_nh(d);
 	if (rc || (rc = sepk_flush_gathers(d)))
 		return rc;
-	if (which == SEPDEV_V)
-		d->sumv2_valid = 0;
-	if ((rc = stage_in(d, src3n, (size_t)d->n * 3 * sizeof(double))))
-		return rc;
-	const unsigned nb = sepk_blocks(d->n);
-	if (which == SEPDEV_X) {
-		k_scatter_pos<<<nb, SEPK_BLOCK, 0, d->st>>>(d->s[0].pos, (const double *)d->dstage, d->iperm, d->n);
-		d->qpos_stale = 1; // requantized by the next mixed pair call
-	} else {
-		double *dst = vec_field(d, which);
-		if (!dst)
-			return sepk_fail(SEP_GPU_EARG, "put_vec: field %d", which);
-		k_scatter_vec<<<nb, SEPK_BLOCK, 0, d->st>>>(dst, (const double *)d->dstage, d->iperm, d->n, d->npad);
-		if (which == SEPDEV_F)
-			d->f_zero_pending = 0;
-	}
-	SEPK_LAUNCH_CHECK();
+	// the buffer may still feed an earlier launch
+	SEPK_CHECK(hipStreamSynchronize(d->st));
+	*rec = d->hrec;
 	return 0;
 }
 
-extern "C" int sepdev_get_vec(sepdev *d, int which, double *dst3n)
+extern "C" int sepdev_put_close(sepdev *d, unsigned mask)
+{
+	if (mask & (SEPDEV_V | SEPDEV_SCALARS))
+		d->sumv2_valid = 0;
+	if (mask & (SEPDEV_X | SEPDEV_SCALARS))
+		d->qpos_stale = 1; // requantized by the next mixed pair call
+	if (mask & SEPDEV_F)
+		d->f_zero_pending = 0;
+	return scatter_records(d, rec_of(d, mask));
+}
+
+extern "C" int sepdev_get_settle(sepdev *d, unsigned mask)
 {
 	if (d->capturing)
 		return sepk_fail(SEP_GPU_ESTATE, "transfer during graph capture");
-	const unsigned nb = sepk_blocks(d->n);
 	int rc = sepk_flush_nh(d);
+	if (!rc && (mask & SEPDEV_F))
+		rc = sepk_materialize_forces(d);
+	return rc;
+}
+
+extern "C" int sepdev_get_open(sepdev *d, unsigned mask, const char **rec, int *nchunk)
+{
+	int rc = sepdev_get_settle(d, mask);
 	if (rc)
 		return rc;
-	if (which == SEPDEV_F && (rc = sepk_materialize_forces(d)))
-		return rc;
-	if (which == SEPDEV_X) {
-		k_gather_pos<<<nb, SEPK_BLOCK, 0, d->st>>>((double *)d->dstage, d->s[0].pos, d->iperm, d->n);
-	} else {
-		double *src = vec_field(d, which);
-		if (!src)
-			return sepk_fail(SEP_GPU_EARG, "get_vec: field %d", which);
-		k_gather_vec<<<nb, SEPK_BLOCK, 0, d->st>>>((double *)d->dstage, src, d->iperm, d->n, d->npad);
+	long nc = (d->n + SEPK_CHUNK_ATOMS - 1) / SEPK_CHUNK_ATOMS;
+	if (nc > SEPK_CHUNKS)
+		nc = SEPK_CHUNKS;
+	d->chunk = (((d->n + nc - 1) / nc) + 63) / 64 * 64;
+	const sepk_rec r = rec_of(d, mask);
+	int k = 0;
+	for (long o = 0; o < d->n; o += d->chunk, k++) {
+		const long o1 = o + d->chunk < d->n ? o + d->chunk : d->n;
+		k_gather_records<<<rec_blocks(o1 - o), SEPK_BLOCK, 0, d->st>>>(
+			r, (int *)d->hrec, d->iperm, o, o1);
+		SEPK_LAUNCH_CHECK();
+		if (d->n > d->chunk)
+			SEPK_CHECK(hipEventRecord(d->chunk_ev[k], d->st));
 	}
-	SEPK_LAUNCH_CHECK();
-	return stage_out(d, dst3n, (size_t)d->n * 3 * sizeof(double));
+	*rec = d->hrec;
+	*nchunk = k;
+	return 0;
+}
+
+extern "C" int sepdev_get_chunk(sepdev *d, int k, long *i0, long *i1)
+{
+	*i0 = k * d->chunk;
+	*i1 = *i0 + d->chunk < d->n ? *i0 + d->chunk : d->n;
+	return d->n > d->chunk ? (int)hipEventSynchronize(d->chunk_ev[k])
+			       : (int)hipStreamSynchronize(d->st);
+}
+
+extern "C" int sepdev_get_failed(int code)
+{
+	return sepk_fail(SEP_GPU_EDEVICE, "download: %s", hipGetErrorString((hipError_t)code));
 }
 
 // A host 3n array in original order into / out of any 3 x npad device block
 // in device order (adjoint inputs and outputs).
 int sepk_put_vec_to(sepdev *d, double *dst, const double *src3n)
 {
-	int rc = stage_in(d, src3n, (size_t)d->n * 3 * sizeof(double));
-	if (rc)
-		return rc;
-	k_scatter_vec<<<sepk_blocks(d->n), SEPK_BLOCK, 0, d->st>>>(dst, (const double *)d->dstage, d->iperm, d->n, d->npad);
-	SEPK_LAUNCH_CHECK();
-	return 0;
+	// the buffer may still feed an earlier launch
+	SEPK_CHECK(hipStreamSynchronize(d->st));
+	memcpy(d->hrec, src3n, (size_t)d->n * 3 * sizeof(double));
+	sepk_rec r;
+	r.nw = 0;
+	r.byte = -1;
+	rec_add3(r, dst, d->npad, 2);
+	return scatter_records(d, r);
 }
 
 int sepk_get_vec_from(sepdev *d, double *dst3n, const double *src)
 {
-	k_gather_vec<<<sepk_blocks(d->n), SEPK_BLOCK, 0, d->st>>>((double *)d->dstage, src, d->iperm, d->n, d->npad);
+	sepk_rec r;
+	r.nw = 0;
+	r.byte = -1;
+	rec_add3(r, (void *)src, d->npad, 2);
+	k_gather_records<<<rec_blocks(d->n), SEPK_BLOCK, 0, d->st>>>(r, (int *)d->hrec, d->iperm, 0,
+								     d->n);
 	SEPK_LAUNCH_CHECK();
-	return stage_out(d, dst3n, (size_t)d->n * 3 * sizeof(double));
-}
-
-extern "C" int sepdev_put_ivec(sepdev *d, int which, const int *src3n)
-{
-	int rc = stage_in(d, src3n, (size_t)d->n * 3 * sizeof(int));
-	if (rc)
-		return rc;
-	int *dst = which == SEPDEV_CROSS_NB ? d->s[0].cn : d->s[0].cr;
-	k_scatter_ivec<<<sepk_blocks(d->n), SEPK_BLOCK, 0, d->st>>>(dst, (const int *)d->dstage, d->iperm, d->n, d->npad);
-	SEPK_LAUNCH_CHECK();
-	return 0;
-}
-
-extern "C" int sepdev_get_ivec(sepdev *d, int which, int *dst3n)
-{
-	const int *src = which == SEPDEV_CROSS_NB ? d->s[0].cn : d->s[0].cr;
-	k_gather_ivec<<<sepk_blocks(d->n), SEPK_BLOCK, 0, d->st>>>((int *)d->dstage, src, d->iperm, d->n, d->npad);
-	SEPK_LAUNCH_CHECK();
-	return stage_out(d, dst3n, (size_t)d->n * 3 * sizeof(int));
-}
-
-__global__ void k_scatter_scalars(sepk_state s, const double *mass, const double *q,
-				  const signed char *type, const int *mol,
-				  const int *iperm, long n)
-{
-	long o = (long)blockIdx.x * blockDim.x + threadIdx.x;
-	if (o >= n)
-		return;
-	const long t = iperm[o];
-	if (mass)
-		s.m[t] = mass[o];
-	if (q)
-		s.pos[t].q = q[o];
-	if (type)
-		s.type[t] = type[o];
-	if (mol)
-		s.mol[t] = mol[o];
-}
-
-extern "C" int sepdev_put_scalars(sepdev *d, const double *mass, const double *charge,
-				  const signed char *type, const int *molindex)
-{
-	// pack into one staging upload: mass | charge | mol | type
-	const long n = d->n;
-	if (mass)
-		d->sumv2_valid = 0;
-	if (charge)
-		d->qpos_stale = 1; // the quantized records carry the charges
-	const size_t bytes = (size_t)n * (2 * sizeof(double) + sizeof(int) + 1);
-	if (bytes > d->stage_bytes)
-		return sepk_fail(SEP_GPU_EARG, "staging overflow");
 	SEPK_CHECK(hipStreamSynchronize(d->st));
-	char *h = (char *)d->hstage;
-	double *hm = (double *)h;
-	double *hq = hm + n;
-	int *hmol = (int *)(hq + n);
-	signed char *ht = (signed char *)(hmol + n);
-	if (mass) memcpy(hm, mass, n * sizeof(double));
-	if (charge) memcpy(hq, charge, n * sizeof(double));
-	if (molindex) memcpy(hmol, molindex, n * sizeof(int));
-	if (type) memcpy(ht, type, n);
-	SEPK_CHECK(hipMemcpyAsync(d->dstage, d->hstage, bytes, hipMemcpyHostToDevice, d->st));
-	char *g = (char *)d->dstage;
-	double *gm = (double *)g;
-	double *gq = gm + n;
-	int *gmol = (int *)(gq + n);
-	signed char *gt = (signed char *)(gmol + n);
-	k_scatter_scalars<<<sepk_blocks(n), SEPK_BLOCK, 0, d->st>>>(
-		d->s[0], mass ? gm : nullptr, charge ? gq : nullptr,
-		type ? gt : nullptr, molindex ? gmol : nullptr, d->iperm, n);
-	SEPK_LAUNCH_CHECK();
+	memcpy(dst3n, d->hrec, (size_t)d->n * 3 * sizeof(double));
 	return 0;
-}
-
-extern "C" int sepdev_put_charges(sepdev *d, const double *charge)
-{
-	return sepdev_put_scalars(d, nullptr, charge, nullptr, nullptr);
-}
-
-extern "C" int sepdev_put_types(sepdev *d, const signed char *type)
-{
-	return sepdev_put_scalars(d, nullptr, nullptr, type, nullptr);
-}
-
-__global__ void k_scatter_partners(int *dst, const int *src, const int *iperm,
-				   long n, long npad)
-{
-	long o = (long)blockIdx.x * blockDim.x + threadIdx.x;
-	if (o >= n)
-		return;
-	const long t = iperm[o];
-	for (int k = 0; k < 40; k++)
-		dst[k * npad + t] = src[40 * o + k];
 }
 
 extern "C" int sepdev_put_partners(sepdev *d, const int *partners40n)
@@ -520,13 +527,16 @@ extern "C" int sepdev_put_partners(sepdev *d, const int *partners40n)
 			if (rc)
 				return rc;
 		}
-	int rc = stage_in(d, partners40n, (size_t)d->n * 40 * sizeof(int));
-	if (rc)
-		return rc;
-	k_scatter_partners<<<sepk_blocks(d->n), SEPK_BLOCK, 0, d->st>>>(
-		d->s[0].partners, (const int *)d->dstage, d->iperm, d->n, d->npad);
-	SEPK_LAUNCH_CHECK();
-	return 0;
+	if (d->capturing)
+		return sepk_fail(SEP_GPU_ESTATE, "transfer during graph capture");
+	SEPK_CHECK(hipStreamSynchronize(d->st));
+	memcpy(d->hrec, partners40n, (size_t)d->n * 40 * sizeof(int));
+	sepk_rec r;
+	r.nw = 0;
+	r.byte = -1;
+	for (int k = 0; k < 40; k++)
+		rec_add(r, d->s[0].partners + (size_t)k * d->npad, 1, 1);
+	return scatter_records(d, r);
 }
 
 extern "C" int sepdev_put_sys(sepdev *d, const sepdev_sys *s)
@@ -534,10 +544,7 @@ extern "C" int sepdev_put_sys(sepdev *d, const sepdev_sys *s)
 	// the host record replaces everything, including the cached sum m v^2
 	d->max_reset_pending = 0;
 	d->sumv2_valid = 0;
-	SEPK_CHECK(hipStreamSynchronize(d->st));
-	memcpy(d->hstage, s, sizeof *s);
-	SEPK_CHECK(hipMemcpyAsync(d->sys, d->hstage, sizeof *s, hipMemcpyHostToDevice, d->st));
-	return 0;
+	return store_words(d, d->sys, s, sizeof *s);
 }
 
 extern "C" int sepdev_get_sys(sepdev *d, sepdev_sys *s)
@@ -545,12 +552,10 @@ extern "C" int sepdev_get_sys(sepdev *d, sepdev_sys *s)
 	int rc = sepk_flush_tasks(d);
 	if (rc)
 		return rc;
-	SEPK_CHECK(hipMemcpyAsync(d->hstage, d->sys, sizeof *s, hipMemcpyDeviceToHost, d->st));
-	SEPK_CHECK(hipStreamSynchronize(d->st));
-	memcpy(s, d->hstage, sizeof *s);
-	if (d->max_reset_pending)
+	rc = fetch_words(d, s, d->sys, sizeof *s);
+	if (!rc && d->max_reset_pending)
 		s->max_dist2 = 0.0;
-	return 0;
+	return rc;
 }
 
 // ---- slots --------------------------------------------------------------------
@@ -597,24 +602,17 @@ extern "C" int sepdev_ret_get(sepdev *d, int slot, double *words)
 		SEPK_LAUNCH_CHECK();
 		d->ret_zero[slot] = 0;
 	}
-	SEPK_CHECK(hipMemcpyAsync(d->hstage, d->ret + (size_t)slot * SEPDEV_RET_WORDS,
-				  SEPDEV_RET_WORDS * sizeof(double), hipMemcpyDeviceToHost, d->st));
-	SEPK_CHECK(hipStreamSynchronize(d->st));
-	memcpy(words, d->hstage, SEPDEV_RET_WORDS * sizeof(double));
-	return 0;
+	return fetch_words(d, words, d->ret + (size_t)slot * SEPDEV_RET_WORDS,
+			   SEPDEV_RET_WORDS * sizeof(double));
 }
 
 extern "C" int sepdev_ret_put(sepdev *d, int slot, const double *words)
 {
 	if (slot < 0 || slot >= d->nret)
 		return sepk_fail(SEP_GPU_EARG, "ret slot %d", slot);
-	SEPK_CHECK(hipStreamSynchronize(d->st));
 	d->ret_zero[slot] = 0;
-	memcpy(d->hstage, words, SEPDEV_RET_WORDS * sizeof(double));
-	SEPK_CHECK(hipMemcpyAsync(d->ret + (size_t)slot * SEPDEV_RET_WORDS, d->hstage,
-				  SEPDEV_RET_WORDS * sizeof(double), hipMemcpyHostToDevice, d->st));
-	SEPK_CHECK(hipStreamSynchronize(d->st));
-	return 0;
+	return store_words(d, d->ret + (size_t)slot * SEPDEV_RET_WORDS, words,
+			   SEPDEV_RET_WORDS * sizeof(double));
 }
 
 extern "C" int sepdev_scalar_alloc(sepdev *d, double init)
@@ -640,19 +638,12 @@ extern "C" int sepdev_scalar_get(sepdev *d, int slot, double *v)
 	int rc = sepk_flush_nh(d);
 	if (rc || (rc = sepk_flush_tasks(d)))
 		return rc;
-	SEPK_CHECK(hipMemcpyAsync(d->hstage, d->scal + slot, sizeof(double), hipMemcpyDeviceToHost, d->st));
-	SEPK_CHECK(hipStreamSynchronize(d->st));
-	memcpy(v, d->hstage, sizeof(double));
-	return 0;
+	return fetch_words(d, v, d->scal + slot, sizeof(double));
 }
 
 extern "C" int sepdev_scalar_put(sepdev *d, int slot, double v)
 {
-	SEPK_CHECK(hipStreamSynchronize(d->st));
-	memcpy(d->hstage, &v, sizeof(double));
-	SEPK_CHECK(hipMemcpyAsync(d->scal + slot, d->hstage, sizeof(double), hipMemcpyHostToDevice, d->st));
-	SEPK_CHECK(hipStreamSynchronize(d->st));
-	return 0;
+	return store_words(d, d->scal + slot, &v, sizeof(double));
 }
 
 // ---- misc -----------------------------------------------------------------------

@@ -132,6 +132,13 @@ struct sepk_timer {
 	long count;
 };
 
+// Transfers.  A download is launched in chunks so that the host unpacks one
+// while the next crosses the link.
+#define SEPK_HEAD_BYTES 4096
+#define SEPK_REC_WORDS 42
+#define SEPK_CHUNKS 16
+#define SEPK_CHUNK_ATOMS 16384
+
 struct sepdev {
 	long n, npad;
 	hipStream_t st;
@@ -173,8 +180,10 @@ struct sepdev {
 	sepdev_sys *sys;
 
 	// staging
-	void *hstage, *dstage;
-	size_t stage_bytes;
+	void *hstage;  // pinned: SEPK_HEAD_BYTES for small results, then hrec
+	char *hrec;    // pinned atom records (SEPK_REC_WORDS words an atom at most)
+	long chunk;    // atoms per chunk of the download under way
+	hipEvent_t chunk_ev[SEPK_CHUNKS]; // a chunk's records are complete
 
 	// Deferred work, decided on the host so that a captured step replays
 	// the same kernels every time:

@@ -151,56 +151,70 @@ int sep_gpu_batch_synchronize(sep_gpu_batch *b)
 	return seph_dev_fail(sepdev_batch_synchronize(b->dev));
 }
 
+static int unpack_systems(void *arg, int k)
+{
+	sep_gpu_batch *b = arg;
+	int s0, s1;
+	const int rc = sepdev_batch_get_chunk(b->dev, k, &s0, &s1);
+	if (rc)
+		return rc;
+	for (int s = s0; s < s1; s++) {
+		const char *r = sepdev_batch_records(b->dev, s);
+		for (long i = 0; i < b->sys[s]->npart; i++, r += SEPDEV_BATCH_WORDS * sizeof(int)) {
+			seppart *p = &b->atoms[s][i];
+			memcpy(p->x, r, sizeof p->x);
+			memcpy(p->v, r + 24, sizeof p->v);
+			memcpy(p->f, r + 48, sizeof p->f);
+			memcpy(p->a, r + 72, sizeof p->a);
+			memcpy(p->crossings, r + 96, sizeof p->crossings);
+		}
+	}
+	return 0;
+}
+
 int sep_gpu_batch_sync(sep_gpu_batch *b, sepret *rets, double *alpha)
 {
 	if (!b)
 		return seph_fail(SEP_GPU_EARG, "batch: null");
-	int rc = 0;
-	for (int s = 0; s < b->nsys && !rc; s++) {
-		sepsys *y = b->sys[s];
-		seppart *p = b->atoms[s];
-		const long n = y->npart;
-		double *x = malloc(3 * n * sizeof(double));
-		double *v = malloc(3 * n * sizeof(double));
-		double *f = malloc(3 * n * sizeof(double));
-		double *a = malloc(3 * n * sizeof(double));
-		int *cr = malloc(3 * n * sizeof(int));
-		double w[SEPDEV_RET_WORDS], scal[8];
-		rc = seph_dev_fail(sepdev_batch_get(b->dev, s, x, v, f, a, cr, w, scal));
-		if (!rc) {
-			for (long i = 0; i < n; i++)
-				for (int k = 0; k < 3; k++) {
-					p[i].x[k] = x[3 * i + k];
-					p[i].v[k] = v[3 * i + k];
-					p[i].f[k] = f[3 * i + k];
-					p[i].a[k] = a[3 * i + k];
-					p[i].crossings[k] = cr[3 * i + k];
-				}
-			y->max_dist2 = scal[1];
-			y->tnow = scal[2];
-			y->nupdate_neighb = (int)scal[3];
-			y->neighb_flag = (int)scal[4];
-			if (rets) {
-				sepret *r = &rets[s];
-				r->epot = w[SEPDEV_RET_EPOT];
-				r->ecoul = w[SEPDEV_RET_ECOUL];
-				r->ekin = w[SEPDEV_RET_EKIN];
-				for (int i = 0; i < 3; i++)
-					for (int k = 0; k < 3; k++) {
-						r->pot_P[i][k] = w[SEPDEV_RET_POTP + 3 * i + k];
-						r->kin_P[i][k] = w[SEPDEV_RET_KINP + 3 * i + k];
-					}
-			}
-			if (alpha)
-				alpha[s] = scal[0];
-		}
-		free(x);
-		free(v);
-		free(f);
-		free(a);
-		free(cr);
+	int rc = seph_dev_fail(sepdev_batch_fetch(b->dev));
+	if (rc)
+		return rc;
+	/* the systems before the first one that failed, if any */
+	int ok = 0, failed = 0;
+	long atoms = 0;
+	double w[SEPDEV_RET_WORDS], scal[5];
+	for (; ok < b->nsys; ok++) {
+		if ((failed = seph_dev_fail(sepdev_batch_scalars(b->dev, ok, w, scal))))
+			break;
+		atoms += b->sys[ok]->npart;
 	}
-	return rc;
+	int nchunk = 0;
+	if ((rc = seph_dev_fail(sepdev_batch_get_open(b->dev, ok, &nchunk))))
+		return rc;
+	if ((rc = seph_run_jobs(nchunk, atoms, unpack_systems, b)))
+		return seph_dev_fail(sepdev_get_failed(rc));
+	for (int s = 0; s < ok; s++) {
+		sepsys *y = b->sys[s];
+		(void)sepdev_batch_scalars(b->dev, s, w, scal);
+		y->max_dist2 = scal[1];
+		y->tnow = scal[2];
+		y->nupdate_neighb = (int)scal[3];
+		y->neighb_flag = (int)scal[4];
+		if (rets) {
+			sepret *r = &rets[s];
+			r->epot = w[SEPDEV_RET_EPOT];
+			r->ecoul = w[SEPDEV_RET_ECOUL];
+			r->ekin = w[SEPDEV_RET_EKIN];
+			for (int i = 0; i < 3; i++)
+				for (int k = 0; k < 3; k++) {
+					r->pot_P[i][k] = w[SEPDEV_RET_POTP + 3 * i + k];
+					r->kin_P[i][k] = w[SEPDEV_RET_KINP + 3 * i + k];
+				}
+		}
+		if (alpha)
+			alpha[s] = scal[0];
+	}
+	return failed;
 }
 
 int sep_gpu_batch_set_shape(sep_gpu_batch *b, const int *lanes, int grid)

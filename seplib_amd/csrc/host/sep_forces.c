@@ -62,8 +62,8 @@ typedef struct {
 
 /* True when the type filter of source/sepprfrc.c:116-121 keeps every pair:
  * both labels equal and every atom carries that label.  ("AB" never keeps
- * an A-A pair, so it always needs the filter.)  Cached per context until
- * the types are uploaded again. */
+ * an A-A pair, so it always needs the filter.)  An upload of the types by a
+ * synchronised call has answered it; a resident system looks once. */
 static int types_cover_all(seph_ctx *c, const char *types)
 {
 	if (types[0] != types[1])
@@ -93,7 +93,7 @@ static int run_pairs(seppart *ptr, sepsys *sys, sepret *ret, pair_call *pc)
 	if (brute)
 		sys->omp_flag = false;
 	if (!c->resident) {
-		if ((rc = seph_put_x(c)) || (rc = seph_put_f(c)) || (rc = seph_put_scalars(c)))
+		if ((rc = seph_put(c, SEPDEV_X | SEPDEV_F | SEPDEV_SCALARS)))
 			return rc;
 		if (needs_partners(pc->opt) && (rc = seph_put_partners(c)))
 			return rc;
@@ -161,7 +161,7 @@ static int run_pairs(seppart *ptr, sepsys *sys, sepret *ret, pair_call *pc)
 	}
 	if (c->resident)
 		return 0;
-	if ((rc = seph_get_f(c)))
+	if ((rc = seph_get(c, SEPDEV_F)))
 		return rc;
 	return sync_ret_end(c, ret, assign, 0);
 }
@@ -237,7 +237,7 @@ void sep_coulomb_sf(seppart *ptr, double cf, sepsys *sys, sepret *retval,
 		goto out;
 	}
 	if (!c->resident) {
-		if ((rc = seph_put_x(c)) || (rc = seph_put_f(c)) || (rc = seph_put_scalars(c)))
+		if ((rc = seph_put(c, SEPDEV_X | SEPDEV_F | SEPDEV_SCALARS)))
 			goto out;
 		if ((rc = sync_ret_begin(c)))
 			goto out;
@@ -271,7 +271,7 @@ void sep_coulomb_sf(seppart *ptr, double cf, sepsys *sys, sepret *retval,
 	if ((rc = seph_dev_fail(sepdev_coulomb(c->dev, &a, slot))))
 		goto out;
 	if (!c->resident) {
-		if ((rc = seph_get_f(c)))
+		if ((rc = seph_get(c, SEPDEV_F)))
 			goto out;
 		rc = sync_ret_end(c, retval, 0, 0);
 	}
@@ -296,7 +296,7 @@ static void bonded_call(seppart *ptr, int kind, int type, const double *prm,
 	if ((rc = seph_put_topology(c, sys)))
 		goto out;
 	if (!c->resident) {
-		if ((rc = seph_put_x(c)) || (rc = seph_put_f(c)) || (rc = sync_ret_begin(c)))
+		if ((rc = seph_put(c, SEPDEV_X | SEPDEV_F)) || (rc = sync_ret_begin(c)))
 			goto out;
 	}
 	const int slot = ret_slot_for(c, ret);
@@ -322,7 +322,7 @@ static void bonded_call(seppart *ptr, int kind, int type, const double *prm,
 		goto out;
 	if (c->resident)
 		return;
-	if ((rc = seph_get_f(c)))
+	if ((rc = seph_get(c, SEPDEV_F)))
 		goto out;
 	if ((rc = sync_ret_end(c, ret, 0, kind == BONDED_BOND)))
 		goto out;
@@ -403,14 +403,14 @@ void sep_nosehoover(seppart *ptr, double Td, double *alpha, const double Q,
 		}
 	} else {
 		slot = c->alpha_scratch;
-		if ((rc = seph_put_v(c)) || (rc = seph_put_f(c)) || (rc = seph_put_scalars(c)) ||
+		if ((rc = seph_put(c, SEPDEV_V | SEPDEV_F | SEPDEV_SCALARS)) ||
 		    (rc = seph_dev_fail(sepdev_scalar_put(c->dev, slot, *alpha))))
 			goto out;
 	}
 	if ((rc = seph_dev_fail(sepdev_nosehoover(c->dev, Td, Q, sys->dt, slot))))
 		goto out;
 	if (!c->resident) {
-		if ((rc = seph_get_f(c)))
+		if ((rc = seph_get(c, SEPDEV_F)))
 			goto out;
 		rc = seph_dev_fail(sepdev_scalar_get(c->dev, slot, alpha));
 	}
@@ -445,14 +445,16 @@ void sep_leapfrog(seppart *ptr, sepsys *sys, sepret *retval)
 		ds.tnow = sys->tnow;
 		ds.nupdate_neighb = sys->nupdate_neighb;
 		ds.neighb_flag = 0;
-		if ((rc = seph_put_x(c)) || (rc = seph_put_v(c)) || (rc = seph_put_f(c)) ||
-		    (rc = seph_put_xn_cross(c)) || (rc = seph_put_scalars(c)) ||
+		if ((rc = seph_put(c, SEPDEV_X | SEPDEV_V | SEPDEV_F | SEPDEV_XN | SEPDEV_SCALARS |
+					    SEPDEV_CROSS_NB | SEPDEV_CROSS)) ||
 		    (rc = seph_dev_fail(sepdev_put_sys(c->dev, &ds))) || (rc = sync_ret_begin(c)))
 			goto out;
 		if ((rc = seph_dev_fail(sepdev_leapfrog(c->dev, sys->dt, sys->skin, sys->length,
 							 c->ret_scratch))))
 			goto out;
-		if ((rc = seph_get_state(c)) || (rc = seph_dev_fail(sepdev_get_sys(c->dev, &ds))))
+		if ((rc = seph_get(c, SEPDEV_X | SEPDEV_V | SEPDEV_A | SEPDEV_CROSS_NB |
+					    SEPDEV_CROSS)) ||
+		    (rc = seph_dev_fail(sepdev_get_sys(c->dev, &ds))))
 			goto out;
 		if ((rc = sync_ret_end(c, retval, 0, 0)))
 			goto out;
@@ -506,7 +508,7 @@ int sep_gpu_lj_adjoint(seppart *ptr, sepsys *sys, int ntypes, const char *types,
 	if (!c)
 		return sep_gpu_last_error();
 	int rc;
-	if (!c->resident && ((rc = seph_put_x(c)) || (rc = seph_put_scalars(c))))
+	if (!c->resident && ((rc = seph_put(c, SEPDEV_X | SEPDEV_SCALARS))))
 		return rc;
 	sepdev_ljtab_args ta;
 	memset(&ta, 0, sizeof ta);
@@ -534,7 +536,7 @@ int sep_gpu_lj_adjoint_noalloc(seppart *ptr, sepsys *sys, int ntypes, const char
 		return seph_fail(SEP_GPU_EARG, "sys->npart (%ld) differs from the %ld atoms",
 				 sys->npart, c->n);
 	int rc;
-	if (!c->resident && ((rc = seph_put_x(c)) || (rc = seph_put_scalars(c))))
+	if (!c->resident && ((rc = seph_put(c, SEPDEV_X | SEPDEV_SCALARS))))
 		return rc;
 	sepdev_ljtab_args ta;
 	memset(&ta, 0, sizeof ta);
@@ -611,9 +613,7 @@ void sep_omp_make_neighb(seppart *ptr, double cf, sepsys *sys, const unsigned op
 	if (!rc && c->resident)
 		rc = seph_fail(SEP_GPU_ESTATE, "sep_omp_make_neighb on a resident system");
 	if (!rc)
-		rc = seph_put_x(c);
-	if (!rc)
-		rc = seph_put_scalars(c);
+		rc = seph_put(c, SEPDEV_X | SEPDEV_SCALARS);
 	if (!rc && needs_partners(opt))
 		rc = seph_put_partners(c);
 	if (!rc) {

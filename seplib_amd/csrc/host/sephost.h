@@ -50,8 +50,9 @@ typedef struct {
 	unsigned topo_nb, topo_na, topo_nd;
 	int partners_on_device;
 	int timing;
-	/* the single type label shared by all atoms (0 if mixed); trusted only
-	 * while resident, where types change only through sep_gpu_upload */
+	/* the single type label shared by all atoms (0 if mixed): of the types
+	 * a synchronised call uploads, or, while resident, of those at the
+	 * first call that asks (they change only through sep_gpu_upload) */
 	char uniform_type;
 	int uniform_type_valid;
 	/* grids whose list capacity was confirmed on the host (resident mode);
@@ -61,12 +62,7 @@ typedef struct {
 	int nchecked;
 	/* sep_gpu_list_limit: entries per atom a build may write (0: none) */
 	int list_limit;
-	/* host staging */
-	double *v3;
-	int *i3;
-	double *s1, *s2;
-	signed char *c1;
-	int *i1;
+	int *i3; /* host staging of the bonded partners */
 } seph_ctx;
 
 /* registry */
@@ -83,15 +79,12 @@ int seph_fail(int code, const char *fmt, ...);
 int seph_dev_fail(int rc); /* copies the device module's message */
 
 /* transfers between the AoS and the device (original order) */
-int seph_put_x(seph_ctx *c);
-int seph_put_v(seph_ctx *c);
-int seph_put_f(seph_ctx *c);
-int seph_put_xn_cross(seph_ctx *c);
-int seph_put_scalars(seph_ctx *c);
+/* the fields of a SEPDEV_X ... mask, in one pass over the atoms */
+int seph_put(seph_ctx *c, unsigned mask);
+int seph_get(seph_ctx *c, unsigned mask);
+int seph_run_jobs(int njobs, long atoms, int (*job)(void *arg, int k), void *arg);
 int seph_put_partners(seph_ctx *c);
 int seph_put_topology(seph_ctx *c, const sepsys *sys);
-int seph_get_f(seph_ctx *c);
-int seph_get_state(seph_ctx *c); /* x, v, a, cross counters */
 int seph_put_all(seph_ctx *c, const sepsys *sys);
 int seph_get_all(seph_ctx *c, sepsys *sys);
 /* The per-atom state only: device -> AoS (a resident system), and AoS ->

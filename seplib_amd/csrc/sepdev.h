@@ -78,20 +78,28 @@ const char *sepdev_error_message(void);
 int sepdev_last_code(void);
 void sepdev_clear_error(void);
 
-/* ---- host <-> device transfers (original order, AoS-interleaved 3-vectors
- * x0 y0 z0 x1 y1 z1 ...) */
+/* ---- host <-> device transfers: one packed record per atom, original order,
+ * holding the fields of a mask one after another: x, v, f, a, xn (3 doubles
+ * each), mass and charge (doubles), cross_neighb, crossings (3 ints each),
+ * molecule index and type (ints); mass, charge, molecule and type are
+ * SEPDEV_SCALARS (uploads only). */
 enum {
-	SEPDEV_X = 0, SEPDEV_V = 1, SEPDEV_F = 2, SEPDEV_A = 3, SEPDEV_XN = 4
+	SEPDEV_X = 1, SEPDEV_V = 2, SEPDEV_F = 4, SEPDEV_A = 8, SEPDEV_XN = 16,
+	SEPDEV_SCALARS = 32, SEPDEV_CROSS_NB = 64, SEPDEV_CROSS = 128
 };
-enum { SEPDEV_CROSS_NB = 0, SEPDEV_CROSS = 1 };
-int sepdev_put_vec(sepdev *d, int which, const double *src3n);
-int sepdev_get_vec(sepdev *d, int which, double *dst3n);
-int sepdev_put_ivec(sepdev *d, int which, const int *src3n);
-int sepdev_get_ivec(sepdev *d, int which, int *dst3n);
-int sepdev_put_scalars(sepdev *d, const double *mass, const double *charge,
-		       const signed char *type, const int *molindex);
-int sepdev_put_charges(sepdev *d, const double *charge);
-int sepdev_put_types(sepdev *d, const signed char *type);
+int sepdev_record_bytes(unsigned mask);
+/* Upload: open gives the pinned record buffer, which is free for packing,
+ * and close sends it. */
+int sepdev_put_open(sepdev *d, char **rec);
+int sepdev_put_close(sepdev *d, unsigned mask);
+/* Download: open starts it in *nchunk chunks; chunk k holds the records
+ * [*i0, *i1) and may be read once sepdev_get_chunk(k) has returned 0 (any
+ * thread may wait; another value goes to sepdev_get_failed on the caller's).
+ * settle: launches what the fields of the mask still owe, as open does. */
+int sepdev_get_settle(sepdev *d, unsigned mask);
+int sepdev_get_open(sepdev *d, unsigned mask, const char **rec, int *nchunk);
+int sepdev_get_chunk(sepdev *d, int k, long *i0, long *i1);
+int sepdev_get_failed(int code);
 /* bonded partners, 40 ints per atom (bond[10], angle[10], dihed[20]) */
 int sepdev_put_partners(sepdev *d, const int *partners40n);
 int sepdev_put_sys(sepdev *d, const sepdev_sys *s);
@@ -251,9 +259,19 @@ void sepdev_batch_destroy(sepdev_batch *b);
 int sepdev_batch_run(sepdev_batch *b, long nsteps, int mixed, int graph);
 int sepdev_batch_eval(sepdev_batch *b, int mixed);
 int sepdev_batch_synchronize(sepdev_batch *b);
-/* scal: alpha, max_dist2, tnow, nupdate, neighb_flag, max_full, error, sumv2 */
-int sepdev_batch_get(sepdev_batch *b, int s, double *x, double *v, double *f,
-		     double *a, int *cr, double *ret, double *scal);
+/* Results of a batch.  fetch waits for the queued steps; scalars gives a
+ * system's return slot and alpha, max_dist2, tnow, nupdate, neighb_flag, and
+ * returns its device error.  The atoms of systems 0 .. nsys-1 then come as
+ * records of SEPDEV_BATCH_WORDS ints in original order (x, v, f, a as doubles,
+ * the 3 crossings, padding), in chunks of whole systems: the records of
+ * systems [*s0, *s1) may be read once get_chunk has returned 0 (any thread
+ * may wait; another value goes to sepdev_get_failed). */
+#define SEPDEV_BATCH_WORDS 28
+int sepdev_batch_fetch(sepdev_batch *b);
+int sepdev_batch_scalars(sepdev_batch *b, int s, double *ret, double *scal);
+int sepdev_batch_get_open(sepdev_batch *b, int nsys, int *nchunk);
+int sepdev_batch_get_chunk(sepdev_batch *b, int k, int *s0, int *s1);
+const char *sepdev_batch_records(const sepdev_batch *b, int s);
 int sepdev_batch_set_shape(sepdev_batch *b, const int *sub, int grid);
 int sepdev_batch_get_shape(sepdev_batch *b, int *sub, int *grid);
 int sepdev_batch_time_eval(sepdev_batch *b, const int *mask, int mixed, int reps,

@@ -1,0 +1,78 @@
+"""The atoms' way to the device and back: every field survives bit for bit, in
+original order, at sizes on either side of a workgroup of a transfer, of a
+chunk of a download, of the host threads and of the most chunks there are, and
+again once the device has sorted the atoms.  The same for batches whose
+systems share chunks, fill one, or exceed one.
+"""
+import numpy as np
+import pytest
+
+from seplib_amd import batch as B
+from seplib_amd import sep as S
+from seplib_amd import workloads as W
+from seplib_amd.sim import SepSystem
+
+pytestmark = pytest.mark.gpu
+
+DOUBLES = ("x", "v", "f", "a", "xn")
+INTS = ("cross_neighb", "crossings")
+
+
+def _fill(view, seed):
+    n = len(view["x"])
+    for k, name in enumerate(DOUBLES[1:]):
+        view[name] = W.normal(seed + k, 3 * n).reshape(n, 3)
+    for k, name in enumerate(INTS):
+        view[name] = np.arange(3 * n).reshape(n, 3) * (k + 1) % 1013 - 500
+
+
+def _clear(view):
+    for name in DOUBLES + INTS:
+        view[name] = 0
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 16384, 16385, 32767, 32768, 32769, 262145])
+def test_fields_survive(product, n):
+    L = max(12.0, (n / 0.2) ** (1.0 / 3.0))
+    w = dict(x=W.uniform(n, 3 * n).reshape(n, 3) * L, v=np.zeros((n, 3)),
+             m=1.0 + W.uniform(n + 1, n), q=W.normal(n + 2, n), type=np.full(n, b"A"),
+             L=np.full(3, L), mol=np.full(n, -1))
+    s = SepSystem.from_workload(product, w, cf=2.5, dt=0.005, skin=0.3, nneighb=8)
+    try:
+        _fill(s.view, 7)
+        s.view["xn"] = w["x"]
+        want = {k: np.array(s.view[k]) for k in DOUBLES + INTS}
+        s.gpu_resident(True)
+        _clear(s.view)
+        s.gpu_sync()
+        for k in want:
+            assert np.array_equal(s.view[k], want[k]), (k, "as uploaded")
+        # a pair call sorts the atoms and replaces f alone
+        s.gpu_run([s.op_pairs("AA", 2.5, "sep_lj_shift")], 1)
+        _clear(s.view)
+        s.gpu_sync()
+        for k in want:
+            if k != "f":
+                assert np.array_equal(s.view[k], want[k]), (k, "sorted")
+    finally:
+        s.close()
+
+
+@pytest.mark.parametrize("sizes", [[33], [64, 65, 200], [300] * 70, [17000, 40, 20000, 900, 50]])
+def test_batch_survives(product, sizes):
+    reps = [dict(n=n, rho=0.3, T=1.0, w=W.random_packed(n, 0.1, 1.0, seed=5 + k))
+            for k, n in enumerate(sizes)]
+    systems = B.make_systems(product, reps)
+    b = B.Batch(product, systems, [1.0] * len(reps), precision=S.SEP_GPU_FP64)
+    try:
+        want = [(np.array(s.view["x"]), np.array(s.view["v"])) for s in systems]
+        b.eval(S.SEP_GPU_FP64)
+        for s in systems:
+            s.view["x"] = 0
+            s.view["v"] = 0
+        b.sync()
+        for k, s in enumerate(systems):
+            assert np.array_equal(s.view["x"], want[k][0]), (k, "x")
+            assert np.array_equal(s.view["v"], want[k][1]), (k, "v")
+    finally:
+        b.close()
