@@ -153,6 +153,7 @@ extern "C" sepdev *sepdev_create(long npart, int *err)
 	rc |= dalloc(&d->partials, d->partials_words);
 	rc |= dalloc(&d->fin_l2, (size_t)SEPK_MAXTASK * SEPK_MAXNV * SEPK_FIN_BLOCKS);
 	rc |= dalloc(&d->sys, 1);
+	rc |= dalloc(&d->half_cursor, 1);
 	d->ret_cap = 16;
 	rc |= dalloc(&d->ret, (size_t)d->ret_cap * SEPDEV_RET_WORDS);
 	d->ret_zero = (unsigned char *)calloc(d->ret_cap, 1);
@@ -202,7 +203,7 @@ extern "C" void sepdev_destroy(sepdev *d)
 	void *ptrs[] = {d->iperm, d->cell_count, d->cell_start,
 			d->cellid_old, d->order_tmp, d->cell_slot,
 			d->nbr, d->nbr_count, d->partials, d->fin_l2, d->ring, d->ring_n, d->ret,
-			d->scal, d->sys, d->blist, d->alist, d->dlist,
+			d->scal, d->sys, d->half_cursor, d->blist, d->alist, d->dlist,
 			d->bcontrib, d->acontrib, d->dcontrib, d->bcsr_off,
 			d->bcsr_idx, d->acsr_off, d->acsr_idx, d->dcsr_off,
 			d->dcsr_idx, d->blen, d->aval, d->dval};
@@ -211,6 +212,8 @@ extern "C" void sepdev_destroy(sepdev *d)
 			(void)hipFree(p);
 	if (d->hstage)
 		(void)hipHostFree(d->hstage);
+	if (d->half)
+		(void)hipHostFree(d->half);
 	for (hipEvent_t ev : d->chunk_ev)
 		if (ev)
 			(void)hipEventDestroy(ev);
@@ -394,7 +397,7 @@ static int fetch_words(sepdev *d, void *dst, const void *src, size_t bytes)
 	return 0;
 }
 
-static int store_words(sepdev *d, void *dst, const void *src, size_t bytes)
+int sepk_store_words(sepdev *d, void *dst, const void *src, size_t bytes)
 {
 	if (d->capturing)
 		return sepk_fail(SEP_GPU_ESTATE, "transfer during graph capture");
@@ -544,7 +547,7 @@ extern "C" int sepdev_put_sys(sepdev *d, const sepdev_sys *s)
 	// the host record replaces everything, including the cached sum m v^2
 	d->max_reset_pending = 0;
 	d->sumv2_valid = 0;
-	return store_words(d, d->sys, s, sizeof *s);
+	return sepk_store_words(d, d->sys, s, sizeof *s);
 }
 
 extern "C" int sepdev_get_sys(sepdev *d, sepdev_sys *s)
@@ -611,7 +614,7 @@ extern "C" int sepdev_ret_put(sepdev *d, int slot, const double *words)
 	if (slot < 0 || slot >= d->nret)
 		return sepk_fail(SEP_GPU_EARG, "ret slot %d", slot);
 	d->ret_zero[slot] = 0;
-	return store_words(d, d->ret + (size_t)slot * SEPDEV_RET_WORDS, words,
+	return sepk_store_words(d, d->ret + (size_t)slot * SEPDEV_RET_WORDS, words,
 			   SEPDEV_RET_WORDS * sizeof(double));
 }
 
@@ -643,7 +646,7 @@ extern "C" int sepdev_scalar_get(sepdev *d, int slot, double *v)
 
 extern "C" int sepdev_scalar_put(sepdev *d, int slot, double v)
 {
-	return store_words(d, d->scal + slot, &v, sizeof(double));
+	return sepk_store_words(d, d->scal + slot, &v, sizeof(double));
 }
 
 // ---- misc -----------------------------------------------------------------------

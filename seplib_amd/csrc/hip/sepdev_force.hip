@@ -1496,49 +1496,121 @@ extern "C" int sepdev_leapfrog(sepdev *d, double dt, double skin, const double *
 
 // ---- list extraction ------------------------------------------------------------
 
-__global__ void k_half_list(const int *orig, const int *nbr, const int *cnt, long n,
-			    long npad, int *counts, int *half, int stride)
+// Half list (entries j > o, original numbering) of every atom o, written
+// straight into pinned host memory as packed rows: a workgroup takes 64 atoms
+// in original order, a wave an atom; it counts the atoms' entries, takes room
+// for all of them at once and walks the lists again to write them.  Only
+// entries that exist cross the link, and nothing is allocated for the call.
+// Bound by the link and the host's copies out of it.  One thread per atom into
+// rows of the list's capacity, all of them copied to memory allocated for the
+// call, made a synchronised rebuild and its forces take 794 us at 8000 atoms
+// (300 us now) and 10.5 ms at 32000 (1.0 ms).
+// A workgroup that finds no room sets its offset to -1 and runs again in the
+// next pass.
+#define SEPK_HALF_ATOMS 64
+// entries an atom the pinned buffer holds on average (a full list of 128)
+#define SEPK_HALF_MEAN 64
+__global__ __launch_bounds__(SEPK_BLOCK) void
+k_half_list(const int *orig, const int *iperm, const int *nbr, const int *cnt, long n, long npad,
+	    int *counts, long *off, int *rows, unsigned long long room,
+	    unsigned long long *cursor, int again)
 {
-	const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-	if (t >= n)
+	const long o0 = (long)blockIdx.x * SEPK_HALF_ATOMS;
+	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+	__shared__ int len[SEPK_HALF_ATOMS];
+	__shared__ long first;
+	if (again && off[blockIdx.x] != -1)
 		return;
-	const int o = orig[t];
-	int c = 0;
-	for (int k = 0; k < cnt[t]; k++) {
-		const int oj = orig[nbr[sepk_entry(k, t, npad)]];
-		if (oj > o) {
-			if (c < stride)
-				half[(long)o * stride + c] = oj;
-			c++;
+	for (int a = wave; a < SEPK_HALF_ATOMS; a += SEPK_BLOCK / 64) {
+		int c = 0;
+		if (o0 + a < n) {
+			const int o = (int)(o0 + a), t = iperm[o], m = cnt[t];
+			for (int k = 0; k < m; k += 64) {
+				const int hit = k + lane < m &&
+						orig[nbr[sepk_entry(k + lane, t, npad)]] > o;
+				c += __popcll(__ballot(hit));
+			}
+		}
+		if (lane == 0) {
+			len[a] = c;
+			if (o0 + a < n)
+				counts[o0 + a] = c;
 		}
 	}
-	counts[o] = c;
+	__syncthreads();
+	if (wave == 0) {
+		const int own = len[lane];
+		int end = own;
+		for (int s = 1; s < 64; s <<= 1) {
+			const int up = __shfl_up(end, s);
+			end += lane >= s ? up : 0;
+		}
+		len[lane] = end - own;
+		if (lane == 63) {
+			const unsigned long long at =
+				atomicAdd(cursor, (unsigned long long)end);
+			first = at + end <= room ? (long)at : -1;
+			off[blockIdx.x] = first;
+		}
+	}
+	__syncthreads();
+	if (first < 0)
+		return;
+	for (int a = wave; a < SEPK_HALF_ATOMS && o0 + a < n; a += SEPK_BLOCK / 64) {
+		const int o = (int)(o0 + a), t = iperm[o], m = cnt[t];
+		int *row = rows + first + len[a];
+		for (int k = 0; k < m; k += 64) {
+			int oj = -1;
+			if (k + lane < m)
+				oj = orig[nbr[sepk_entry(k + lane, t, npad)]];
+			const unsigned long long hits = __ballot(oj > o);
+			if (oj > o)
+				row[__popcll(hits & ((1ull << lane) - 1))] = oj;
+			row += __popcll(hits);
+		}
+	}
 }
 
-extern "C" int sepdev_get_half_list(sepdev *d, int *counts, int *half, int stride,
-				    int *maxc)
+extern "C" int sepdev_half_pass(sepdev *d, int again, sepdev_half *h)
 {
 	if (!d->list_built)
 		return sepk_fail(SEP_GPU_ESTATE, "no neighbour list");
-	int rc0 = sepk_flush_tasks(d);
-	if (rc0)
-		return rc0;
-	int *dc = nullptr, *dh = nullptr;
-	SEPK_CHECK(hipMalloc(&dc, d->n * sizeof(int)));
-	SEPK_CHECK(hipMalloc(&dh, (size_t)d->n * stride * sizeof(int)));
-	k_half_list<<<sepk_blocks(d->n), SEPK_BLOCK, 0, d->st>>>(d->s[0].orig, d->nbr, d->nbr_count,
-								 d->n, d->npad, dc, dh, stride);
+	if (d->capturing)
+		return sepk_fail(SEP_GPU_ESTATE, "transfer during graph capture");
+	int rc = sepk_flush_tasks(d);
+	if (rc)
+		return rc;
+	const long nblk = (d->n + SEPK_HALF_ATOMS - 1) / SEPK_HALF_ATOMS;
+	// any one workgroup's rows fit
+	size_t room = (size_t)d->npad * SEPK_HALF_MEAN;
+	if (room < (size_t)SEPK_HALF_ATOMS * d->cap)
+		room = (size_t)SEPK_HALF_ATOMS * d->cap;
+	if (room > d->half_room) {
+		if (d->half)
+			(void)hipHostFree(d->half);
+		d->half = nullptr;
+		d->half_room = 0;
+		SEPK_CHECK(hipHostMalloc((void **)&d->half,
+					 nblk * sizeof(long) + (d->npad + room) * sizeof(int),
+					 hipHostMallocDefault));
+		d->half_room = room;
+	}
+	long *off = (long *)d->half;
+	int *counts = (int *)(off + nblk);
+	int *rows = counts + d->npad;
+	const unsigned long long zero = 0;
+	if ((rc = sepk_store_words(d, d->half_cursor, &zero, sizeof zero)))
+		return rc;
+	k_half_list<<<(unsigned)nblk, SEPK_BLOCK, 0, d->st>>>(
+		d->s[0].orig, d->iperm, d->nbr, d->nbr_count, d->n, d->npad, counts, off, rows,
+		d->half_room, d->half_cursor, again);
 	SEPK_LAUNCH_CHECK();
-	SEPK_CHECK(hipMemcpyAsync(counts, dc, d->n * sizeof(int), hipMemcpyDeviceToHost, d->st));
-	SEPK_CHECK(hipMemcpyAsync(half, dh, (size_t)d->n * stride * sizeof(int), hipMemcpyDeviceToHost, d->st));
 	SEPK_CHECK(hipStreamSynchronize(d->st));
-	(void)hipFree(dc);
-	(void)hipFree(dh);
-	int mc = 0;
-	for (long o = 0; o < d->n; o++)
-		if (counts[o] > mc)
-			mc = counts[o];
-	*maxc = mc;
+	h->nblk = nblk;
+	h->atoms = SEPK_HALF_ATOMS;
+	h->off = off;
+	h->counts = counts;
+	h->rows = rows;
 	return 0;
 }
 

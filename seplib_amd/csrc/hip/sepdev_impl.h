@@ -184,6 +184,10 @@ struct sepdev {
 	char *hrec;    // pinned atom records (SEPK_REC_WORDS words an atom at most)
 	long chunk;    // atoms per chunk of the download under way
 	hipEvent_t chunk_ev[SEPK_CHUNKS]; // a chunk's records are complete
+	// pinned half list (sepdev_half): room entries, made at the first call
+	void *half;
+	size_t half_room;
+	unsigned long long *half_cursor;
 
 	// Deferred work, decided on the host so that a captured step replays
 	// the same kernels every time:
@@ -613,6 +617,7 @@ int sepk_fresh_qpos(sepdev *d, const double *L);
 // launches a pair call recorded for a fused step, if any (sepdev_force.hip)
 int sepk_flush_pair(sepdev *d);
 int sepk_flush_nh(sepdev *d);
+int sepk_store_words(sepdev *d, void *dst, const void *src, size_t bytes);
 int sepk_put_vec_to(sepdev *d, double *dst, const double *src3n);
 int sepk_get_vec_from(sepdev *d, double *dst3n, const double *src);
 void sepk_task_ret(sepdev *d, sepk_task &t, int slot);

@@ -657,29 +657,77 @@ void seph_grid_own(const sepsys *sys, double rlist, unsigned opt, int bonded_rul
 
 /* ---- list build ------------------------------------------------------- */
 
+typedef struct {
+	sepdev_half h;
+	long n;
+	void (*row)(void *arg, long i, const int *entries, int count);
+	void *arg;
+	int missing;
+} half_walk;
+
+#define HALF_JOB 32 /* blocks a job */
+
+static int half_job(void *arg, int k)
+{
+	half_walk *w = arg;
+	for (long b = (long)k * HALF_JOB; b < (k + 1L) * HALF_JOB && b < w->h.nblk; b++) {
+		if (w->h.off[b] < 0) {
+			if (w->h.off[b] == -1)
+				__atomic_store_n(&w->missing, 1, __ATOMIC_RELAXED);
+			continue;
+		}
+		const int *e = w->h.rows + w->h.off[b];
+		for (long i = b * w->h.atoms; i < (b + 1) * w->h.atoms && i < w->n; i++) {
+			w->row(w->arg, i, e, w->h.counts[i]);
+			e += w->h.counts[i];
+		}
+		w->h.off[b] = -2; /* done: another pass leaves it alone */
+	}
+	return 0;
+}
+
+int seph_half_lists(seph_ctx *c, int (*begin)(void *arg, const int *counts),
+		    void (*row)(void *arg, long i, const int *entries, int count), void *arg)
+{
+	half_walk w = {.n = c->n, .row = row, .arg = arg};
+	int rc = seph_dev_fail(sepdev_half_pass(c->dev, 0, &w.h));
+	if (rc || (rc = begin(arg, w.h.counts)))
+		return rc;
+	for (;;) {
+		w.missing = 0;
+		/* an entry weighs less than an atom's record, a row more */
+		seph_run_jobs((int)((w.h.nblk + HALF_JOB - 1) / HALF_JOB), 4 * c->n, half_job, &w);
+		if (!w.missing)
+			return 0;
+		if ((rc = seph_dev_fail(sepdev_half_pass(c->dev, 1, &w.h))))
+			return rc;
+	}
+}
+
+static int rows_fit(void *arg, const int *counts)
+{
+	const seph_ctx *c = arg;
+	int maxc = 0;
+	for (long i = 0; i < c->n; i++)
+		if (counts[i] > maxc)
+			maxc = counts[i];
+	return maxc < c->nneighb ? 0 : seph_fail(SEP_GPU_ENEIGHB,
+						 "Too many neighbours (%d >= capacity %d)", maxc,
+						 c->nneighb);
+}
+
+static void write_row(void *arg, long i, const int *entries, int count)
+{
+	int *row = ((seph_ctx *)arg)->atoms[i].neighb;
+	memcpy(row, entries, sizeof(int) * (size_t)count);
+	row[count] = -1;
+}
+
 /* Writes the device list into atoms[i].neighb as a -1 terminated half list
  * (entries j > i, original numbering). */
 static int write_half_lists(seph_ctx *c)
 {
-	if (c->nneighb <= 0)
-		return 0;
-	const int stride = sepdev_list_capacity(c->dev);
-	int *counts = malloc(sizeof(int) * (size_t)c->n);
-	int *half = malloc(sizeof(int) * (size_t)c->n * (size_t)stride);
-	int maxc = 0;
-	int rc = seph_dev_fail(sepdev_get_half_list(c->dev, counts, half, stride, &maxc));
-	if (rc == 0 && maxc >= c->nneighb)
-		rc = seph_fail(SEP_GPU_ENEIGHB, "Too many neighbours (%d >= capacity %d)", maxc,
-			       c->nneighb);
-	if (rc == 0)
-		for (long i = 0; i < c->n; i++) {
-			memcpy(c->atoms[i].neighb, half + (size_t)i * stride,
-			       sizeof(int) * (size_t)counts[i]);
-			c->atoms[i].neighb[counts[i]] = -1;
-		}
-	free(counts);
-	free(half);
-	return rc;
+	return c->nneighb <= 0 ? 0 : seph_half_lists(c, rows_fit, write_row, c);
 }
 
 /* After a build that overflowed the list (SEP_GPU_ENEIGHB, longest list

@@ -381,36 +381,49 @@ int sep_gpu_restore(seppart *atoms, sepsys *sys, sepret *ret, double *alpha, con
 
 /* ---- diagnostics ------------------------------------------------------ */
 
+typedef struct {
+	long n, cap, *npairs;
+	int *pairs;  /* null, or 2 * cap ints */
+	long *first; /* first pair of each atom */
+} pair_out;
+
+static int count_pairs(void *arg, const int *counts)
+{
+	pair_out *o = arg;
+	long tot = 0;
+	for (long i = 0; i < o->n; i++) {
+		o->first[i] = tot;
+		tot += counts[i];
+	}
+	*o->npairs = tot;
+	if (tot > o->cap)
+		o->pairs = NULL;
+	return 0;
+}
+
+static void write_pairs(void *arg, long i, const int *entries, int count)
+{
+	const pair_out *o = arg;
+	if (o->pairs)
+		for (int e = 0; e < count; e++) {
+			o->pairs[2 * (o->first[i] + e)] = (int)i;
+			o->pairs[2 * (o->first[i] + e) + 1] = entries[e];
+		}
+}
+
 int sep_gpu_neighbour_pairs(seppart *atoms, sepsys *sys, int *pairs, long cap,
 			    long *npairs)
 {
 	seph_ctx *c = seph_ctx_for(atoms, sys);
 	if (!c)
 		return sep_gpu_last_error();
-	const int stride = sepdev_list_capacity(c->dev);
-	if (stride <= 0)
+	if (sepdev_list_capacity(c->dev) <= 0)
 		return seph_fail(SEP_GPU_ESTATE, "no neighbour list on the device");
-	int *counts = malloc(sizeof(int) * (size_t)c->n);
-	int *half = malloc(sizeof(int) * (size_t)c->n * (size_t)stride);
-	int maxc = 0;
-	int rc = seph_dev_fail(sepdev_get_half_list(c->dev, counts, half, stride, &maxc));
-	if (rc == 0) {
-		long tot = 0;
-		for (long i = 0; i < c->n; i++)
-			tot += counts[i];
-		*npairs = tot;
-		if (pairs && tot <= cap) {
-			long w = 0;
-			for (long i = 0; i < c->n; i++)
-				for (int e = 0; e < counts[i]; e++) {
-					pairs[2 * w] = (int)i;
-					pairs[2 * w + 1] = half[(size_t)i * stride + e];
-					w++;
-				}
-		}
-	}
-	free(counts);
-	free(half);
+	pair_out o = {c->n, cap, npairs, pairs, malloc(sizeof(long) * (size_t)c->n)};
+	if (!o.first)
+		return seph_fail(SEP_GPU_EHOST, "sep_gpu_neighbour_pairs: out of host memory");
+	const int rc = seph_half_lists(c, count_pairs, write_pairs, &o);
+	free(o.first);
 	return rc;
 }
 

@@ -82,6 +82,11 @@ int seph_dev_fail(int rc); /* copies the device module's message */
 /* the fields of a SEPDEV_X ... mask, in one pass over the atoms */
 int seph_put(seph_ctx *c, unsigned mask);
 int seph_get(seph_ctx *c, unsigned mask);
+/* Every atom's half list: begin sees all counts first (nonzero ends the call),
+ * then row is called once per atom, in any order and from several threads. */
+int seph_half_lists(seph_ctx *c, int (*begin)(void *arg, const int *counts),
+		    void (*row)(void *arg, long i, const int *entries, int count), void *arg);
+/* jobs 0 .. njobs-1, on several threads when they handle many atoms */
 int seph_run_jobs(int njobs, long atoms, int (*job)(void *arg, int k), void *arg);
 int seph_put_partners(seph_ctx *c);
 int seph_put_topology(seph_ctx *c, const sepsys *sys);

@@ -137,10 +137,19 @@ int sepdev_list_limit(sepdev *d, int cap, int *applied);
 int sepdev_list_capacity(sepdev *d);
 /* sys->max_dist2 = 0 on the device (resident sep_reset_force) */
 int sepdev_reset_max_dist(sepdev *d);
-/* half list in original numbering: counts[o] entries j > o for atom o,
- * written to half[o*stride + e]; returns the largest count in *maxc */
-int sepdev_get_half_list(sepdev *d, int *counts, int *half, int stride,
-			 int *maxc);
+/* Half list in original numbering: atom o has counts[o] entries j > o.  The
+ * rows of atoms [k * atoms, (k + 1) * atoms) follow each other from rows +
+ * off[k] on, for every k with off[k] >= 0.  Where some off[k] is -1 the rows did
+ * not all fit: another pass (again = 1) replaces the rows by those of the
+ * missing k, whose off it sets; the caller marks the others (any value but -1)
+ * if it has to tell them apart.  Valid until the next call on d. */
+typedef struct {
+	long nblk;
+	int atoms;
+	long *off;
+	const int *counts, *rows;
+} sepdev_half;
+int sepdev_half_pass(sepdev *d, int again, sepdev_half *h);
 int sepdev_list_stats(sepdev *d, double *mean_full, int *max_full);
 
 /* ---- forces */

@@ -76,3 +76,31 @@ def test_batch_survives(product, sizes):
             assert np.array_equal(s.view["v"], want[k][1]), (k, "v")
     finally:
         b.close()
+
+
+@pytest.mark.parametrize("n,clump", [(2, 0), (64, 64), (65, 65), (500, 400), (3000, 700)])
+def test_half_rows(product, oracle, n, clump):
+    """The rows written to neighb, in atom order and within their own arrays,
+    from few atoms up to clumps whose rows take more room than the buffer has
+    (several passes)."""
+    L = 14.0
+    x = W.uniform(n, 3 * n).reshape(n, 3) * L
+    x[:clump] = 4.0 + W.uniform(n + 1, 3 * clump).reshape(clump, 3) * 1.5
+    w = dict(x=x, v=np.zeros((n, 3)), m=np.ones(n), q=np.zeros(n), type=np.full(n, b"A"),
+             L=np.full(3, L), mol=np.full(n, -1))
+
+    pairs = []
+    for api in (product, oracle):
+        s = SepSystem.from_workload(api, w, cf=2.5, dt=0.005, skin=0.3, nneighb=n + 2,
+                                    nsubbox=(5, 5, 5))
+        try:
+            s.reset_retval()
+            s.reset_force()
+            s.force_pairs("AA", 2.5, "sep_lj_shift")
+            pairs.append(s.half_pairs())
+            if api is product:
+                pairs.append(s.gpu_pairs())
+        finally:
+            s.close()
+    assert np.array_equal(pairs[0], pairs[2])
+    assert np.array_equal(pairs[1], pairs[2])
