@@ -146,6 +146,10 @@ extern "C" sepdev *sepdev_create(long npart, int *err)
 		const long brows = d->npad * 20 / SEPK_BLOCK + 8;
 		if (brows > rows)
 			rows = brows;
+		// a wide walk's row per 16 atoms
+		const long wrows = d->npad / 16 + 8 * SEPK_NXCD;
+		if (d->npad <= SEPK_WIDE_ATOMS + 64 && wrows > rows)
+			rows = wrows;
 		d->region_rows = rows;
 		d->region_words = rows * SEPK_MAXNV;
 		d->partials_words = d->region_words * SEPK_NREGION;

@@ -106,19 +106,10 @@ __device__ __forceinline__ void sepk_pair_epilogue(
 template <bool FAST>
 __device__ __forceinline__ double sepk_image(double d, double L, double iL, double &k)
 {
-	if (FAST) {
-		k = rint(d * iL);
-		return fma(-L, k, d);
-	}
-	k = 0.0;
-	if (d > 0.5 * L) {
-		k = 1.0;
-		d -= L;
-	} else if (d < -0.5 * L) {
-		k = -1.0;
-		d += L;
-	}
-	return d;
+	// selected, not branched to: the pairs of a batch are evaluated side by
+	// side (d - L and d + L are the fma's results for k = 1 and -1)
+	k = FAST ? rint(d * iL) : d > 0.5 * L ? 1.0 : d < -0.5 * L ? -1.0 : 0.0;
+	return fma(-L, k, d);
 }
 
 // Adds one pair's force ft r to the atom and its energy; the stress gets
@@ -627,6 +618,35 @@ struct sepk_coul {
 	float cff, icff, icf2f;
 };
 
+// Force factor and energy of a pair of charge product qq at squared distance r2
+// (source/sepcoulomb.c:130-140): qq (1/r2 - 1/rc^2) / r and
+// qq (1/r + (r - rc)/rc^2 - 1/rc).  r, 1/r, 1/r2 and the last division come
+// from one hardware reciprocal square root (2^-24), a coupled Newton step and a
+// residual correction each, which leaves every one of them at the rounding of
+// the operation it stands for; a square root and three divisions took three
+// times the instructions, most of the FP64 walk's (a step of 96000 atoms of water:
+// 251 -> 211 us).
+__device__ __forceinline__ void sepk_coul_pair(const sepk_coul &c, double qq, double r2, double &ft,
+					       double &e)
+{
+	const double y = __builtin_amdgcn_rsq(r2);
+	double h = 0.5 * y, r = r2 * y;
+	const double d = fma(-r, h, 0.5);
+	r = fma(r, d, r);
+	h = fma(h, d, h);
+	r = fma(fma(-r, r, r2), h, r);
+	double ri = 2.0 * h;
+	ri = fma(ri, fma(-r, ri, 1.0), ri);
+	double ri2 = ri * ri;
+	ri2 = fma(ri2, fma(-r2, ri2, 1.0), ri2);
+	const double a = qq * (ri2 - c.icf2);
+	ft = a * ri;
+	ft = fma(fma(-r, ft, a), ri, ft);
+	// charges in one place: the energy stays infinite
+	const bool zero = r2 == 0.0;
+	e = qq * ((zero ? __builtin_inf() : ri) + ((zero ? 0.0 : r) - c.cf) * c.icf2 - c.icf);
+}
+
 // The mixed form of the pair loop below: positions and charges from the
 // 16-byte quantized records (integer minimum image, charge as FP32 in w),
 // r^2 and the cutoff test in FP64 from the exact integer differences, the
@@ -748,10 +768,8 @@ __global__ __launch_bounds__(SEPK_BLOCK) void k_coulomb(
 				const double r2 = dx * dx + dy * dy + dz * dz;
 				if (!(r2 < c.cf2))
 					continue;
-				const double qq = pj[u].q * pi.q;
-				const double r = sqrt(r2);
-				const double ft = qq * (1.0 / r2 - c.icf2) / r;
-				const double e = qq * (1.0 / r + (r - c.cf) * c.icf2 - c.icf);
+				double ft, e;
+				sepk_coul_pair(c, pj[u].q * pi.q, r2, ft, e);
 				sepk_pair_accumulate(ft, e, dx, dy, dz, kx, ky, kz, c.L0, c.L1, c.L2,
 						     fx, fy, fz, acc);
 			}
@@ -759,6 +777,441 @@ __global__ __launch_bounds__(SEPK_BLOCK) void k_coulomb(
 	}
 	sepk_pair_epilogue<OVERWRITE>(t, sub, n, npad, act, fx, fy, fz, pi.x, pi.y, pi.z, acc,
 				      s.f, partial, lb, rows, frozen);
+}
+
+// ---- wide walks ------------------------------------------------------------------
+//
+// Four lanes an atom leave a small system waiting: each lane goes through its
+// quarter of the list batch by batch, a gather's latency and a batch's
+// arithmetic after the other, on a chip that is mostly empty.  A wide walk gives
+// an atom 16 lanes, four for each of its four lanes: lane (g, sub) evaluates the
+// batches g, g + 4, ... of lane sub, four of them at a time, with the gathers of
+// the next four in flight.  The sums stay those of the walk by four lanes, bit
+// for bit: a lane leaves its pairs' force factors, energies and separations in
+// LDS, and the four lanes of one sub then each go through all four batches' pairs
+// in list order for their own column -- the three force components and the
+// energy, and two of the crossing stress each for three of them.  A pair left
+// out stands there with factor, energy and separation zero, which add nothing.
+// A wave holds 4 atoms and exchanges within itself; a workgroup, 16 atoms: its
+// first wave takes their sums over as one wave of the kernel by four lanes does,
+// and its row is that wave's (sepk_task::wide).
+//
+// An array is 32 bytes longer than its values, so that what the lanes of different
+// g read from different arrays lies in different banks.
+#define SEPK_WIDE_LEN (SEPK_BATCH * 64 + 4)
+template <int NT>
+struct sepk_wide_wave {
+	double fe[NT][2][SEPK_WIDE_LEN]; // force factor, energy
+	double d[3][SEPK_WIDE_LEN];
+	unsigned cross[64]; // image count, two's complement in two bits an axis, a byte an entry
+};
+
+// per term: fx, fy, fz, e and the six crossing columns, by lane of the kernel by
+// four lanes; then what else its lanes carry
+template <int NT>
+union sepk_wide_lds {
+	sepk_wide_wave<NT> w[SEPK_BLOCK / 64];
+	struct {
+		double col[NT][10][64];
+		int band[64];
+	} r;
+};
+
+// one lane's evaluated batch
+template <int NT>
+struct sepk_wide_batch {
+	double ft[NT][SEPK_BATCH], e[NT][SEPK_BATCH], d[3][SEPK_BATCH];
+	unsigned cross;
+};
+
+// a lane's columns: its force component (or the energy) and crossing columns
+template <int NT>
+struct sepk_wide_acc {
+	double m[NT], x0[NT], x1[NT];
+};
+
+__device__ __forceinline__ unsigned sepk_cross_code(double kx, double ky, double kz)
+{
+	return ((int)kx & 3) | ((int)ky & 3) << 2 | ((int)kz & 3) << 4;
+}
+
+__device__ __forceinline__ void sepk_wave_lds_fence()
+{
+	__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+	__builtin_amdgcn_wave_barrier();
+}
+
+// The four batches' pairs of an atom's sub, in list order, into a lane's columns;
+// CROSS: some pair of the wave crosses the box.  Lanes g = 0, 1, 2 take the
+// crossing columns xx, xy | xz, yy | yz, zz: separation along axes sa, g, image
+// along ia, ib; a pair that does not cross has image 0 and adds nothing.
+template <bool CROSS, int NT>
+__device__ __forceinline__ void sepk_wide_columns(const sepk_wide_wave<NT> &w, double L0, double L1,
+						  double L2, sepk_wide_acc<NT> &acc)
+{
+	const int ln = threadIdx.x & 63, g = (ln >> 2) & 3;
+	const int first = ln & ~12; // lane (0, sub) of the atom
+	const bool comp = g < 3;
+	const double *pd = w.d[comp ? g : 0] + first;
+	const double *ps = w.d[g == 2 ? 1 : 0] + first;
+	const int ia = g == 0 ? 0 : 4, ib = g < 2 ? 2 : 4; // bits of the image axes
+	const double La = g == 0 ? L0 : L2, Lb = g < 2 ? L1 : L2;
+	const double *pa[NT];
+#pragma unroll
+	for (int k = 0; k < NT; k++)
+		pa[k] = w.fe[k][comp ? 0 : 1] + first;
+#pragma unroll
+	for (int q = 0; q < 4; q++) {
+		const unsigned code = CROSS ? w.cross[first + 4 * q] : 0u;
+#pragma unroll
+		for (int u = 0; u < SEPK_BATCH; u++) {
+			const int i = u * 64 + 4 * q;
+			const double d = comp ? pd[i] : 1.0;
+			double a[NT];
+#pragma unroll
+			for (int k = 0; k < NT; k++) {
+				a[k] = pa[k][i];
+				acc.m[k] = fma(a[k], d, acc.m[k]);
+			}
+			if (CROSS) {
+				const double ka = La * (double)((int)(code << (30 - 8 * u - ia)) >> 30);
+				const double kb = Lb * (double)((int)(code << (30 - 8 * u - ib)) >> 30);
+				const double da = ps[i];
+#pragma unroll
+				for (int k = 0; k < NT; k++) {
+					acc.x0[k] = fma(-a[k] * da, ka, acc.x0[k]);
+					acc.x1[k] = fma(-a[k] * d, kb, acc.x1[k]);
+				}
+			}
+		}
+	}
+}
+
+// Adds the wave's evaluated batches to the lanes' columns.
+template <int NT>
+__device__ __forceinline__ void sepk_wide_add(sepk_wide_wave<NT> &w, const sepk_wide_batch<NT> &b,
+					      double L0, double L1, double L2,
+					      sepk_wide_acc<NT> &acc)
+{
+	const int ln = threadIdx.x & 63;
+#pragma unroll
+	for (int u = 0; u < SEPK_BATCH; u++) {
+#pragma unroll
+		for (int k = 0; k < NT; k++) {
+			w.fe[k][0][u * 64 + ln] = b.ft[k][u];
+			w.fe[k][1][u * 64 + ln] = b.e[k][u];
+		}
+#pragma unroll
+		for (int k = 0; k < 3; k++)
+			w.d[k][u * 64 + ln] = b.d[k][u];
+	}
+	w.cross[ln] = b.cross;
+	sepk_wave_lds_fence();
+	if (__ballot(b.cross != 0))
+		sepk_wide_columns<true>(w, L0, L1, L2, acc);
+	else
+		sepk_wide_columns<false>(w, L0, L1, L2, acc);
+	sepk_wave_lds_fence(); // read before the next batches replace it
+}
+
+// Hands the block's columns to its first wave, lane (16 atoms) x 4 as in the
+// kernel by four lanes: f and acc (energy, crossing stress) of each term, and
+// band.  The other waves return false; they are done.
+template <int NT>
+__device__ __forceinline__ bool sepk_wide_hand_over(sepk_wide_lds<NT> &lds,
+						    const sepk_wide_acc<NT> &w, bool &band,
+						    double (&f)[NT][3], double (&acc)[NT][7])
+{
+	const int g = (threadIdx.x >> 2) & 3;
+	const int at = (threadIdx.x >> 4) * 4 + (threadIdx.x & 3);
+	__syncthreads(); // the walks are over
+	if (threadIdx.x < 64)
+		lds.r.band[threadIdx.x] = 0;
+#pragma unroll
+	for (int k = 0; k < NT; k++) {
+		lds.r.col[k][g][at] = w.m[k];
+		if (g < 3) {
+			lds.r.col[k][4 + 2 * g][at] = w.x0[k];
+			lds.r.col[k][5 + 2 * g][at] = w.x1[k];
+		}
+	}
+	__syncthreads();
+	if (band)
+		lds.r.band[at] = 1; // any of the four lanes: the same value
+	__syncthreads();
+	if (threadIdx.x >= 64)
+		return false;
+	band = lds.r.band[threadIdx.x] != 0;
+#pragma unroll
+	for (int k = 0; k < NT; k++) {
+#pragma unroll
+		for (int i = 0; i < 3; i++)
+			f[k][i] = lds.r.col[k][i][threadIdx.x];
+#pragma unroll
+		for (int i = 0; i < 7; i++)
+			acc[k][i] = lds.r.col[k][3 + i][threadIdx.x];
+	}
+	return true;
+}
+
+// The batches of atom t's lane (g, sub): fetch(j, rec) gathers a batch's records,
+// eval(rec, batch) evaluates it.  The records of the next batch and the indices
+// of the one after it are under way while one is evaluated.
+template <int NT, class REC, class FETCH, class EVAL>
+__device__ __forceinline__ void sepk_wide_walk(sepk_wide_wave<NT> &w, const int *__restrict__ nbr,
+					       const int *__restrict__ cnt, long npad, int maxbat,
+					       long t, bool act, double L0, double L1, double L2,
+					       FETCH fetch, EVAL eval, sepk_wide_acc<NT> &acc)
+{
+	const int g = (threadIdx.x >> 2) & 3, sub = threadIdx.x & 3;
+	const size_t stride = (size_t)npad * SEPK_SUB;
+	const int4 *lp = sepk_lane_list(nbr, act ? t : 0, sub);
+	// the first indices go out with the count: the allocation holds them,
+	// whatever the list's length
+	int4 j0 = make_int4(0, 0, 0, 0), j1 = j0;
+	if (act && g < maxbat)
+		j0 = lp[g * stride];
+	if (act && g + 4 < maxbat)
+		j1 = lp[(g + 4) * stride];
+	const int nbat = act ? (cnt[t] + SEPK_PAD - 1) / SEPK_PAD : 0;
+	REC now[SEPK_BATCH], next[SEPK_BATCH];
+	if (g < nbat)
+		fetch(j0, now);
+	for (int b = g; __ballot(b - g < nbat); b += 4) {
+		if (b + 4 < nbat)
+			fetch(j1, next);
+		if (b + 8 < nbat)
+			j1 = lp[(b + 8) * stride];
+		sepk_wide_batch<NT> v;
+		v.cross = 0;
+#pragma unroll
+		for (int u = 0; u < SEPK_BATCH; u++) {
+#pragma unroll
+			for (int k = 0; k < NT; k++)
+				v.ft[k][u] = v.e[k][u] = 0.0;
+#pragma unroll
+			for (int k = 0; k < 3; k++)
+				v.d[k][u] = 0.0;
+		}
+		if (b < nbat)
+			eval(now, v);
+		sepk_wide_add(w, v, L0, L1, L2, acc);
+#pragma unroll
+		for (int u = 0; u < SEPK_BATCH; u++)
+			now[u] = next[u];
+	}
+}
+
+template <int NT>
+__device__ __forceinline__ sepk_wide_acc<NT> sepk_wide_zero()
+{
+	sepk_wide_acc<NT> a;
+#pragma unroll
+	for (int k = 0; k < NT; k++)
+		a.m[k] = a.x0[k] = a.x1[k] = 0.0;
+	return a;
+}
+
+// The walk of k_lj_coul by wide walk: true in the block's first wave, whose lane
+// then holds what the lane of k_lj_coul holds for atom 16 lb + lane / 4, lane
+// sub = lane % 4.
+template <bool TYPED, bool MIXED, bool FAST>
+__device__ __forceinline__ bool sepk_lj_coul_pairs_wide(
+	sepk_wide_lds<2> &lds, const sepk_state &s, const int *__restrict__ nbr,
+	const int *__restrict__ cnt, long n, long npad, int maxbat, const sepk_lj &c,
+	const sepk_coul &cc, long lb, double (&f)[2][3], double (&acc)[2][7], bool &band)
+{
+	const long t = lb * (SEPK_BLOCK / 16) + threadIdx.x / 16;
+	const bool act = t < n;
+	sepk_wide_wave<2> &w = lds.w[threadIdx.x >> 6];
+	sepk_wide_acc<2> wa = sepk_wide_zero<2>();
+	band = false;
+	const signed char ti = TYPED && act ? s.type[t] : 0;
+	const bool act_l = act && (!TYPED || ti == c.t0 || ti == c.t1);
+	const sepk_pos pi = act ? s.pos[t] : sepk_pos{0.0, 0.0, 0.0, 0.0};
+	const bool act_c = act && !(fabs(pi.q) < DBL_EPSILON);
+	const bool walks = act_l || act_c;
+	const auto typed = [&](signed char tj) {
+		return !TYPED || (ti == c.t0 && tj == c.t1) || (ti == c.t1 && tj == c.t0);
+	};
+	if (MIXED) {
+		struct rec {
+			int4 q;
+			signed char t;
+		};
+		const int4 qi = walks ? s.qpos[t] : make_int4(0, 0, 0, SEPK_QPHANTOM);
+		const float qif = __int_as_float(qi.w);
+		const float epsf = (float)DBL_EPSILON;
+		sepk_wide_walk<2, rec>(
+			w, nbr, cnt, npad, maxbat, t, walks, c.L0, c.L1, c.L2,
+			[&](const int4 &jb, rec (&r)[SEPK_BATCH]) {
+				const int j[SEPK_BATCH] = {jb.x, jb.y, jb.z, jb.w};
+#pragma unroll
+				for (int u = 0; u < SEPK_BATCH; u++) {
+					r[u].q = sepk_at(s.qpos, (unsigned)j[u]);
+					r[u].t = TYPED ? s.type[(unsigned)j[u]] : 0;
+				}
+			},
+			[&](const rec (&r)[SEPK_BATCH], sepk_wide_batch<2> &v) {
+#pragma unroll
+				for (int u = 0; u < SEPK_BATCH; u++) {
+					const unsigned ux = (unsigned)qi.x, vx = (unsigned)r[u].q.x;
+					const unsigned uy = (unsigned)qi.y, vy = (unsigned)r[u].q.y;
+					const unsigned uz = (unsigned)qi.z, vz = (unsigned)r[u].q.z;
+					const int ix = (int)(ux - vx), iy = (int)(uy - vy),
+						  iz = (int)(uz - vz);
+					const double dx = (double)ix * c.qd0;
+					const double dy = (double)iy * c.qd1;
+					const double dz = (double)iz * c.qd2;
+					const double r2 = dx * dx + dy * dy + dz * dz;
+					const bool lj = act_l && typed(r[u].t) && r[u].q.w != SEPK_QPHANTOM;
+					if (lj && !(r2 < c.cf2lo))
+						band |= r2 < c.cf2hi;
+					const bool in_l = lj && r2 < c.cf2lo;
+					if (in_l) {
+						const float q = c.sig2f * __builtin_amdgcn_rcpf((float)r2);
+						const float q3 = q * q * q;
+						v.ft[0][u] = (double)(fmaf(c.Af, q3, c.nBf) * q3 * q);
+						v.e[0][u] = (double)fmaf(fmaf(c.Cf, q3, c.nDf), q3, c.ushiftf);
+					}
+					const float qjf = __int_as_float(r[u].q.w);
+					const bool in_c = act_c && fabsf(qjf) >= epsf && r2 < cc.cf2;
+					// most listed pairs are inside: evaluated without a
+					// branch, the four entries' chains overlap
+					const float r2f = (float)r2;
+					const float ri = __builtin_amdgcn_rsqf(r2f);
+					const float rf = r2f * ri;
+					const float qq = qjf * qif;
+					const float dc = cc.cff - rf;
+					const float qs = qq * cc.icf2f * ri;
+					v.ft[1][u] = in_c ? (double)(qs * (dc * (cc.cff + rf)) * (ri * ri)) : 0.0;
+					v.e[1][u] = in_c ? (double)(qs * (dc * dc)) : 0.0;
+					v.d[0][u] = dx;
+					v.d[1][u] = dy;
+					v.d[2][u] = dz;
+					if (in_l || in_c) {
+						const bool bx = (ux < vx) != (ix < 0), by = (uy < vy) != (iy < 0),
+							   bz = (uz < vz) != (iz < 0);
+						v.cross |= ((bx ? (ix < 0 ? 1u : 3u) : 0u) |
+							    (by ? (iy < 0 ? 4u : 12u) : 0u) |
+							    (bz ? (iz < 0 ? 16u : 48u) : 0u))
+							   << (8 * u);
+					}
+				}
+			},
+			wa);
+	} else {
+		struct rec {
+			sepk_pos p;
+			signed char t;
+		};
+		const char *pb = (const char *)s.pos;
+		sepk_wide_walk<2, rec>(
+			w, nbr, cnt, npad, maxbat, t, walks, c.L0, c.L1, c.L2,
+			[&](const int4 &jb, rec (&r)[SEPK_BATCH]) {
+				const int j[SEPK_BATCH] = {jb.x, jb.y, jb.z, jb.w};
+#pragma unroll
+				for (int u = 0; u < SEPK_BATCH; u++) {
+					r[u].p = sepk_rec(pb, j[u]);
+					r[u].t = TYPED ? s.type[(unsigned)j[u]] : 0;
+				}
+			},
+			[&](const rec (&r)[SEPK_BATCH], sepk_wide_batch<2> &v) {
+#pragma unroll
+				for (int u = 0; u < SEPK_BATCH; u++) {
+					const sepk_pos &p = r[u].p;
+					double kx, ky, kz;
+					const double dx = sepk_image<FAST>(pi.x - p.x, c.L0, c.iL0, kx);
+					const double dy = sepk_image<FAST>(pi.y - p.y, c.L1, c.iL1, ky);
+					const double dz = sepk_image<FAST>(pi.z - p.z, c.L2, c.iL2, kz);
+					const double r2 = dx * dx + dy * dy + dz * dz;
+					const bool in_l = act_l && typed(r[u].t) && r2 < c.cf2;
+					if (in_l) {
+						const double q = c.sig2 * sepk_recip(r2);
+						const double q3 = q * q * q;
+						v.ft[0][u] = fma(c.A, q3, c.nB) * q3 * q;
+						v.e[0][u] = fma(fma(c.C, q3, c.nD), q3, c.ushift);
+					}
+					const bool in_c = act_c && !(fabs(p.q) < DBL_EPSILON) && r2 < cc.cf2;
+					// most listed pairs are inside: evaluated without a
+					// branch, the four entries' chains overlap
+					double ft, e;
+					sepk_coul_pair(cc, p.q * pi.q, in_c ? r2 : 1.0, ft, e);
+					v.ft[1][u] = in_c ? ft : 0.0;
+					v.e[1][u] = in_c ? e : 0.0;
+					if (in_l || in_c) {
+						v.d[0][u] = dx;
+						v.d[1][u] = dy;
+						v.d[2][u] = dz;
+						v.cross |= sepk_cross_code(kx, ky, kz) << (8 * u);
+					}
+				}
+			},
+			wa);
+	}
+	return sepk_wide_hand_over<2>(lds, wa, band, f, acc);
+}
+
+// The end of k_lj_coul, from each lane's sums of the two terms: the force as the
+// two calls would leave it, and the block's (WIDE: the wave's) row of each term.
+template <bool OVERWRITE, bool MIXED, bool WIDE>
+__device__ __forceinline__ void sepk_lj_coul_finish(
+	const sepk_state &s, long n, long npad, const sepk_lj &c, long t, int sub, bool act_l,
+	bool act_c, bool frozen, const sepk_pos &pi, const int4 &qi, double (&fl)[3],
+	double (&fc)[3], double (&al)[7], double (&ac)[7], double *part_lj, double *part_c,
+	long row, long rows)
+{
+	// the two epilogues of sepk_pair_epilogue, the second adding to the first
+#pragma unroll
+	for (int k = 0; k < 3; k++) {
+		fl[k] = sepk_atom_sum(fl[k]);
+		fc[k] = sepk_atom_sum(fc[k]);
+	}
+	if (t < n && sub == 0 && !frozen) {
+		for (int k = 0; k < 3; k++) {
+			double v = OVERWRITE ? fl[k] : s.f[k * npad + t];
+			if (!OVERWRITE && act_l)
+				v += fl[k];
+			if (act_c)
+				v += fc[k];
+			s.f[k * npad + t] = v;
+		}
+	}
+	// the stress identity's positions: quantized (mixed) or FP64
+	const double px = MIXED ? (double)(unsigned)qi.x * c.qd0 : pi.x;
+	const double py = MIXED ? (double)(unsigned)qi.y * c.qd1 : pi.y;
+	const double pz = MIXED ? (double)(unsigned)qi.z * c.qd2 : pi.z;
+	if (act_l && sub == 0) {
+		const double gx = 2.0 * fl[0], gy = 2.0 * fl[1], gz = 2.0 * fl[2];
+		al[1] = fma(gx, px, al[1]);
+		al[2] = fma(gx, py, al[2]);
+		al[3] = fma(gx, pz, al[3]);
+		al[4] = fma(gy, py, al[4]);
+		al[5] = fma(gy, pz, al[5]);
+		al[6] = fma(gz, pz, al[6]);
+	}
+	if (act_c && sub == 0) {
+		const double gx = 2.0 * fc[0], gy = 2.0 * fc[1], gz = 2.0 * fc[2];
+		ac[1] = fma(gx, px, ac[1]);
+		ac[2] = fma(gx, py, ac[2]);
+		ac[3] = fma(gx, pz, ac[3]);
+		ac[4] = fma(gy, py, ac[4]);
+		ac[5] = fma(gy, pz, ac[5]);
+		ac[6] = fma(gz, pz, ac[6]);
+	}
+	double v[14];
+#pragma unroll
+	for (int k = 0; k < 7; k++) {
+		v[k] = al[k];
+		v[7 + k] = ac[k];
+	}
+	const auto out = [=](int i, double r) {
+		(i < 7 ? part_lj : part_c)[(size_t)(i < 7 ? i : i - 7) * rows + row] = r;
+	};
+	if constexpr (WIDE)
+		sepk_wave_reduce<false>(v, 0.0, out);
+	else
+		sepk_block_reduce<false>(v, 0.0, out);
 }
 
 // A pair call (LJ, typed or not) and the shifted-force Coulomb call right
@@ -834,10 +1287,8 @@ __global__ __launch_bounds__(SEPK_BLOCK) void k_lj_coul(
 							     fl[0], fl[1], fl[2], al);
 				}
 				if (act_c && !(fabs(pj[u].q) < DBL_EPSILON) && r2 < cc.cf2) {
-					const double qq = pj[u].q * pi.q;
-					const double r = sqrt(r2);
-					const double ft = qq * (1.0 / r2 - cc.icf2) / r;
-					const double e = qq * (1.0 / r + (r - cc.cf) * cc.icf2 - cc.icf);
+					double ft, e;
+					sepk_coul_pair(cc, pj[u].q * pi.q, r2, ft, e);
 					sepk_pair_accumulate(ft, e, dx, dy, dz, kx, ky, kz, cc.L0, cc.L1,
 							     cc.L2, fc[0], fc[1], fc[2], ac);
 				}
@@ -926,53 +1377,54 @@ __global__ __launch_bounds__(SEPK_BLOCK) void k_lj_coul(
 			sepk_lj_mixed_band<TYPED, FAST>(s, nbr, cnt, npad, c, t, sub, ti, qi, fl[0],
 							fl[1], fl[2], al);
 	}
-	// the two epilogues of sepk_pair_epilogue, the second adding to the first
-#pragma unroll
-	for (int k = 0; k < 3; k++) {
-		fl[k] = sepk_atom_sum(fl[k]);
-		fc[k] = sepk_atom_sum(fc[k]);
+	sepk_lj_coul_finish<OVERWRITE, MIXED, false>(s, n, npad, c, t, sub, act_l, act_c, frozen, pi, qi,
+						     fl, fc, al, ac, part_lj, part_c, lb, rows);
+}
+
+// k_lj_coul by wide walk (maxbat: batches a list's allocation holds), for systems
+// of up to SEPK_WIDE_ATOMS atoms.  The walk by four lanes is a chain of 26 batches
+// in 0.4 wavefronts a SIMD at 6000 atoms of water; this one is 7 rounds in 1.5.
+// What bounds it is the exchange through LDS.  The line lies where its workgroups
+// (59 KB of LDS, two a CU) stop being resident all at once.  Per step of water, four
+// lanes -> 16 (us), FP64 and mixed: 3000 atoms 79 -> 48, 69 -> 49; 6000 86 -> 63,
+// 75 -> 61; 8000 84 -> 62, 77 -> 62; and past the line 9000 85 -> 76, 78 -> 77; 16000
+// 90 -> 97, 84 -> 97.
+template <bool TYPED, bool OVERWRITE, bool MIXED, bool FAST>
+__global__ __launch_bounds__(SEPK_BLOCK) void k_lj_coul_wide(
+	sepk_state s, const int *__restrict__ nbr, const int *__restrict__ cnt, long n,
+	long npad, int maxbat, sepk_lj c, sepk_coul cc, double *part_lj, double *part_c, long rows)
+{
+	__shared__ sepk_wide_lds<2> lds;
+	const long lb = sepk_xcd_block();
+	const bool frozen = *s.err != 0;
+	double f[2][3], acc[2][7];
+	bool band;
+	if (!sepk_lj_coul_pairs_wide<TYPED, MIXED, FAST>(lds, s, nbr, cnt, n, npad, maxbat, c, cc, lb, f,
+							 acc, band))
+		return;
+	const long t = lb * (SEPK_BLOCK / 16) + threadIdx.x / SEPK_SUB;
+	const int sub = threadIdx.x % SEPK_SUB;
+	bool act_l = t < n, act_c = t < n;
+	signed char ti = 0;
+	if (act_l && TYPED) {
+		ti = s.type[t];
+		act_l = ti == c.t0 || ti == c.t1;
 	}
-	if (t < n && sub == 0 && !frozen) {
-		for (int k = 0; k < 3; k++) {
-			double v = OVERWRITE ? fl[k] : s.f[k * npad + t];
-			if (!OVERWRITE && act_l)
-				v += fl[k];
-			if (act_c)
-				v += fc[k];
-			s.f[k * npad + t] = v;
-		}
+	sepk_pos pi = {0.0, 0.0, 0.0, 0.0};
+	if (t < n)
+		pi = s.pos[t];
+	if (act_c)
+		act_c = !(fabs(pi.q) < DBL_EPSILON);
+	int4 qi = make_int4(0, 0, 0, SEPK_QPHANTOM);
+	if (MIXED && (act_l || act_c)) {
+		qi = s.qpos[t];
+		if (band)
+			sepk_lj_mixed_band<TYPED, FAST>(s, nbr, cnt, npad, c, t, sub, ti, qi, f[0][0],
+							f[0][1], f[0][2], acc[0]);
 	}
-	// the stress identity's positions: quantized (mixed) or FP64
-	const double px = MIXED ? (double)(unsigned)qi.x * c.qd0 : pi.x;
-	const double py = MIXED ? (double)(unsigned)qi.y * c.qd1 : pi.y;
-	const double pz = MIXED ? (double)(unsigned)qi.z * c.qd2 : pi.z;
-	if (act_l && sub == 0) {
-		const double gx = 2.0 * fl[0], gy = 2.0 * fl[1], gz = 2.0 * fl[2];
-		al[1] = fma(gx, px, al[1]);
-		al[2] = fma(gx, py, al[2]);
-		al[3] = fma(gx, pz, al[3]);
-		al[4] = fma(gy, py, al[4]);
-		al[5] = fma(gy, pz, al[5]);
-		al[6] = fma(gz, pz, al[6]);
-	}
-	if (act_c && sub == 0) {
-		const double gx = 2.0 * fc[0], gy = 2.0 * fc[1], gz = 2.0 * fc[2];
-		ac[1] = fma(gx, px, ac[1]);
-		ac[2] = fma(gx, py, ac[2]);
-		ac[3] = fma(gx, pz, ac[3]);
-		ac[4] = fma(gy, py, ac[4]);
-		ac[5] = fma(gy, pz, ac[5]);
-		ac[6] = fma(gz, pz, ac[6]);
-	}
-	double v[14];
-#pragma unroll
-	for (int k = 0; k < 7; k++) {
-		v[k] = al[k];
-		v[7 + k] = ac[k];
-	}
-	sepk_block_reduce<false>(v, 0.0, [=](int i, double r) {
-		(i < 7 ? part_lj : part_c)[(size_t)(i < 7 ? i : i - 7) * rows + lb] = r;
-	});
+	sepk_lj_coul_finish<OVERWRITE, MIXED, true>(s, n, npad, c, t, sub, act_l, act_c, frozen, pi, qi,
+						    f[0], f[1], acc[0], acc[1], part_lj, part_c, lb,
+						    rows);
 }
 
 // The recorded pair call and this Coulomb call as one k_lj_coul launch,
@@ -1004,21 +1456,34 @@ static int launch_lj_coul(sepdev *d, const sepk_coul &cc, int ret_slot)
 	if ((rc = sepk_fork_point(d)) || (rc = sepk_flush_gathers(d)))
 		return rc;
 	const bool over = d->f_zero_pending != 0;
+#define SEPK_LJ_COUL(K)                                                                          \
+	{{{{K<false, false, false, false>, K<false, false, false, true>},                        \
+	   {K<false, false, true, false>, K<false, false, true, true>}},                         \
+	  {{K<false, true, false, false>, K<false, true, false, true>},                          \
+	   {K<false, true, true, false>, K<false, true, true, true>}}},                          \
+	 {{{K<true, false, false, false>, K<true, false, false, true>},                          \
+	   {K<true, false, true, false>, K<true, false, true, true>}},                           \
+	  {{K<true, true, false, false>, K<true, true, false, true>},                            \
+	   {K<true, true, true, false>, K<true, true, true, true>}}}}
 	typedef void (*kfn)(sepk_state, const int *, const int *, long, long, sepk_lj, sepk_coul,
 			    double *, double *, long);
-	static const kfn table[2][2][2][2] = {
-		{{{k_lj_coul<false, false, false, false>, k_lj_coul<false, false, false, true>},
-		  {k_lj_coul<false, false, true, false>, k_lj_coul<false, false, true, true>}},
-		 {{k_lj_coul<false, true, false, false>, k_lj_coul<false, true, false, true>},
-		  {k_lj_coul<false, true, true, false>, k_lj_coul<false, true, true, true>}}},
-		{{{k_lj_coul<true, false, false, false>, k_lj_coul<true, false, false, true>},
-		  {k_lj_coul<true, false, true, false>, k_lj_coul<true, false, true, true>}},
-		 {{k_lj_coul<true, true, false, false>, k_lj_coul<true, true, false, true>},
-		  {k_lj_coul<true, true, true, false>, k_lj_coul<true, true, true, true>}}}};
-	const kfn k = table[d->pc_typed ? 1 : 0][over ? 1 : 0][d->pc_mixed ? 1 : 0][d->pc_fast ? 1 : 0];
+	typedef void (*wfn)(sepk_state, const int *, const int *, long, long, int, sepk_lj,
+			    sepk_coul, double *, double *, long);
+	static const kfn table[2][2][2][2] = SEPK_LJ_COUL(k_lj_coul);
+	static const wfn wtable[2][2][2][2] = SEPK_LJ_COUL(k_lj_coul_wide);
+#undef SEPK_LJ_COUL
+	const bool wide = d->n <= SEPK_WIDE_ATOMS;
+	const int kt = d->pc_typed ? 1 : 0, ko = over ? 1 : 0, km = d->pc_mixed ? 1 : 0,
+		  kf = d->pc_fast ? 1 : 0;
 	const unsigned nb = sepk_blocks_xcd(d->n * SEPK_SUB);
-	k<<<nb, SEPK_BLOCK, 0, d->st>>>(d->s[0], d->nbr, d->nbr_count, d->n, d->npad, d->pc_lj, cc,
-					  sepk_region(d, r1), sepk_region(d, r2), d->region_rows);
+	if (wide)
+		wtable[kt][ko][km][kf]<<<4 * nb, SEPK_BLOCK, 0, d->st>>>(
+			d->s[0], d->nbr, d->nbr_count, d->n, d->npad, d->cap / SEPK_PAD, d->pc_lj, cc,
+			sepk_region(d, r1), sepk_region(d, r2), d->region_rows);
+	else
+		table[kt][ko][km][kf]<<<nb, SEPK_BLOCK, 0, d->st>>>(
+			d->s[0], d->nbr, d->nbr_count, d->n, d->npad, d->pc_lj, cc,
+			sepk_region(d, r1), sepk_region(d, r2), d->region_rows);
 	SEPK_LAUNCH_CHECK();
 	d->f_zero_pending = 0;
 	d->last_fused = 0;
@@ -1028,6 +1493,7 @@ static int launch_lj_coul(sepdev *d, const sepk_coul &cc, int ret_slot)
 	f.region = r1;
 	f.nblk = (int)nb;
 	f.nv = 7;
+	f.wide = wide;
 	f.epot_assign = d->pc_epot_assign;
 	sepk_task_ret(d, f, d->pc_ret);
 	if ((rc = sepk_queue_task(d, f)))
@@ -1037,6 +1503,7 @@ static int launch_lj_coul(sepdev *d, const sepk_coul &cc, int ret_slot)
 	f.region = r2;
 	f.nblk = (int)nb;
 	f.nv = 7;
+	f.wide = wide;
 	f.also_ecoul = 1;
 	sepk_task_ret(d, f, ret_slot);
 	return sepk_queue_task(d, f);

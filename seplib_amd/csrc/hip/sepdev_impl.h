@@ -90,6 +90,7 @@ struct sepk_task {
 	int with_stress;  // BONDED: add the stress to pot_P and pot_P_bond
 	double *alpha;    // NH / LF with a fused thermostat
 	double Td, dt_tau2, npart;
+	int wide;         // four rows (a wave's each) make one: SEPK_WIDE_ATOMS
 	int nh_fused;     // LF: the leapfrog applied a pending Nose-Hoover
 	int reset_max;    // LF: max_dist2 was reset since the last leapfrog
 	double skin, dt;
@@ -131,6 +132,10 @@ struct sepk_timer {
 	double ms;
 	long count;
 };
+
+// Systems of up to this many atoms walk their lists for LJ and Coulomb together
+// with 16 lanes an atom (k_lj_coul_wide says why the line lies here).
+#define SEPK_WIDE_ATOMS 8192
 
 // Transfers.  A download is launched in chunks so that the host unpacks one
 // while the next crosses the link.
@@ -546,6 +551,23 @@ __device__ __forceinline__ void sepk_block_reduce(const double (&v)[NV], double 
 		for (int w = 1; w < NW; w++)
 			r = top ? fmax(r, sh[w][i]) : r + sh[w][i];
 		out(i, r);
+	}
+}
+
+// The wave's part of sepk_block_reduce: the same trees, one result a wave,
+// for a wave that leaves the sum over the block's waves to the finisher.
+template <bool MAX, int NV, class OUT>
+__device__ __forceinline__ void sepk_wave_reduce(const double (&v)[NV], double mx, OUT out)
+{
+	const int lane = threadIdx.x & (SEPK_WAVE - 1);
+	const double s = sepk_wave_sums(v);
+	const int c = lane / SEPK_COL_LANES(NV);
+	if (lane % SEPK_COL_LANES(NV) == 0 && c < NV)
+		out(c, s);
+	if (MAX) {
+		const double m = sepk_wave_max(mx);
+		if (lane == 0)
+			out(NV, m);
 	}
 }
 

@@ -120,6 +120,16 @@ __device__ static double fin_comb(bool mx, double a, double b)
 	return mx ? fmax(a, b) : a + b;
 }
 
+// Row r of a task's column p: the block's sum, or its waves' in index order,
+// as sepk_block_reduce adds them.
+__device__ __forceinline__ double fin_row(const sepk_task &k, bool mx, const double *p, long r)
+{
+	if (!k.wide)
+		return p[r];
+	const double a = p[4 * r], b = p[4 * r + 1], c = p[4 * r + 2], d = p[4 * r + 3];
+	return fin_comb(mx, fin_comb(mx, fin_comb(mx, a, b), c), d);
+}
+
 // A task's columns over the wave, left as sepk_wave_sums leaves them; the
 // column whose bit is set in maxmask (at most one) takes the maximum.
 __device__ static double fin_wave(const sepk_task &k, const double (&v)[SEPK_MAXNV])
@@ -160,7 +170,8 @@ __global__ __launch_bounds__(FIN_THREADS) void k_fin_rows(const double *partials
 			double v[SEPK_MAXNV];
 #pragma unroll
 			for (int i = 0; i < SEPK_MAXNV; i++)
-				v[i] = p[(size_t)(i < k.nv ? i : 0) * f.region_rows + r];
+				v[i] = fin_row(k, (k.maxmask >> i) & 1u,
+					       p + (size_t)(i < k.nv ? i : 0) * f.region_rows, r);
 #pragma unroll
 			for (int i = 0; i < SEPK_MAXNV; i++)
 				a[i] = fin_comb((k.maxmask >> i) & 1u, a[i], v[i]);
@@ -292,7 +303,9 @@ __global__ __launch_bounds__(FIN_ONE_THREADS) void k_fin_one(const double *parti
 			double v[FIN_ONE_ROWS / 64];
 #pragma unroll
 			for (int i = 0; i < FIN_ONE_ROWS / 64; i++)
-				v[i] = i < chunk && r0 + i < k.nblk ? p[(size_t)q * f.region_rows + r0 + i] : 0.0;
+				v[i] = i < chunk && r0 + i < k.nblk
+					       ? fin_row(k, mx, p + (size_t)q * f.region_rows, r0 + i)
+					       : 0.0;
 #pragma unroll
 			for (int i = 0; i < FIN_ONE_ROWS / 64; i++)
 				v[i] = fin_comb(mx, 0.0, v[i]);
