@@ -13,9 +13,9 @@
 //   k_bscan       one workgroup per flagged system: scan of the counts
 //                 into cell starts
 //   k_bscatter    the members of every cell in slot order
-//                 (batches of more than SEPB_FMAP systems: k_bbin, one
-//                 workgroup per flagged system with LDS counters, instead
-//                 of these three)
+//                 (k_bbin, one workgroup per flagged system with LDS
+//                 counters, instead of these three: batches of small systems
+//                 and of more than SEPB_FMAP)
 //   k_bsort       one wave per cell of a flagged system: rank the members
 //                 by original index (the new order, independent of the
 //                 atomic order that listed them) and move their state to it
@@ -23,7 +23,8 @@
 //   k_bbuild      one workgroup per cell of a flagged system: the
 //                 candidates of the distinct neighbour cells staged in LDS,
 //                 tested 64 at a time against each home atom (ballots kept
-//                 in LDS), then written to the lists in candidate order
+//                 in LDS), then written to the lists in candidate order; the
+//                 near build does the same in FP32 where cells are few
 //   k_bstep       persistent: the grid walks a table of tiles (a system and
 //                 a run of its atoms, lanes per atom chosen per system);
 //                 pair forces, Nose-Hoover and leapfrog for the tile's
@@ -124,6 +125,7 @@ struct sepdev_batch {
 	int4 *sub_tiles; // a subset (autotuner)
 	int grid;
 	sepb_lj lj;
+	int few, small;  // which build and binning serve it (SEPB_FEW_CELLS, SEPB_BIN_ATOMS)
 	hipGraph_t graph;
 	hipGraphExec_t exec;
 	int graph_mixed, graph_steps;
@@ -143,6 +145,17 @@ __device__ __forceinline__ int sepb_mod(int a, int n)
 #define SEPB_BIN_THREADS 1024
 #define SEPB_MAX_CELLS 8192 // cells per system (LDS counters)
 #define SEPB_BIN_UNROLL 8
+// Batches whose systems have at most SEPB_BIN_ATOMS atoms each are binned by k_bbin
+// in one launch (so are those of more than SEPB_FMAP systems), others by k_bcount,
+// k_bscan and k_bscatter; mixed steps, three launches -> one (us): 12 systems of 500
+// to 3000 atoms 63.6 -> 57.7, of 3000 to 8000 66.1 -> 64.6; 4 of 8000 to 16000 48.7 ->
+// 49.4.
+#define SEPB_BIN_ATOMS 8192
+// Batches of at most SEPB_FEW_CELLS cells are built by k_bbuild<true>, whose cells are
+// done sooner but fit four a CU instead of seven; mixed steps, <false> -> <true> (us):
+// 4 systems of 500 to 1500 atoms 38.1 -> 35.9, 12 of 500 to 3000 63.6 -> 58.3; 5500
+// cells (48 systems) 106.5 -> 100.8, 7500 cells 106.3 -> 107.2, 16300 cells 200 -> 206.
+#define SEPB_FEW_CELLS 6144
 
 // Cell of position q in system y (floor of x / l, by the reciprocal edge il,
 // and periodic wrap); an atom outside [0, L) on some axis (x == L after a
@@ -371,8 +384,8 @@ __device__ __forceinline__ bool sepb_work_cell(const sepb_view &b, const int *fp
 }
 
 // Binning of the flagged systems' atoms across the whole grid, for batches
-// of up to SEPB_FMAP systems (k_bbin, one workgroup per system, serves
-// larger ones): k_bcount gives every atom its cell and its slot among the
+// of up to SEPB_FMAP systems with a large one among them (k_bbin, one workgroup
+// per system, serves the others): k_bcount gives every atom its cell and its slot among the
 // cell's members (global counters, one atomic add per distinct cell of a
 // wave), k_bscan turns each flagged system's counts into cell starts (one
 // workgroup per system) and k_bscatter lists the members of every cell.
@@ -588,9 +601,6 @@ struct sepb_build_lds {
 	double hx[SEPB_BHOME], hy[SEPB_BHOME], hz[SEPB_BHOME];
 	unsigned long long vote[SEPB_BHOME][SEPB_BWORDS];
 	int hcnt[2][SEPB_BHOME]; // list lengths before / after the chunk
-	int segjs[27], segpre[28];
-	double segsh[27][3];
-	int wmax[SEPB_BLOCK / 64];
 };
 
 // Tests the staged candidates [q0, q0 + 64) of a chunk of kn against the
@@ -658,9 +668,129 @@ __device__ __forceinline__ void sepb_build_emit(sepb_build_lds &L, int kn, int h
 	}
 }
 
-__global__ __launch_bounds__(SEPB_BLOCK) __attribute__((amdgpu_waves_per_eu(7))) void k_bbuild(sepb_view b)
+// The near build: the cells of a system of at least three cells an axis with every
+// atom in the box, up to SEPB_NEAR candidates a cell and SEPB_NCAP entries a list.
+// The candidates are staged as FP32 offsets from the cell's centre (x, y, z, and
+// the index with the segment above it), and a wave tests its home atoms against
+// them two at a time.  An FP32 r^2 within `band` of the list cutoff is decided by
+// the FP64 test of the general path, a few in 10^4 atoms, so the lists are the
+// same.  The accepted candidates collect in LDS rows at their rank among the
+// passing lanes and go to the list four entries a store.  The general path reads
+// three FP64 coordinates of the home atom from LDS for every 64 candidates, keeps
+// the ballots and lets one thread per 64 candidates store its hits one by one.  Both
+// wait more than they issue while cells are few; per step of 12 systems of 500 to
+// 3000 atoms the build took 28.9 us and takes 24.
+#define SEPB_NEAR 1344
+#define SEPB_NCAP 256
+#define SEPB_SEGBIT 26 // systems have at most 2^26 atoms
+struct sepb_near_lds {
+	float4 cand[SEPB_NEAR];
+	// two rows a wave, the phantom after them
+	int row[SEPB_BLOCK / 64][2][SEPB_NCAP + 64];
+};
+
+template <bool NEAR>
+union sepb_cell_lds {
+	sepb_build_lds far;
+};
+template <>
+union sepb_cell_lds<true> {
+	sepb_build_lds far;
+	sepb_near_lds near;
+};
+
+// The home atoms of a cell, i = wid, wid + 4, ... < m, against its T staged
+// candidates; returns the longest list of this wave's atoms.
+__device__ __forceinline__ int sepb_build_near(sepb_near_lds &L, const double (&segsh)[27][3], int T, int m, int h0, int n,
+					       int npad, int sub, int lg, int cap, const sepk_pos *pn,
+					       const double (&cen)[3], double rl2, float lo2,
+					       float hi2, int *lst, int *count, sepb_sys *y)
 {
-	__shared__ sepb_build_lds L;
+	const int lane = threadIdx.x & 63;
+	const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); // wave-uniform
+	const int qq = sub * SEPB_BATCH;
+	int full = 0;
+	for (int i = wid; i < m; i += 2 * (SEPB_BLOCK / 64)) {
+		const int i1 = min(i + SEPB_BLOCK / 64, m - 1);
+		const int h[2] = {h0 + i, h0 + i1};
+		float hx[2], hy[2], hz[2];
+#pragma unroll
+		for (int a = 0; a < 2; a++) {
+			const sepk_pos p = pn[h[a]];
+			hx[a] = (float)(p.x - cen[0]);
+			hy[a] = (float)(p.y - cen[1]);
+			hz[a] = (float)(p.z - cen[2]);
+		}
+		int len[2] = {0, 0};
+		for (int q0 = 0; q0 < T; q0 += 64) {
+			const float4 c = L.cand[q0 + lane]; // the array ends on a whole wave
+			const unsigned long long held = T - q0 < 64 ? ~(~0ull << (T - q0)) : ~0ull;
+			const int js = __float_as_int(c.w);
+			const int j = js & ((1 << SEPB_SEGBIT) - 1);
+#pragma unroll
+			for (int a = 0; a < 2; a++) {
+				const float dx = hx[a] - c.x, dy = hy[a] - c.y, dz = hz[a] - c.z;
+				const float r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+				unsigned long long take = __ballot(r2 < lo2) & held;
+				const unsigned long long edge = __ballot(r2 < hi2) & held & ~take;
+				if (edge) {
+					bool in = false;
+					if (edge >> lane & 1ull) {
+						const sepk_pos pi = pn[h[a]], pj = pn[j];
+						const double *sh = segsh[js >> SEPB_SEGBIT];
+						const double ddx = pi.x - (pj.x + sh[0]);
+						const double ddy = pi.y - (pj.y + sh[1]);
+						const double ddz = pi.z - (pj.z + sh[2]);
+						in = ddx * ddx + ddy * ddy + ddz * ddz < rl2;
+					}
+					take |= __ballot(in);
+				}
+				take &= __ballot(j != h[a]);
+				const int e = len[a] + (int)__builtin_amdgcn_mbcnt_hi(
+							       (unsigned)(take >> 32),
+							       __builtin_amdgcn_mbcnt_lo((unsigned)take, 0u));
+				if ((take >> lane & 1ull) && e < SEPB_NCAP)
+					L.row[wid][a][e] = j;
+				len[a] += __popcll(take);
+			}
+		}
+#pragma unroll
+		for (int a = 0; a < 2; a++) {
+			if (a == 1 && i + SEPB_BLOCK / 64 >= m)
+				continue; // the second atom was the last one again
+			full = max(full, len[a]);
+			if (len[a] > cap && lane == 0)
+				atomicCAS(&y->error, 0, SEP_GPU_ENEIGHB);
+			const int cnt = min(len[a], cap);
+			// whole batches of every lane (cap is one), the phantom after the
+			// last entry: at most 64 past it, as qq is
+			const int pad = (cnt + qq - 1) / qq * qq;
+			if (cnt + lane < pad)
+				L.row[wid][a][cnt + lane] = n;
+			__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+			__builtin_amdgcn_wave_barrier();
+			for (int w = lane; w < pad / SEPB_BATCH; w += 64) {
+				const int e = (w >> lg) * qq + (w & (sub - 1));
+				const int *r = L.row[wid][a] + e;
+				*(int4 *)(lst + sepb_entry(e, h[a], npad, sub, lg)) =
+					make_int4(r[0], r[sub], r[2 * sub], r[3 * sub]);
+			}
+			if (lane == 0)
+				count[h[a]] = cnt;
+		}
+		__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+		__builtin_amdgcn_wave_barrier(); // read before the next rows replace it
+	}
+	return full;
+}
+
+template <bool NEAR>
+__global__ __launch_bounds__(SEPB_BLOCK) __attribute__((amdgpu_waves_per_eu(NEAR ? 4 : 7))) void k_bbuild(sepb_view b)
+{
+	__shared__ sepb_cell_lds<NEAR> U;
+	sepb_build_lds &L = U.far;
+	__shared__ int segjs[27], segpre[28], wmax[SEPB_BLOCK / 64];
+	__shared__ double segsh[27][3];
 	__shared__ int fpre[SEPB_FMAP + 1];
 	const bool mapped = b.nsys <= SEPB_FMAP;
 	long total = b.ncell_tot;
@@ -701,10 +831,10 @@ __global__ __launch_bounds__(SEPB_BLOCK) __attribute__((amdgpu_waves_per_eu(7)))
 					  uz = czi + oz[lane / (nox * noy)];
 				const int c2 =
 					sepb_mod(ux, nx) + nx * (sepb_mod(uy, ny) + ny * sepb_mod(uz, nz));
-				L.segjs[lane] = st[c2];
-				L.segsh[lane][0] = ux >= nx ? L0 : (ux < 0 ? -L0 : 0.0);
-				L.segsh[lane][1] = uy >= ny ? L1 : (uy < 0 ? -L1 : 0.0);
-				L.segsh[lane][2] = uz >= nz ? L2 : (uz < 0 ? -L2 : 0.0);
+				segjs[lane] = st[c2];
+				segsh[lane][0] = ux >= nx ? L0 : (ux < 0 ? -L0 : 0.0);
+				segsh[lane][1] = uy >= ny ? L1 : (uy < 0 ? -L1 : 0.0);
+				segsh[lane][2] = uz >= nz ? L2 : (uz < 0 ? -L2 : 0.0);
 				len = st[c2 + 1] - st[c2];
 			}
 			int incl = len;
@@ -714,14 +844,59 @@ __global__ __launch_bounds__(SEPB_BLOCK) __attribute__((amdgpu_waves_per_eu(7)))
 					incl += u;
 			}
 			if (lane < nseg)
-				L.segpre[lane + 1] = incl;
+				segpre[lane + 1] = incl;
 			if (lane == 0)
-				L.segpre[0] = 0;
+				segpre[0] = 0;
 		}
 		__syncthreads();
-		const int T = L.segpre[nseg];
+		const int T = segpre[nseg];
 		int full = 0;
-		for (int hb = 0; hb < m; hb += SEPB_BHOME) {
+		bool near = false;
+		if constexpr (NEAR)
+			near = shift && T <= SEPB_NEAR && cap <= SEPB_NCAP;
+		if constexpr (NEAR) if (near) {
+			const double cen[3] = {(c % nx + 0.5) * y->lcell[0],
+					       (c / nx % ny + 0.5) * y->lcell[1],
+					       (c / (nx * ny) + 0.5) * y->lcell[2]};
+			for (int k0 = threadIdx.x; k0 < T; k0 += 2 * SEPB_BLOCK) {
+				sepk_pos pq[2];
+				int oq[2], jq[2];
+#pragma unroll
+				for (int r = 0; r < 2; r++) {
+					const int k = min(k0 + r * SEPB_BLOCK, T - 1);
+					int o = 0; // the last segment starting at or before k
+#pragma unroll
+					for (int step = 16; step > 0; step >>= 1)
+						if (o + step < nseg && segpre[o + step] <= k)
+							o += step;
+					oq[r] = o;
+					jq[r] = segjs[o] + (k - segpre[o]);
+					pq[r] = pn[jq[r]];
+				}
+#pragma unroll
+				for (int r = 0; r < 2; r++) {
+					const int k = k0 + r * SEPB_BLOCK;
+					if (k >= T)
+						continue;
+					const double *sh = segsh[oq[r]];
+					U.near.cand[k] = make_float4(
+						(float)(pq[r].x + sh[0] - cen[0]),
+						(float)(pq[r].y + sh[1] - cen[1]),
+						(float)(pq[r].z + sh[2] - cen[2]),
+						__int_as_float(oq[r] << SEPB_SEGBIT | jq[r]));
+				}
+			}
+			__syncthreads();
+			// u = 2^-24: an offset (at most M = 1.6 cell edges) is rounded
+			// by u M, a difference of two is off by 4 u M, and r^2 at the
+			// cutoff rl by 14 u M rl and 4 u rl^2 of its own arithmetic
+			const double M = 1.6 * fmax(y->lcell[0], fmax(y->lcell[1], y->lcell[2]));
+			const double band = 0x1p-24 * (24.0 * M * sqrt(rl2) + 16.0 * rl2);
+			full = sepb_build_near(U.near, segsh, T, m, h0, n, npad, sub, lg, cap, pn, cen,
+					       rl2, (float)(rl2 - band), (float)(rl2 + band), lst,
+					       b.nbr_count + off, y);
+		}
+		for (int hb = near ? m : 0; hb < m; hb += SEPB_BHOME) {
 			const int hn = min(m - hb, SEPB_BHOME);
 			if (threadIdx.x < SEPB_BHOME)
 				L.hcnt[0][threadIdx.x] = 0;
@@ -742,10 +917,10 @@ __global__ __launch_bounds__(SEPB_BLOCK) __attribute__((amdgpu_waves_per_eu(7)))
 					int o = 0; // the last segment starting at or before k
 #pragma unroll
 					for (int step = 16; step > 0; step >>= 1)
-						if (o + step < nseg && L.segpre[o + step] <= k)
+						if (o + step < nseg && segpre[o + step] <= k)
 							o += step;
 					rq[r] = q < kn ? o : -1;
-					jq[r] = L.segjs[o] + (k - L.segpre[o]);
+					jq[r] = segjs[o] + (k - segpre[o]);
 				}
 #pragma unroll
 				for (int r = 0; r < PER; r++)
@@ -758,9 +933,9 @@ __global__ __launch_bounds__(SEPB_BLOCK) __attribute__((amdgpu_waves_per_eu(7)))
 					const int q = threadIdx.x + r * SEPB_BLOCK;
 					double px = pq[r].x, py = pq[r].y, pz = pq[r].z;
 					if (shift) {
-						px += L.segsh[rq[r]][0];
-						py += L.segsh[rq[r]][1];
-						pz += L.segsh[rq[r]][2];
+						px += segsh[rq[r]][0];
+						py += segsh[rq[r]][1];
+						pz += segsh[rq[r]][2];
 					}
 					L.cx[q] = px;
 					L.cy[q] = py;
@@ -807,12 +982,12 @@ __global__ __launch_bounds__(SEPB_BLOCK) __attribute__((amdgpu_waves_per_eu(7)))
 		for (int o = 32; o > 0; o >>= 1)
 			full = max(full, __shfl_xor(full, o, 64));
 		if (lane == 0)
-			L.wmax[wid] = full;
+			wmax[wid] = full;
 		__syncthreads();
 		if (threadIdx.x == 0) {
 			int mx = 0;
 			for (int v = 0; v < SEPB_BLOCK / 64; v++)
-				mx = max(mx, L.wmax[v]);
+				mx = max(mx, wmax[v]);
 			if (mx > 0)
 				atomicMax(&y->max_full, mx);
 		}
@@ -1299,6 +1474,11 @@ extern "C" sepdev_batch *sepdev_batch_create(int nsys, const sepdev_batch_sys *i
 	}
 	b->slots = slots;
 	b->ncell_tot = cells;
+	b->few = cells - nsys <= SEPB_FEW_CELLS;
+	b->small = 1;
+	for (int s = 0; s < nsys; s++)
+		if (nsys <= SEPB_FMAP && b->hsys[s].n > SEPB_BIN_ATOMS)
+			b->small = 0;
 	b->prow = slots / 16 + nsys + 64; // tiles hold at least 16 atoms
 	int rc = 0;
 	if (hipStreamCreateWithFlags(&b->st, hipStreamNonBlocking) != hipSuccess)
@@ -1446,7 +1626,7 @@ extern "C" sepdev_batch *sepdev_batch_create(int nsys, const sepdev_batch_sys *i
 static int launch_rebuild(sepdev_batch *b)
 {
 	const sepb_view v = view_of(b);
-	if (b->nsys <= SEPB_FMAP) {
+	if (!b->small) {
 		k_bcount<<<SEPB_BGRID, SEPB_BLOCK, 0, b->st>>>(v);
 		k_bscan<<<b->nsys, SEPB_BIN_THREADS, 0, b->st>>>(v);
 		k_bscatter<<<SEPB_BGRID, SEPB_BLOCK, 0, b->st>>>(v);
@@ -1456,7 +1636,7 @@ static int launch_rebuild(sepdev_batch *b)
 	SEPK_LAUNCH_CHECK();
 	k_bsort<<<512, SEPB_BLOCK, 0, b->st>>>(v);
 	SEPK_LAUNCH_CHECK();
-	k_bbuild<<<SEPB_BGRID, SEPB_BLOCK, 0, b->st>>>(v);
+	(b->few ? k_bbuild<true> : k_bbuild<false>)<<<SEPB_BGRID, SEPB_BLOCK, 0, b->st>>>(v);
 	SEPK_LAUNCH_CHECK();
 	return 0;
 }
