@@ -503,10 +503,14 @@ __global__ __launch_bounds__(1024) void k_order(sepk_state src, sepk_state dst, 
 		sstart[c] = 0;
 	// an error set while this runs is an atom outside the grid, which every
 	// workgroup finds by itself; one set before is looked at once
-	if (tid == 0)
-		failed = bad = sys->error != 0;
-	if (blockIdx.x == 0 && tid == 0)
-		sys->max_full = 0; // the build's atomic maximum starts here
+	if (tid == 0) {
+		const bool err = sys->error != 0;
+		failed = bad = err;
+		// the build's atomic maximum starts here; after an overflow it
+		// stays for the host, which grows the list by it
+		if (blockIdx.x == 0 && !err)
+			sys->max_full = 0;
+	}
 	__syncthreads();
 	const double il0 = 1.0 / g.l[0], il1 = 1.0 / g.l[1], il2 = 1.0 / g.l[2];
 	// whole waves iterate together

@@ -16,6 +16,7 @@ word, and every later kernel of the run reads it and leaves the state
 alone.
 """
 import ctypes as C
+import re
 
 import numpy as np
 import pytest
@@ -129,3 +130,93 @@ def test_list_limit_in_synchronised_mode(product):
         assert np.abs(np.array(s.view["f"])).max() > 0
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("graph", [False, True], ids=["eager", "graph"])
+@pytest.mark.parametrize("k,extra", [(10, 1), (10, 40), (21, 5)])
+def test_overflow_of_a_bound_names_it(product, k, extra, graph):
+    """However many steps follow the one that overflowed, the report holds the
+    length that build found and the bound (4000 and 37044 atoms: the two ways
+    the atoms are ordered)."""
+    w = W.lj_fcc(k, 0.8442, 1.0, seed=4)
+    lib = product.lib
+    s = SepSystem.from_workload(product, w, **KW)
+    try:
+        s.gpu_resident(True)
+        assert _run(s, 2, graph=False) == 0
+        mean, mx = C.c_double(0.0), C.c_int(0)
+        assert lib.sep_gpu_list_stats(s.atoms, C.byref(mean), C.byref(mx)) == 0
+        assert lib.sep_gpu_list_limit(s.atoms, s.sysp, 48) == 0
+        s.sys.neighb_flag = 1  # the next step rebuilds
+        assert lib.sep_gpu_upload(s.atoms, s.sysp) == 0
+        assert _run(s, 1 + extra, graph) == S.SEP_GPU_ENEIGHB
+        said = lib.sep_gpu_last_error_message().decode()
+        found = re.search(r"a list of (\d+) entries exceeds the limit of 48", said)
+        assert found, said
+        # the lists of a liquid two steps apart: nearly the same
+        assert 0.8 * mx.value <= int(found.group(1)) <= 1.25 * mx.value, (said, mx.value)
+    finally:
+        s.close()
+
+
+def _implosion(n, seed):
+    """Atoms of type B (no pair call of "AA" moves them) on their way to the
+    centre, which they would reach after 200 steps, and a few of type A at
+    rest, whose forces the run computes."""
+    L = (n / 0.25) ** (1.0 / 3.0)
+    x = W.uniform(seed, 3 * n).reshape(n, 3) * L
+    v = (0.5 * L - x) / (200 * 0.005)
+    t = np.full(n, b"B")
+    t[::50], v[::50] = b"A", 0.0
+    na = len(t[::50])
+    k = int(np.ceil(na ** (1.0 / 3.0)))
+    g = np.stack(np.meshgrid(*[np.arange(k)] * 3, indexing="ij"), -1).reshape(-1, 3)[:na]
+    x[::50] = (g + 0.5) * (L / k)
+    return dict(x=x, v=v, m=np.ones(n), q=np.zeros(n), type=t, L=np.full(3, L),
+                mol=np.full(n, -1))
+
+
+@pytest.mark.parametrize("graph", [False, True], ids=["eager", "graph"])
+@pytest.mark.parametrize("n", [2000, 20000, 33000])
+def test_run_continues_after_its_list_outgrew_the_allocation(product, n, graph):
+    """Lists that grow several times beyond what the first build was given: each
+    run that overflows says how long its longest list was and grows the list,
+    the next one goes on, and the end is bit for bit that of a system whose
+    list had room for all of it."""
+    w = _implosion(n, 31)
+    lib = product.lib
+    a = SepSystem.from_workload(product, w, **KW)
+    b = SepSystem.from_workload(product, w, **KW)
+    steps = 110
+    try:
+        for s in (a, b):
+            s.gpu_resident(True)
+        assert lib.sep_gpu_list_limit(a.atoms, a.sysp, 1024) == 0
+        ops = [b.op_pairs("AA", 2.5), b.op_leapfrog()]
+        arr = (S.sep_gpu_op * len(ops))(*ops)
+        flags = S.SEP_GPU_RUN_GRAPH if graph else 0
+
+        def go(s, k):
+            return lib.sep_gpu_run(s.atoms, s.sysp, s.retp, arr, len(ops), k, flags)
+
+        assert go(a, steps) == 0
+        done, grown, longest = 0, 0, 0
+        while done < steps:
+            t0 = b.sys.tnow
+            rc = go(b, steps - done)
+            if rc:
+                assert rc == S.SEP_GPU_ENEIGHB
+                found = re.search(r"longest list (\d+)", lib.sep_gpu_last_error_message().decode())
+                assert int(found.group(1)) > max(longest, 64)
+                longest = int(found.group(1))
+                grown += 1
+                assert grown < 12
+            b.gpu_sync()
+            new = int(round((b.sys.tnow - t0) / KW["dt"]))
+            assert (new > 0 or grown > 0) and (rc or new == steps - done)
+            done += new
+        assert grown >= 2
+        _same(_snap(b), _snap(a))
+    finally:
+        a.close()
+        b.close()
