@@ -601,22 +601,35 @@ __global__ __launch_bounds__(1024) void k_order(sepk_state src, sepk_state dst, 
 			mem[sstart[c] - base + atomicAdd(&fill[c - c0], 1)] = (unsigned short)t;
 	}
 	__syncthreads();
-	const bool small = m <= SEPK_ORDER_KEYS;
-	for (int i = tid; i < m && small; i += 1024)
-		keys[i] = sepk_at(src.orig, (unsigned)mem[i]);
-	__syncthreads();
-	// each member ranked by its original index within its cell and moved
-	for (int i = tid; i < m; i += 1024) {
-		const int o = mem[i], c = cid[o];
-		const int a = sstart[c] - base, b = sstart[c + 1] - base;
-		const int key = small ? keys[i] : sepk_at(src.orig, (unsigned)o);
+	// Each member ranked by its original index within its cell and moved.  The
+	// keys are in LDS, SEPK_ORDER_KEYS at a time where the share holds more (a
+	// few very full cells; all atoms in one, where the box has no three cells
+	// an axis).  A pair call that rebuilds, 10000 atoms in one cell: 5.2 ms;
+	// 11.9 with the keys of such a share read from memory for every member,
+	// 9.6 with the three launches; 1000 atoms: 82 us, 108 with the ranking not
+	// unrolled, 135 with the three launches.
+	for (int i0 = 0; i0 < m; i0 += 1024) {
+		const int i = i0 + tid;
+		const bool act = i < m;
+		const int o = act ? mem[i] : 0, c = act ? cid[o] : c0;
+		const int a = sstart[c] - base, b = act ? sstart[c + 1] - base : a;
+		const int key = act ? sepk_at(src.orig, (unsigned)o) : 0;
 		int rank = 0;
-		if (small)
-			for (int j = a; j < b; j++)
+		for (int k0 = 0; k0 < m; k0 += SEPK_ORDER_KEYS) {
+			const int kn = min(m - k0, SEPK_ORDER_KEYS);
+			if (i0 == 0 || m > SEPK_ORDER_KEYS) { // the same for the workgroup
+				__syncthreads(); // the previous keys are no longer read
+				for (int q = tid; q < kn; q += 1024)
+					keys[q] = k0 + q == i ? key : sepk_at(src.orig, (unsigned)mem[k0 + q]);
+				__syncthreads();
+			}
+			const int e = min(b - k0, kn);
+#pragma unroll 4
+			for (int j = max(a - k0, 0); j < e; j++)
 				rank += keys[j] < key;
-		else
-			for (int j = a; j < b; j++)
-				rank += sepk_at(src.orig, (unsigned)mem[j]) < key;
+		}
+		if (!act)
+			continue;
 		const int t = sstart[c] + rank;
 		sepk_move_atom(src, o, dst, t, npad, pending);
 		sepk_at(iperm, (unsigned)key) = t;

@@ -137,6 +137,27 @@ def test_wide_cells(product, oracle, n, clump):
     assert np.array_equal(*pairs)
 
 
+@pytest.mark.parametrize("n", [1024, 1025, 2047, 2049, 4097])
+def test_one_cell(product, oracle, n):
+    """A box of fewer than three list cutoffs an edge: all atoms in one cell,
+    ranked by several rounds of threads against several rounds of keys."""
+    L = 6.0
+    w = _workload(W.uniform(29, 3 * n).reshape(n, 3) * L, [L] * 3)
+    pairs = []
+    for api in (product, oracle):
+        s = SepSystem.from_workload(api, w, cf=1.9, dt=0.005, skin=0.15, nneighb=n + 1,
+                                    update=S.SEP_NEIGHBLIST)
+        try:
+            s.reset_retval()
+            s.reset_force()
+            s.force_pairs("AA", 1.9, "sep_lj", S.SEP_ALL)
+            pairs.append(s.half_pairs())
+        finally:
+            s.close()
+    assert len(pairs[1]) > 0
+    assert np.array_equal(*pairs)
+
+
 @pytest.mark.parametrize("n", [2, 63, 65, 4096, 4097, 32767, 32768, 32769])
 def test_sums_over_blocks(product, oracle, n):
     """Energies and stress where the number of partial rows crosses the
