@@ -264,13 +264,13 @@ static int pack_job(void *arg, int k)
 	return 0;
 }
 
-int seph_put(seph_ctx *c, unsigned mask)
+static int put_fields(seph_ctx *c, unsigned mask, int threads)
 {
 	xfer t = {c, mask, NULL, 0, c->atoms[0].type, 0, 0};
 	int rc = seph_dev_fail(sepdev_put_open(c->dev, &t.rec));
 	if (rc)
 		return rc;
-	const int jobs = c->n >= SEPH_THREAD_ATOMS ? 4 * SEPH_WORKERS : 1;
+	const int jobs = threads && c->n >= SEPH_THREAD_ATOMS ? 4 * SEPH_WORKERS : 1;
 	t.per = (c->n + jobs - 1) / jobs;
 	seph_run_jobs(jobs, c->n, pack_job, &t);
 	if (mask & SEPDEV_SCALARS) {
@@ -279,6 +279,10 @@ int seph_put(seph_ctx *c, unsigned mask)
 	}
 	return seph_dev_fail(sepdev_put_close(c->dev, mask));
 }
+
+int seph_put(seph_ctx *c, unsigned mask) { return put_fields(c, mask, 1); }
+
+int seph_put_noalloc(seph_ctx *c, unsigned mask) { return put_fields(c, mask, 0); }
 
 static int unpack_job(void *arg, int k)
 {

@@ -536,7 +536,7 @@ int sep_gpu_lj_adjoint_noalloc(seppart *ptr, sepsys *sys, int ntypes, const char
 		return seph_fail(SEP_GPU_EARG, "sys->npart (%ld) differs from the %ld atoms",
 				 sys->npart, c->n);
 	int rc;
-	if (!c->resident && ((rc = seph_put(c, SEPDEV_X | SEPDEV_SCALARS))))
+	if (!c->resident && ((rc = seph_put_noalloc(c, SEPDEV_X | SEPDEV_SCALARS))))
 		return rc;
 	sepdev_ljtab_args ta;
 	memset(&ta, 0, sizeof ta);

@@ -81,6 +81,8 @@ int seph_dev_fail(int rc); /* copies the device module's message */
 /* transfers between the AoS and the device (original order) */
 /* the fields of a SEPDEV_X ... mask, in one pass over the atoms */
 int seph_put(seph_ctx *c, unsigned mask);
+/* the same by the caller alone: a thread is started with memory of its own */
+int seph_put_noalloc(seph_ctx *c, unsigned mask);
 int seph_get(seph_ctx *c, unsigned mask);
 /* Every atom's half list: begin sees all counts first (nonzero ends the call),
  * then row is called once per atom, in any order and from several threads. */

@@ -68,3 +68,22 @@ def test_noalloc_adjoint_matches_allocating_form(product):
     finally:
         for s in systems:
             s.close()
+
+
+def test_noalloc_adjoint_of_a_large_system(product):
+    """Past the size from which other calls pack their uploads on several
+    threads (this one does not)."""
+    lib = product.lib
+    w = W.ka_mixture(40000, 1.2, 0.8, seed=14)
+    s = SepSystem.from_workload(product, w, cf=2.5, dt=0.001, skin=0.3, nneighb=FM.NNEIGHB)
+    try:
+        FM.DeviceForces(s, TABLE).forces(w["x"], THETA)
+        g = np.random.default_rng(14).normal(size=(s.n, 3))
+        rc, dx, full = _adjoint(lib, s, g, False)
+        assert rc == 0 and np.abs(dx).max() > 0
+        rc, dx2, full2 = _adjoint(lib, s, g, True)
+        assert rc == 0, lib.sep_gpu_last_error_message()
+        assert np.array_equal(dx2, dx)
+        assert np.array_equal(full2, full)
+    finally:
+        s.close()
