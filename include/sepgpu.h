@@ -21,6 +21,12 @@
  * A system on the device holds at most 2^27 - 64 atoms (every per-atom
  * record is reached by a 32-bit byte offset); a larger one is refused with
  * SEP_GPU_EARG when its device state is created.
+ *
+ * A call that moves atoms to or from the device starts up to three helper
+ * threads and joins them before it returns, from 32768 atoms on (8192 where
+ * it writes neighbour rows): sep_gpu_resident, _upload, _sync, _batch_sync,
+ * _neighbour_pairs and the reference's calls on a system that is not
+ * resident.  They take none of the program's signals.
  */
 #ifndef SEP_MI355X_SEPGPU_H
 #define SEP_MI355X_SEPGPU_H

@@ -4,6 +4,7 @@
  */
 #include <math.h>
 #include <pthread.h>
+#include <signal.h>
 #include <stdarg.h>
 #include <stdio.h>
 #include <stdlib.h>
@@ -199,10 +200,21 @@ int seph_run_jobs(int njobs, long atoms, int (*job)(void *arg, int k), void *arg
 	job_queue q = {njobs, 0, 0, job, arg};
 	pthread_t th[SEPH_WORKERS];
 	int nth = 0;
-	if (atoms >= SEPH_THREAD_ATOMS)
+	if (atoms >= SEPH_THREAD_ATOMS) {
+		/* the program's signals stay with its own threads: a helper takes
+		 * none but those its own instructions raise */
+		sigset_t block, mask;
+		sigfillset(&block);
+		sigdelset(&block, SIGSEGV);
+		sigdelset(&block, SIGBUS);
+		sigdelset(&block, SIGFPE);
+		sigdelset(&block, SIGILL);
+		pthread_sigmask(SIG_BLOCK, &block, &mask);
 		while (nth < SEPH_WORKERS - 1 && nth < njobs - 1 &&
 		       pthread_create(&th[nth], NULL, run_queue, &q) == 0)
 			nth++;
+		pthread_sigmask(SIG_SETMASK, &mask, NULL);
+	}
 	run_queue(&q);
 	for (int i = 0; i < nth; i++)
 		pthread_join(th[i], NULL);

@@ -2,7 +2,9 @@
 replaced by the test program's own (CPU), one program a promise:
 
   * tests/host/adjoint_noalloc.c: sep_gpu_lj_adjoint_noalloc neither allocates
-    nor starts a thread.
+    nor starts a thread;
+  * tests/host/thread_signals.c: the threads that calls on many atoms start
+    take none of the program's signals, and the caller's mask is as it was.
 """
 import glob
 import os
@@ -38,3 +40,7 @@ def _run(tmp_path, name, wrap):
 
 def test_noalloc_adjoint_allocates_nothing(tmp_path):
     _run(tmp_path, "adjoint_noalloc", ["malloc", "calloc", "realloc", "pthread_create"])
+
+
+def test_helper_threads_take_no_signals(tmp_path):
+    _run(tmp_path, "thread_signals", [])
