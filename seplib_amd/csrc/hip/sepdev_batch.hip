@@ -53,6 +53,9 @@
 #define SEPB_NV 16
 #define SEPB_BATCH 4
 #define SEPB_REC_ATOMS 64 // atoms per workgroup of a download
+// slots the pinned records of a download hold (64 MiB), or the largest system's;
+// batches of more come in several passes
+#define SEPB_REC_SLOTS (64L * 1024 * 1024 / (SEPDEV_BATCH_WORDS * (long)sizeof(int)))
 
 // One system on the device.  Read by every kernel; written only by the
 // finishing tile of k_bstep, the last cell of k_bbuild and the host.
@@ -129,9 +132,11 @@ struct sepdev_batch {
 	hipGraph_t graph;
 	hipGraphExec_t exec;
 	int graph_mixed, graph_steps;
-	int *hrec; // pinned records of a download
+	int *hrec;      // pinned records of a download, rec_slots of them
+	long rec_slots;
+	long rec_off;   // first slot of the pass in hrec
 	hipEvent_t chunk_ev[SEPK_CHUNKS];
-	int chunk_sys[SEPK_CHUNKS]; // first system past each chunk
+	int chunk_sys[SEPK_CHUNKS + 1]; // the pass's first system; the first one past each chunk
 };
 
 __device__ __forceinline__ int sepb_mod(int a, int n)
@@ -1407,6 +1412,20 @@ static void drop_graph(sepdev_batch *b)
 	b->graph = nullptr;
 }
 
+// The pinned records, if they are not there.
+static int records_room(sepdev_batch *b)
+{
+	if (b->hrec)
+		return 0;
+	const size_t bytes = (size_t)b->rec_slots * SEPDEV_BATCH_WORDS * sizeof(int);
+	if (hipHostMalloc((void **)&b->hrec, bytes, hipHostMallocDefault) != hipSuccess) {
+		(void)hipGetLastError();
+		b->hrec = nullptr;
+		return sepk_fail(SEP_GPU_EDEVICE, "batch: no %zu bytes of pinned host memory", bytes);
+	}
+	return 0;
+}
+
 extern "C" sepdev_batch *sepdev_batch_create(int nsys, const sepdev_batch_sys *in, double cf,
 					     int cap, int *err)
 {
@@ -1499,9 +1518,14 @@ extern "C" sepdev_batch *sepdev_batch_create(int nsys, const sepdev_batch_sys *i
 	rc |= balloc(&b->partial, (size_t)b->prow * SEPB_NV);
 	rc |= balloc(&b->tiles, b->prow);
 	rc |= balloc(&b->sub_tiles, b->prow);
-	if (hipHostMalloc((void **)&b->hrec, (size_t)slots * SEPDEV_BATCH_WORDS * sizeof(int),
-			  hipHostMallocDefault) != hipSuccess)
-		rc |= sepk_fail(SEP_GPU_EDEVICE, "batch: hipHostMalloc failed");
+	b->rec_slots = SEPB_REC_SLOTS;
+	for (int s = 0; s < nsys; s++)
+		if (b->rec_slots < b->hsys[s].npad)
+			b->rec_slots = b->hsys[s].npad;
+	if (b->rec_slots > slots)
+		b->rec_slots = slots;
+	// a batch without it runs; its download asks again
+	(void)records_room(b);
 	for (hipEvent_t &ev : b->chunk_ev)
 		if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess)
 			rc |= sepk_fail(SEP_GPU_EDEVICE, "batch: hipEventCreate failed");
@@ -1734,15 +1758,13 @@ extern "C" int sepdev_batch_synchronize(sepdev_batch *b)
 	return 0;
 }
 
-// State of system s in its original atom order (3n interleaved vectors;
-// any pointer may be null), its return slot (SEPDEV_RET_WORDS) and scalars
-// {alpha, max_dist2, tnow, nupdate, neighb_flag, max_full, error, sumv2}.
 // Records of the systems s0 + blockIdx.y: x, v, f, a (3 doubles each), the
 // crossings and one word of padding per atom, in original order, written to
-// pinned host memory (system s's from record sys[s].off on).  A record is 112
-// contiguous bytes, so the link sees whole accesses although the atoms arrive
+// pinned host memory (system s's from record sys[s].off - off0 on).  A record is
+// 112 contiguous bytes, so the link sees whole accesses although the atoms arrive
 // in cell order.
-__global__ void k_bgather(const sepb_sys *sys, const sepb_state *st, long slots, int s0, int *rec)
+__global__ void k_bgather(const sepb_sys *sys, const sepb_state *st, long slots, int s0, long off0,
+			  int *rec)
 {
 	const sepb_sys &y = sys[s0 + blockIdx.y];
 	const sepb_state &S = st[y.cur];
@@ -1763,26 +1785,32 @@ __global__ void k_bgather(const sepb_sys *sys, const sepb_state *st, long slots,
 		} else if (w < 27) {
 			v = S.cr[(w - 24) * slots + g];
 		}
-		rec[(y.off + S.orig[g]) * SEPDEV_BATCH_WORDS + w] = v;
+		rec[(y.off - off0 + S.orig[g]) * SEPDEV_BATCH_WORDS + w] = v;
 	}
 }
 
-// Starts the download of the first nsys systems' records in *nchunk chunks
-// of whole systems.  Per-system results (and errors) come from
+// Starts the download of the records of the systems from s0 on that there is room
+// for, of the first nsys, in *nchunk chunks of whole systems; *end is the first
+// system past them.  Per-system results (and errors) come from
 // sepdev_batch_scalars before it.
-extern "C" int sepdev_batch_get_open(sepdev_batch *b, int nsys, int *nchunk)
+extern "C" int sepdev_batch_get_open(sepdev_batch *b, int s0, int nsys, int *end, int *nchunk)
 {
-	int k = 0, s = 0;
+	int rc = records_room(b);
+	if (rc)
+		return rc;
+	int k = 0, s = s0, last = s0;
 	long left = 0;
-	for (int i = 0; i < nsys; i++)
-		left += b->hsys[i].npad;
-	while (s < nsys) {
+	for (; last < nsys && left + b->hsys[last].npad <= b->rec_slots; last++)
+		left += b->hsys[last].npad;
+	b->chunk_sys[0] = s0;
+	b->rec_off = s0 < nsys ? b->hsys[s0].off : 0;
+	while (s < last) {
 		// equal shares of what is left, by atoms
 		const long share = k + 1 < SEPK_CHUNKS ? left / (SEPK_CHUNKS - k) : left;
-		const int s0 = s;
+		const int c0 = s;
 		long atoms = 0;
 		int widest = 0;
-		while (s < nsys && (s == s0 || atoms + b->hsys[s].npad <= share ||
+		while (s < last && (s == c0 || atoms + b->hsys[s].npad <= share ||
 				    atoms + b->hsys[s].npad <= SEPK_CHUNK_ATOMS ||
 				    k + 1 == SEPK_CHUNKS)) {
 			atoms += b->hsys[s].npad;
@@ -1791,14 +1819,16 @@ extern "C" int sepdev_batch_get_open(sepdev_batch *b, int nsys, int *nchunk)
 			s++;
 		}
 		left -= atoms;
-		for (int q = s0; q < s; q += 32768) // grid.y limit
+		for (int q = c0; q < s; q += 32768) // grid.y limit
 			k_bgather<<<dim3((widest + SEPB_REC_ATOMS - 1) / SEPB_REC_ATOMS,
 					 s - q < 32768 ? s - q : 32768),
-				    SEPB_BLOCK, 0, b->st>>>(b->dsys, b->dS, b->slots, q, b->hrec);
+				    SEPB_BLOCK, 0, b->st>>>(b->dsys, b->dS, b->slots, q, b->rec_off,
+							    b->hrec);
 		SEPK_LAUNCH_CHECK();
 		SEPK_CHECK(hipEventRecord(b->chunk_ev[k], b->st));
-		b->chunk_sys[k++] = s;
+		b->chunk_sys[++k] = s;
 	}
+	*end = last;
 	*nchunk = k;
 	return 0;
 }
@@ -1806,14 +1836,14 @@ extern "C" int sepdev_batch_get_open(sepdev_batch *b, int nsys, int *nchunk)
 // Waits for chunk k and gives its systems [*s0, *s1); any thread may call it.
 extern "C" int sepdev_batch_get_chunk(sepdev_batch *b, int k, int *s0, int *s1)
 {
-	*s0 = k ? b->chunk_sys[k - 1] : 0;
-	*s1 = b->chunk_sys[k];
+	*s0 = b->chunk_sys[k];
+	*s1 = b->chunk_sys[k + 1];
 	return (int)hipEventSynchronize(b->chunk_ev[k]);
 }
 
 extern "C" const char *sepdev_batch_records(const sepdev_batch *b, int s)
 {
-	return (const char *)(b->hrec + (size_t)b->hsys[s].off * SEPDEV_BATCH_WORDS);
+	return (const char *)(b->hrec + (size_t)(b->hsys[s].off - b->rec_off) * SEPDEV_BATCH_WORDS);
 }
 
 // Waits for the batch and reads every system's descriptor.

@@ -188,11 +188,12 @@ int sep_gpu_batch_sync(sep_gpu_batch *b, sepret *rets, double *alpha)
 			break;
 		atoms += b->sys[ok]->npart;
 	}
-	int nchunk = 0;
-	if ((rc = seph_dev_fail(sepdev_batch_get_open(b->dev, ok, &nchunk))))
-		return rc;
-	if ((rc = seph_run_jobs(nchunk, atoms, unpack_systems, b)))
-		return seph_dev_fail(sepdev_get_failed(rc));
+	for (int s = 0, end = 0, nchunk = 0; s < ok; s = end) {
+		if ((rc = seph_dev_fail(sepdev_batch_get_open(b->dev, s, ok, &end, &nchunk))))
+			return rc;
+		if ((rc = seph_run_jobs(nchunk, atoms, unpack_systems, b)))
+			return seph_dev_fail(sepdev_get_failed(rc));
+	}
 	for (int s = 0; s < ok; s++) {
 		sepsys *y = b->sys[s];
 		(void)sepdev_batch_scalars(b->dev, s, w, scal);

@@ -272,13 +272,14 @@ int sepdev_batch_synchronize(sepdev_batch *b);
  * system's return slot and alpha, max_dist2, tnow, nupdate, neighb_flag, and
  * returns its device error.  The atoms of systems 0 .. nsys-1 then come as
  * records of SEPDEV_BATCH_WORDS ints in original order (x, v, f, a as doubles,
- * the 3 crossings, padding), in chunks of whole systems: the records of
- * systems [*s0, *s1) may be read once get_chunk has returned 0 (any thread
- * may wait; another value goes to sepdev_get_failed). */
+ * the 3 crossings, padding), in passes: open starts one, of the systems from
+ * s0 to *end, in chunks of whole systems.  The records of systems [*s0, *s1)
+ * may be read once get_chunk has returned 0 (any thread may wait; another value
+ * goes to sepdev_get_failed) and until the next open. */
 #define SEPDEV_BATCH_WORDS 28
 int sepdev_batch_fetch(sepdev_batch *b);
 int sepdev_batch_scalars(sepdev_batch *b, int s, double *ret, double *scal);
-int sepdev_batch_get_open(sepdev_batch *b, int nsys, int *nchunk);
+int sepdev_batch_get_open(sepdev_batch *b, int s0, int nsys, int *end, int *nchunk);
 int sepdev_batch_get_chunk(sepdev_batch *b, int k, int *s0, int *s1);
 const char *sepdev_batch_records(const sepdev_batch *b, int s);
 int sepdev_batch_set_shape(sepdev_batch *b, const int *sub, int grid);

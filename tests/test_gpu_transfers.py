@@ -4,6 +4,8 @@ chunk of a download, of the host threads and of the most chunks there are, and
 again once the device has sorted the atoms.  The same for batches whose
 systems share chunks, fill one, or exceed one.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -104,3 +106,34 @@ def test_half_rows(product, oracle, n, clump):
             s.close()
     assert np.array_equal(pairs[0], pairs[2])
     assert np.array_equal(pairs[1], pairs[2])
+
+
+def test_batch_in_several_passes(product):
+    """More records than the pinned buffer holds (64 MiB: 9362 systems of one to
+    three atoms, each with 64 slots), a larger system among each pass's."""
+    reps = []
+    for k in range(9500):
+        n = 300 if k in (4000, 9450) else 1 + k % 3
+        x = (W.uniform(k, 3 * n).reshape(n, 3) + 0.01) * 5.8
+        reps.append(dict(n=n, rho=n / 216.0, T=1.0, w=dict(
+            x=x, v=W.normal(k, 3 * n).reshape(n, 3), m=np.ones(n), q=np.zeros(n),
+            type=np.full(n, b"A"), L=np.full(3, 6.0), mol=np.full(n, -1))))
+    systems = B.make_systems(product, reps, nneighb=4)
+    b = B.Batch(product, systems, [1.0] * len(reps), precision=S.SEP_GPU_FP64)
+    try:
+        b.eval(S.SEP_GPU_FP64)
+        for s in systems:
+            for k in ("x", "v"):
+                s.view[k] = 0
+            for k in ("f", "a", "crossings"):
+                s.view[k] = 7
+        b.sync()
+        for s, r in zip(systems, reps):
+            assert np.array_equal(s.view["x"], r["w"]["x"])
+            assert np.array_equal(s.view["v"], r["w"]["v"])
+            assert not (np.array(s.view["f"]) == 7).any()
+            assert not np.array(s.view["a"]).any() and not np.array(s.view["crossings"]).any()
+    finally:
+        b.close()
+        for s in systems:
+            s.close()
