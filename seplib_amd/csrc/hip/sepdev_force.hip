@@ -1973,10 +1973,12 @@ extern "C" int sepdev_leapfrog(sepdev *d, double dt, double skin, const double *
 // call, made a synchronised rebuild and its forces take 794 us at 8000 atoms
 // (300 us now) and 10.5 ms at 32000 (1.0 ms).
 // A workgroup that finds no room sets its offset to -1 and runs again in the
-// next pass.
+// next pass, which has its counts.
 #define SEPK_HALF_ATOMS 64
-// entries an atom the pinned buffer holds on average (a full list of 128)
+// entries an atom the pinned buffer holds on average (a full list of 128), and
+// entries it holds at most (256 MiB; or one workgroup's, where those are more)
 #define SEPK_HALF_MEAN 64
+#define SEPK_HALF_MOST (64L * 1024 * 1024)
 __global__ __launch_bounds__(SEPK_BLOCK) void
 k_half_list(const int *orig, const int *iperm, const int *nbr, const int *cnt, long n, long npad,
 	    int *counts, long *off, int *rows, unsigned long long room,
@@ -1990,7 +1992,9 @@ k_half_list(const int *orig, const int *iperm, const int *nbr, const int *cnt, l
 		return;
 	for (int a = wave; a < SEPK_HALF_ATOMS; a += SEPK_BLOCK / 64) {
 		int c = 0;
-		if (o0 + a < n) {
+		if (again) {
+			c = o0 + a < n ? counts[o0 + a] : 0;
+		} else if (o0 + a < n) {
 			const int o = (int)(o0 + a), t = iperm[o], m = cnt[t];
 			for (int k = 0; k < m; k += 64) {
 				const int hit = k + lane < m &&
@@ -2000,7 +2004,7 @@ k_half_list(const int *orig, const int *iperm, const int *nbr, const int *cnt, l
 		}
 		if (lane == 0) {
 			len[a] = c;
-			if (o0 + a < n)
+			if (!again && o0 + a < n)
 				counts[o0 + a] = c;
 		}
 	}
@@ -2050,6 +2054,8 @@ extern "C" int sepdev_half_pass(sepdev *d, int again, sepdev_half *h)
 	const long nblk = (d->n + SEPK_HALF_ATOMS - 1) / SEPK_HALF_ATOMS;
 	// any one workgroup's rows fit
 	size_t room = (size_t)d->npad * SEPK_HALF_MEAN;
+	if (room > SEPK_HALF_MOST)
+		room = SEPK_HALF_MOST;
 	if (room < (size_t)SEPK_HALF_ATOMS * d->cap)
 		room = (size_t)SEPK_HALF_ATOMS * d->cap;
 	if (room > d->half_room) {

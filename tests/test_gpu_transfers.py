@@ -137,3 +137,42 @@ def test_batch_in_several_passes(product):
         b.close()
         for s in systems:
             s.close()
+
+
+def test_half_rows_in_several_passes(product):
+    """Rows that fill more than the largest buffer (256 MiB), against the count
+    of the full lists."""
+    n, L, cf = 38000, 15.0, 4.9
+    x = W.uniform(91, 3 * n).reshape(n, 3) * L
+    w = dict(x=x, v=np.zeros((n, 3)), m=np.ones(n), q=np.zeros(n), type=np.full(n, b"A"),
+             L=np.full(3, L), mol=np.full(n, -1))
+    s = SepSystem.from_workload(product, w, cf=cf, dt=0.005, skin=0.0, nneighb=4,
+                                nsubbox=(3, 3, 3))
+    lib = product.lib
+    try:
+        s.gpu_resident(True)
+        s.gpu_run([s.op_pairs("BB", cf)], 1)
+        mean, mx = C.c_double(0.0), C.c_int(0)
+        assert lib.sep_gpu_list_stats(s.atoms, C.byref(mean), C.byref(mx)) == 0
+        total = int(round(mean.value * n)) // 2
+        assert total > 64 * 1024 * 1024 * 1.5
+        got = np.empty(2 * total, dtype=np.int32)
+        cnt = C.c_long(0)
+        assert lib.sep_gpu_neighbour_pairs(s.atoms, s.sysp, got.ctypes.data_as(C.POINTER(C.c_int)),
+                                           total, C.byref(cnt)) == 0
+        assert cnt.value == total
+        # rows in atom order, their entries above the atom
+        i, j = got[0::2], got[1::2]
+        assert (np.diff(i) >= 0).all() and (j > i).all() and j.max() < n
+        # the counts of a few atoms, from the positions
+        deg = np.bincount(i, minlength=n) + np.bincount(j, minlength=n)
+        for a in (0, 1, 777, 20000, 31000, n - 1):
+            d = x - x[a]
+            d -= L * np.rint(d / L)
+            r2 = (d * d).sum(1)
+            lo, hi = (r2 < (cf * cf) * (1 - 1e-12)).sum() - 1, (r2 < (cf * cf) * (1 + 1e-12)).sum() - 1
+            assert lo <= deg[a] <= hi, a
+            row = j[slice(*np.searchsorted(i, [a, a + 1]))]
+            assert len(np.unique(row)) == len(row)
+    finally:
+        s.close()
