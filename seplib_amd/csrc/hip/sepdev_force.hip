@@ -623,9 +623,11 @@ struct sepk_coul {
 // qq (1/r + (r - rc)/rc^2 - 1/rc).  r, 1/r, 1/r2 and the last division come
 // from one hardware reciprocal square root (2^-24), a coupled Newton step and a
 // residual correction each, which leaves every one of them at the rounding of
-// the operation it stands for; a square root and three divisions took three
-// times the instructions, most of the FP64 walk's (a step of 96000 atoms of water:
-// 251 -> 211 us).
+// the operation it stands for (against long double, r from 1e-6 to the cutoff
+// 2.5, u = 2^-53: the force within 2.7 u |qq| (1/r^2 + 1/rc^2), where operations
+// each at their own rounding may leave 9; the energy within a third of what they
+// may); a square root and three divisions took three times the instructions, most
+// of the FP64 walk's (a step of 96000 atoms of water: 251 -> 211 us).
 __device__ __forceinline__ void sepk_coul_pair(const sepk_coul &c, double qq, double r2, double &ft,
 					       double &e)
 {
