@@ -14,7 +14,7 @@
 //                  of atomic timing) and move each member's state to its new
 //                  cell-sorted index in the spare copy
 //                  (k_order: all of these in one launch, for systems of up to
-//                  32768 atoms)
+//                  32768 atoms, where it says so)
 //   k_build_q      a wave per slab of a cell's atoms (k_build: a workgroup per
 //                  cell, for boxes that are not cubic): the stencil's atoms
 //                  within the list cutoff, 64 candidates at a time; then copy
@@ -466,13 +466,23 @@ __global__ __launch_bounds__(SEPK_BLOCK) void k_sort_permute_wg(
 // SEPK_ORDER_ATOMS atoms and SEPK_ORDER_CELLS cells: every workgroup bins all
 // atoms and scans the cell counts in its LDS, and permutes the cells of its
 // own share, so that no workgroup waits for another and the three launches of
-// a larger system (k_bin, k_scan_scatter, k_sort_permute) are one.  Reading
-// every position in each of 64 workgroups costs a few us a rebuild up to this
-// size; what it saves is two launches in every step, rebuilt or not, and the
-// chain of three kernels' memory round trips in a rebuild.  Per step: N = 1000
-// 23.8 -> 20.3 us, 27000 28.7 -> 27.5, water 6000 98 -> 96.1 (at 27000 a rebuild
-// already spends more on the binning; larger systems gain nothing).
+// a larger system (k_bin, k_scan_scatter, k_sort_permute) are one.  What it saves
+// is two launches in every step, rebuilt or not, and the chain of three kernels'
+// memory round trips in a rebuild; what it costs is the reading of every
+// position in each of 64 workgroups, 31 us a rebuild at 27000 atoms.  Per step,
+// which rebuilds when the flag is set (three launches -> one, us, FP64 LJ liquid at
+// T = 1): 4000 atoms 22.4 -> 19.0, 16000 24.0 -> 21.3, 27000 29.0 -> 27.5, 32000
+// 30.3 -> 29.0; with a rebuild every fifth step (T = 2) 27000 32.0 -> 31.4, 32000
+// 33.7 -> 33.8; water 6000 98 -> 96.1.
+// A call that is sure to rebuild (synchronised, brute force) pays the cost each
+// time and saves the launches once: 8000 atoms 44.8 -> 41.6, 14000 49.9 -> 50.4,
+// 16000 51.5 -> 53.3, 24000 55.7 -> 62.2, 32000 65.3 -> 77.3, so there the line is
+// SEPK_ORDER_BUILD; except where the cells hold more than SEPK_ORDER_FULL atoms on
+// average, whose ranking by 256 threads a cell takes longer than by 1024 (32768
+// atoms in 27 cells 1350 -> 1284, in one 99.3 -> 52.6 ms).
 #define SEPK_ORDER_ATOMS 32768
+#define SEPK_ORDER_BUILD 16384
+#define SEPK_ORDER_FULL 1024
 #define SEPK_ORDER_CELLS 4096
 #define SEPK_ORDER_GRID 64
 #define SEPK_ORDER_KEYS 2048
@@ -1683,7 +1693,8 @@ extern "C" int sepdev_build_list(sepdev *d, const sepdev_grid *gp, int condition
 	sepk_state &cur = d->s[0];   // current state, fixed addresses
 	sepk_state &spare = d->s[1]; // receives the permuted order
 	const int hp = cur.partners != nullptr;
-	if (d->n <= SEPK_ORDER_ATOMS && ncell <= SEPK_ORDER_CELLS) {
+	const bool one = conditional || d->n <= SEPK_ORDER_BUILD || d->n > SEPK_ORDER_FULL * ncell;
+	if (one && d->n <= SEPK_ORDER_ATOMS && ncell <= SEPK_ORDER_CELLS) {
 		const unsigned ob = (unsigned)(ncell < SEPK_ORDER_GRID ? ncell : SEPK_ORDER_GRID);
 		(d->n <= SEPK_ORDER_ATOMS / 8 ? k_order<SEPK_ORDER_ATOMS / 8> : k_order<SEPK_ORDER_ATOMS>)<<<ob, 1024, 0, d->st>>>(
 			cur, spare, d->n, d->npad, g, (int)ncell, d->cell_start, d->iperm, d->sys,

@@ -137,6 +137,28 @@ def test_wide_cells(product, oracle, n, clump):
     assert np.array_equal(*pairs)
 
 
+@pytest.mark.parametrize("resident", [False, True])
+@pytest.mark.parametrize("n", [4097, 16384, 16385, 32768])
+def test_orderings(product, oracle, n, resident):
+    """A call that is sure to rebuild and a step that rebuilds when flagged order
+    the atoms in one launch up to different sizes."""
+    w = W.random_packed(n, 0.5, 1.0, seed=33)
+    grid = [int(l / RL) for l in w["L"]]
+    s = SepSystem.from_workload(product, w, cf=CF, dt=0.005, skin=SKIN, nneighb=200, nsubbox=grid)
+    o = SepSystem.from_workload(oracle, w, cf=CF, dt=0.005, skin=SKIN, nneighb=200, nsubbox=grid)
+    try:
+        if resident:
+            s.gpu_resident(True)
+            s.gpu_run([s.op_pairs("AA", CF, "sep_lj")], 1)
+        else:
+            s.force_pairs("AA", CF, "sep_lj")
+        o.force_pairs("AA", CF, "sep_lj")
+        assert np.array_equal(s.gpu_pairs(), o.half_pairs())
+    finally:
+        s.close()
+        o.close()
+
+
 @pytest.mark.parametrize("n", [1024, 1025, 2047, 2049, 4097])
 def test_one_cell(product, oracle, n):
     """A box of fewer than three list cutoffs an edge: all atoms in one cell,
