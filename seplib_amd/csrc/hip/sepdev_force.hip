@@ -1383,14 +1383,10 @@ __global__ __launch_bounds__(SEPK_BLOCK) void k_lj_coul(
 						     fl, fc, al, ac, part_lj, part_c, lb, rows);
 }
 
-// k_lj_coul by wide walk (maxbat: batches a list's allocation holds), for systems
-// of up to SEPK_WIDE_ATOMS atoms.  The walk by four lanes is a chain of 26 batches
+// k_lj_coul by wide walk (maxbat: batches a list's allocation holds), for the
+// systems that sepk_wide chooses.  The walk by four lanes is a chain of 26 batches
 // in 0.4 wavefronts a SIMD at 6000 atoms of water; this one is 7 rounds in 1.5.
-// What bounds it is the exchange through LDS.  The line lies where its workgroups
-// (59 KB of LDS, two a CU) stop being resident all at once.  Per step of water, four
-// lanes -> 16 (us), FP64 and mixed: 3000 atoms 79 -> 48, 69 -> 49; 6000 86 -> 63,
-// 75 -> 61; 8000 84 -> 62, 77 -> 62; and past the line 9000 85 -> 76, 78 -> 77; 16000
-// 90 -> 97, 84 -> 97.
+// What bounds it is the exchange through LDS.
 template <bool TYPED, bool OVERWRITE, bool MIXED, bool FAST>
 __global__ __launch_bounds__(SEPK_BLOCK) void k_lj_coul_wide(
 	sepk_state s, const int *__restrict__ nbr, const int *__restrict__ cnt, long n,
@@ -1427,6 +1423,24 @@ __global__ __launch_bounds__(SEPK_BLOCK) void k_lj_coul_wide(
 	sepk_lj_coul_finish<OVERWRITE, MIXED, true>(s, n, npad, c, t, sub, act_l, act_c, frozen, pi, qi,
 						    f[0], f[1], acc[0], acc[1], part_lj, part_c, lb,
 						    rows);
+}
+
+// Whether 16 lanes an atom take the walk.  Its workgroups (59 KB of LDS, two a CU)
+// stop being resident all at once at SEPK_WIDE_ATOMS; and a short list leaves most
+// of an atom's lanes without a batch, while there are four times the waves.  How
+// long the lists are the host knows from their allocation, twice the expected mean
+// and 64.  Per step, four lanes -> 16 (us, FP64; mixed within 1 of it), by mean
+// list length:
+//   9 (room 96)     1000 atoms 16.3 -> 18.1, 8192 17.4 -> 20.9:       never
+//   30 (128)        1000 18.9 -> 18.3, 3000 19.9 -> 18.7, 5000 20.3 -> 20.4, 8192 20.3 -> 21.2
+//   72 (224)        1000 22.5 -> 20.8, 3000 22.7 -> 21.1, 5000 22.7 -> 23.9, 8192 23.0 -> 24.7
+//                                                                     up to half the atoms
+//   121 (320)       1000 27.6 -> 22.7, 5000 27.1 -> 25.9, 8192 27.0 -> 26.5
+//   water, 413      3000 79 -> 48, 6000 86 -> 63, 8000 84 -> 62; past the line 9000 85 -> 76
+//                   (mixed 78 -> 77), 16000 90 -> 97
+static bool sepk_wide(const sepdev *d)
+{
+	return d->n <= (d->cap >= 256 ? SEPK_WIDE_ATOMS : d->cap >= 128 ? SEPK_WIDE_ATOMS / 2 : 0);
 }
 
 // The recorded pair call and this Coulomb call as one k_lj_coul launch,
@@ -1474,7 +1488,7 @@ static int launch_lj_coul(sepdev *d, const sepk_coul &cc, int ret_slot)
 	static const kfn table[2][2][2][2] = SEPK_LJ_COUL(k_lj_coul);
 	static const wfn wtable[2][2][2][2] = SEPK_LJ_COUL(k_lj_coul_wide);
 #undef SEPK_LJ_COUL
-	const bool wide = d->n <= SEPK_WIDE_ATOMS;
+	const bool wide = sepk_wide(d);
 	const int kt = d->pc_typed ? 1 : 0, ko = over ? 1 : 0, km = d->pc_mixed ? 1 : 0,
 		  kf = d->pc_fast ? 1 : 0;
 	const unsigned nb = sepk_blocks_xcd(d->n * SEPK_SUB);

@@ -133,8 +133,8 @@ struct sepk_timer {
 	long count;
 };
 
-// Systems of up to this many atoms walk their lists for LJ and Coulomb together
-// with 16 lanes an atom (k_lj_coul_wide says why the line lies here).
+// Systems of up to this many atoms may walk their lists for LJ and Coulomb together
+// with 16 lanes an atom (sepk_wide says when, and why the line lies here).
 #define SEPK_WIDE_ATOMS 8192
 
 // Transfers.  A download is launched in chunks so that the host unpacks one

@@ -28,10 +28,13 @@ def _system(n, rho, seed):
                 type=t, L=np.full(3, L), mol=np.full(n, -1))
 
 
-def _run(product, w, types, precision, used, together):
+def _run(product, w, types, precision, used, together, room=0):
     s = SepSystem.from_workload(product, w, cf=2.5, dt=0.001, skin=0.25)
     try:
         s.gpu_precision(precision)
+        if room:  # the list's allocation, without a bound on it
+            for entries in (room, 0):
+                s.check(s._lib().sep_gpu_list_limit(s.atoms, s.sysp, entries))
         s.gpu_resident(True)
         if together:
             ops = [s.op_pairs(types, 2.5, "sep_lj_shift"), s.op_coulomb(2.4), s.op_leapfrog()]
@@ -63,5 +66,17 @@ def test_wide_walk_same_bits(product, n, rho, types, used, precision):
     w = _system(n, rho, 11 + n)
     a = _run(product, w, types, precision, used, True)
     b = _run(product, w, types, precision, used, False)
+    for k in a:
+        assert np.array_equal(np.asarray(a[k]), np.asarray(b[k])), k
+
+
+@pytest.mark.parametrize("room", [128, 512])
+@pytest.mark.parametrize("n,rho", [(1, 0.001), (15, 0.05), (17, 0.05), (64, 0.2), (4096, 0.1),
+                                   (4097, 0.1), (8192, 0.1), (8193, 0.1)])
+def test_walks_of_short_lists(product, n, rho, room):
+    """Short lists, whose allocation decides how many lanes walk them."""
+    w = _system(n, rho, 11 + n)
+    a = _run(product, w, "AB", S.SEP_GPU_FP64, False, True, room)
+    b = _run(product, w, "AB", S.SEP_GPU_FP64, False, False)
     for k in a:
         assert np.array_equal(np.asarray(a[k]), np.asarray(b[k])), k
