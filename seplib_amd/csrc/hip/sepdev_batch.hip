@@ -152,15 +152,24 @@ __device__ __forceinline__ int sepb_mod(int a, int n)
 #define SEPB_BIN_UNROLL 8
 // Batches whose systems have at most SEPB_BIN_ATOMS atoms each are binned by k_bbin
 // in one launch (so are those of more than SEPB_FMAP systems), others by k_bcount,
-// k_bscan and k_bscatter; mixed steps, three launches -> one (us): 12 systems of 500
-// to 3000 atoms 63.6 -> 57.7, of 3000 to 8000 66.1 -> 64.6; 4 of 8000 to 16000 48.7 ->
-// 49.4.
+// k_bscan and k_bscatter; steps, three launches -> one (us, mixed and FP64): 48 systems
+// of 180 to 400 atoms 63.8 -> 55.8, 12 of 500 to 3000 48 -> 42, 12 of 3000 to 8000 61.9
+// -> 59.2 and 63.2 -> 60.6, 48 of 1000 to 8000 104.7 -> 102.9 and 109.0 -> 107.1, one
+// of 8000 28.5 -> 25.5; 4 of 8000 to 16000 48.7 -> 49.4 and 48.3 -> 48.1.
 #define SEPB_BIN_ATOMS 8192
 // Batches of at most SEPB_FEW_CELLS cells are built by k_bbuild<true>, whose cells are
-// done sooner but fit four a CU instead of seven; mixed steps, <false> -> <true> (us):
-// 4 systems of 500 to 1500 atoms 38.1 -> 35.9, 12 of 500 to 3000 63.6 -> 58.3; 5500
-// cells (48 systems) 106.5 -> 100.8, 7500 cells 106.3 -> 107.2, 16300 cells 200 -> 206.
+// done sooner but fit four a CU instead of seven; steps, <false> -> <true> (us, mixed
+// and FP64 within 1 of each other unless given): 48 systems of 180 to 400 atoms 57.1 ->
+// 55.6, 12 of 500 to 3000 46.4 -> 41.7, 48 of 300 to 2500 80.6 -> 75.6 (FP64 82.3 ->
+// 77.4), 60 of 500 to 6000 (4540 cells) 99.6 -> 92.1; 7500 cells 106.3 -> 107.2, 48 of
+// 500 to 32000 200 -> 206 (FP64 172.4 -> 177.5), 10400 cells at a quarter of the
+// density 56 -> 64.  Not where a system's cells would all run at once in one form
+// and not in the other, from SEPB_FEW_LOW to the seven-a-CU grid a system on
+// average: one of 16000 atoms (729 cells) 31.7 -> 31.3, of 20000 (1000) 35.1 -> 37.6, of
+// 30000 (1331) 38.8 -> 42.6, 4 of 24000 to 32000 (1166 each) 75.3 -> 82.9, one of 60000
+// (2744) 70.5 -> 62.1.
 #define SEPB_FEW_CELLS 6144
+#define SEPB_FEW_LOW 768
 
 // Cell of position q in system y (floor of x / l, by the reciprocal edge il,
 // and periodic wrap); an atom outside [0, L) on some axis (x == L after a
@@ -1493,7 +1502,8 @@ extern "C" sepdev_batch *sepdev_batch_create(int nsys, const sepdev_batch_sys *i
 	}
 	b->slots = slots;
 	b->ncell_tot = cells;
-	b->few = cells - nsys <= SEPB_FEW_CELLS;
+	const long each = (cells - nsys) / nsys; // cells a system
+	b->few = cells - nsys <= SEPB_FEW_CELLS && (each <= SEPB_FEW_LOW || each > SEPB_BGRID);
 	b->small = 1;
 	for (int s = 0; s < nsys; s++)
 		if (nsys <= SEPB_FMAP && b->hsys[s].n > SEPB_BIN_ATOMS)

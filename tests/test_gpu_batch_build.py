@@ -94,3 +94,14 @@ def test_binning_same_bits(product, n):
     both = _forces(product, reps, 0, 0, S.SEP_GPU_FP64)
     assert np.array_equal(alone[0][0], both[0][0])
     assert alone[0][1] == both[0][1]
+
+
+def test_build_choice_same_bits(product):
+    """A system of 1000 cells alone, built by the general path, and beside small
+    ones, with which the batch takes the near one."""
+    big = dict(n=20000, rho=0.9, T=1.0, w=W.random_packed(20000, 0.9, 1.0, seed=12))
+    small = dict(n=200, rho=0.8, T=1.0, w=W.random_packed(200, 0.8, 1.0, seed=13))
+    alone = _forces(product, [big], 0, 0, S.SEP_GPU_FP64)
+    both = _forces(product, [big, small, small], 0, 0, S.SEP_GPU_FP64)
+    for a, b in zip(alone[0], both[0]):
+        assert np.array_equal(np.asarray(a), np.asarray(b))
