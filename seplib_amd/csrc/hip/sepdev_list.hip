@@ -1737,11 +1737,15 @@ extern "C" int sepdev_build_list(sepdev *d, const sepdev_grid *gp, int condition
 	// full: at least 16 atoms a slice, at most SEPK_BHOME, about 1024
 	// slices.  Quantized, a wave a slice: about SEPK_QSLICE atoms, fewer
 	// where there would not be 2048 slices (N = 27000: 37.5 us a step; 38.5
-	// with 4096 slices, 39.4 with a workgroup a cell).
+	// with 4096 slices, 39.4 with a workgroup a cell), 4096 where the cells
+	// hold more than 64 atoms, so that slices of several atoms are left (a
+	// pair call that rebuilds, us: 16000 atoms in 125 cells 148 -> 121, in 216
+	// 97 -> 81, 32000 317 -> 254 and 189 -> 159; 8000 in 125 53 -> 56, so not
+	// below.  The FP64 build took 134, 90, 287, 180 and 69).
 	const long avg = (d->n + ncell - 1) / ncell;
 	const long least = qnt ? (avg + 31) / 32 : (avg + SEPK_BHOME - 1) / SEPK_BHOME;
 	const long most = qnt ? avg : (avg + 15) / 16;
-	const long fill = ((qnt ? 2048 : 1024) + ncell - 1) / ncell;
+	const long fill = ((qnt ? avg > 64 ? 4096 : 2048 : 1024) + ncell - 1) / ncell;
 	long nslice = qnt ? (avg + SEPK_QSLICE / 2) / SEPK_QSLICE : 1;
 	if (nslice < fill)
 		nslice = fill;

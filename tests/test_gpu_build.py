@@ -78,6 +78,14 @@ def test_grids(product, oracle, cells, per_cell):
     _check(product, oracle, _workload(_edge_pairs(_points(n, L, 3), L, 5), [L] * 3))
 
 
+@pytest.mark.parametrize("cells,per_cell", [(5, 64), (5, 65), (6, 130)])
+def test_slices(product, oracle, cells, per_cell):
+    """Cells of more atoms than a wave, cut into more slices."""
+    L = RL * cells * 1.0001
+    n = per_cell * cells ** 3
+    _check(product, oracle, _workload(_edge_pairs(_points(n, L, 15), L, 17), [L] * 3), nneighb=1200)
+
+
 @pytest.mark.parametrize("clump", [60, 65, 200, 700])
 @pytest.mark.parametrize("opt", [S.SEP_ALL, S.SEP_EXCL_SAME_MOL, S.SEP_EXCL_BONDED])
 def test_full_cells(product, oracle, clump, opt):
