@@ -22,11 +22,11 @@
  * record is reached by a 32-bit byte offset); a larger one is refused with
  * SEP_GPU_EARG when its device state is created.
  *
- * A call that moves atoms to or from the device starts up to three helper
- * threads and joins them before it returns, from 32768 atoms on (8192 where
- * it writes neighbour rows): sep_gpu_resident, _upload, _sync, _batch_sync,
- * _neighbour_pairs and the reference's calls on a system that is not
- * resident.  They take none of the program's signals.
+ * A call that moves atoms to or from the device may start up to three helper
+ * threads, which it joins before it returns: sep_gpu_upload, _sync and
+ * _batch_sync from 32768 atoms on, sep_gpu_resident and the reference's calls
+ * on a system that is not resident from 49152 on, and calls that write
+ * neighbour rows from 16384 on.  The threads take none of the program's signals.
  */
 #ifndef SEP_MI355X_SEPGPU_H
 #define SEP_MI355X_SEPGPU_H

@@ -173,10 +173,17 @@ seph_ctx *seph_ctx_for(seppart *atoms, const sepsys *sys)
 
 /* Runs jobs 0 .. njobs-1, on SEPH_WORKERS threads when they handle many
  * atoms in all: the atom array (568 bytes an atom) is more than one core
- * streams while its records cross the link (256000 atoms unpacked in 4.4 ms by
- * one thread, in 1.6 ms by four); smaller arrays are unpacked within 0.2 ms. */
+ * streams while its records cross the link (sep_gpu_sync of 256000 atoms 4.1 ms
+ * by one thread, 1.6 by four, of 50000 0.55 -> 0.34; sep_gpu_upload of 32768
+ * 350 -> 218 us).  A program of synchronised calls goes through the array six
+ * times a step, and what its one core holds of it after a call is spread over
+ * four cores by threads: there the line is SEPH_CALL_ATOMS (a step of
+ * sep_force_pairs, sep_nosehoover and sep_leapfrog, one thread -> four: 32768 atoms
+ * 1.08 -> 1.80 ms, 40000 1.41 -> 1.83, 49152 2.05 -> 2.20, 55000 2.55 -> 2.26, 65000
+ * 3.80 -> 2.80, 100000 6.5 -> 4.1). */
 #define SEPH_WORKERS 4
 #define SEPH_THREAD_ATOMS 32768
+#define SEPH_CALL_ATOMS 49152
 
 typedef struct {
 	int njobs, next, rc;
@@ -276,15 +283,21 @@ static int pack_job(void *arg, int k)
 	return 0;
 }
 
-static int put_fields(seph_ctx *c, unsigned mask, int threads)
+/* The atoms that decide whether a transfer of c starts threads. */
+static long transfer_atoms(const seph_ctx *c)
+{
+	return c->resident || c->n >= SEPH_CALL_ATOMS ? c->n : 0;
+}
+
+static int put_fields(seph_ctx *c, unsigned mask, long atoms)
 {
 	xfer t = {c, mask, NULL, 0, c->atoms[0].type, 0, 0};
 	int rc = seph_dev_fail(sepdev_put_open(c->dev, &t.rec));
 	if (rc)
 		return rc;
-	const int jobs = threads && c->n >= SEPH_THREAD_ATOMS ? 4 * SEPH_WORKERS : 1;
+	const int jobs = atoms >= SEPH_THREAD_ATOMS ? 4 * SEPH_WORKERS : 1;
 	t.per = (c->n + jobs - 1) / jobs;
-	seph_run_jobs(jobs, c->n, pack_job, &t);
+	seph_run_jobs(jobs, atoms, pack_job, &t);
 	if (mask & SEPDEV_SCALARS) {
 		c->uniform_type = t.mixed ? 0 : t.type0;
 		c->uniform_type_valid = 1;
@@ -292,7 +305,7 @@ static int put_fields(seph_ctx *c, unsigned mask, int threads)
 	return seph_dev_fail(sepdev_put_close(c->dev, mask));
 }
 
-int seph_put(seph_ctx *c, unsigned mask) { return put_fields(c, mask, 1); }
+int seph_put(seph_ctx *c, unsigned mask) { return put_fields(c, mask, transfer_atoms(c)); }
 
 int seph_put_noalloc(seph_ctx *c, unsigned mask) { return put_fields(c, mask, 0); }
 
@@ -332,7 +345,7 @@ static int get_fields(seph_ctx *c, unsigned mask, int xn_pending)
 	if (rc)
 		return rc;
 	xfer t = {c, mask, (char *)rec, xn_pending, 0, 0, 0};
-	rc = seph_run_jobs(nchunk, c->n, unpack_job, &t);
+	rc = seph_run_jobs(nchunk, transfer_atoms(c), unpack_job, &t);
 	return rc ? seph_dev_fail(sepdev_get_failed(rc)) : 0;
 }
 
@@ -711,8 +724,10 @@ int seph_half_lists(seph_ctx *c, int (*begin)(void *arg, const int *counts),
 		return rc;
 	for (;;) {
 		w.missing = 0;
-		/* an entry weighs less than an atom's record, a row more */
-		seph_run_jobs((int)((w.h.nblk + HALF_JOB - 1) / HALF_JOB), 4 * c->n, half_job, &w);
+		/* rows take longer than records: a pair call that rebuilds, one thread
+		 * -> four, 8192 atoms 277 -> 287 us, 16000 419 -> 402, 24000 539 -> 518,
+		 * 32767 759 -> 654 */
+		seph_run_jobs((int)((w.h.nblk + HALF_JOB - 1) / HALF_JOB), 2 * c->n, half_job, &w);
 		if (!w.missing)
 			return 0;
 		if ((rc = seph_dev_fail(sepdev_half_pass(c->dev, 1, &w.h))))

@@ -60,6 +60,28 @@ def test_fields_survive(product, n):
         s.close()
 
 
+@pytest.mark.parametrize("n", [16384, 49151, 49152])
+def test_synchronised_step(product, n):
+    """A synchronised leapfrog without forces, packed and unpacked by the caller
+    alone and by several threads: x moves by v dt, and nothing else does."""
+    L, dt = 50.0, 0.004
+    x = W.uniform(n, 3 * n).reshape(n, 3) * (L - 2.0) + 1.0
+    v = W.normal(n + 1, 3 * n).reshape(n, 3)
+    w = dict(x=x, v=v, m=1.0 + W.uniform(n + 2, n), q=np.zeros(n), type=np.full(n, b"A"),
+             L=np.full(3, L), mol=np.full(n, -1))
+    s = SepSystem.from_workload(product, w, cf=2.5, dt=dt, skin=0.3, nneighb=8)
+    try:
+        s.view["crossings"] = np.arange(3 * n).reshape(n, 3)
+        s.view["xn"] = x
+        s.leapfrog()
+        assert np.array_equal(s.view["x"], x + v * dt)
+        assert np.array_equal(s.view["v"], v) and not np.array(s.view["a"]).any()
+        assert np.array_equal(s.view["crossings"], np.arange(3 * n).reshape(n, 3))
+        assert np.array_equal(s.view["xn"], x)
+    finally:
+        s.close()
+
+
 @pytest.mark.parametrize("sizes", [[33], [64, 65, 200], [300] * 70, [17000, 40, 20000, 900, 50]])
 def test_batch_survives(product, sizes):
     reps = [dict(n=n, rho=0.3, T=1.0, w=W.random_packed(n, 0.1, 1.0, seed=5 + k))
