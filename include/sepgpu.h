@@ -23,10 +23,10 @@
  * SEP_GPU_EARG when its device state is created.
  *
  * A call that moves atoms to or from the device may start up to three helper
- * threads, which it joins before it returns: sep_gpu_upload, _sync and
- * _batch_sync from 32768 atoms on, sep_gpu_resident and the reference's calls
- * on a system that is not resident from 49152 on, and calls that write
- * neighbour rows from 16384 on.  The threads take none of the program's signals.
+ * threads, which it joins before it returns: sep_gpu_resident, _upload, _sync
+ * and _batch_sync from 32768 atoms on, the reference's calls on a system that is
+ * not resident from 49152 on, and calls that write neighbour rows from 16384 on.
+ * The threads take none of the program's signals.
  */
 #ifndef SEP_MI355X_SEPGPU_H
 #define SEP_MI355X_SEPGPU_H

@@ -283,11 +283,8 @@ static int pack_job(void *arg, int k)
 	return 0;
 }
 
-/* The atoms that decide whether a transfer of c starts threads. */
-static long transfer_atoms(const seph_ctx *c)
-{
-	return c->resident || c->n >= SEPH_CALL_ATOMS ? c->n : 0;
-}
+/* The atoms that decide whether a call's transfers start threads. */
+static long call_atoms(const seph_ctx *c) { return c->n >= SEPH_CALL_ATOMS ? c->n : 0; }
 
 static int put_fields(seph_ctx *c, unsigned mask, long atoms)
 {
@@ -305,7 +302,7 @@ static int put_fields(seph_ctx *c, unsigned mask, long atoms)
 	return seph_dev_fail(sepdev_put_close(c->dev, mask));
 }
 
-int seph_put(seph_ctx *c, unsigned mask) { return put_fields(c, mask, transfer_atoms(c)); }
+int seph_put(seph_ctx *c, unsigned mask) { return put_fields(c, mask, call_atoms(c)); }
 
 int seph_put_noalloc(seph_ctx *c, unsigned mask) { return put_fields(c, mask, 0); }
 
@@ -337,7 +334,7 @@ static int unpack_job(void *arg, int k)
 	return 0;
 }
 
-static int get_fields(seph_ctx *c, unsigned mask, int xn_pending)
+static int get_fields(seph_ctx *c, unsigned mask, long atoms, int xn_pending)
 {
 	const char *rec;
 	int nchunk;
@@ -345,13 +342,13 @@ static int get_fields(seph_ctx *c, unsigned mask, int xn_pending)
 	if (rc)
 		return rc;
 	xfer t = {c, mask, (char *)rec, xn_pending, 0, 0, 0};
-	rc = seph_run_jobs(nchunk, transfer_atoms(c), unpack_job, &t);
+	rc = seph_run_jobs(nchunk, atoms, unpack_job, &t);
 	return rc ? seph_dev_fail(sepdev_get_failed(rc)) : 0;
 }
 
 int seph_get(seph_ctx *c, unsigned mask)
 {
-	return get_fields(c, mask, 0);
+	return get_fields(c, mask, call_atoms(c), 0);
 }
 
 int seph_put_partners(seph_ctx *c)
@@ -463,7 +460,7 @@ static int get_atoms(seph_ctx *c, sepdev_sys *ds)
 	if ((rc = seph_dev_fail(sepdev_get_settle(c->dev, mask))) ||
 	    (rc = seph_dev_fail(sepdev_get_sys(c->dev, ds))))
 		return rc;
-	return get_fields(c, mask, ds->xn_pending != 0);
+	return get_fields(c, mask, c->n, ds->xn_pending != 0);
 }
 
 int seph_get_atoms(seph_ctx *c)
@@ -474,8 +471,8 @@ int seph_get_atoms(seph_ctx *c)
 
 int seph_put_atoms(seph_ctx *c)
 {
-	const int rc = seph_put(c, SEPDEV_X | SEPDEV_V | SEPDEV_F | SEPDEV_A | SEPDEV_XN |
-					   SEPDEV_SCALARS | SEPDEV_CROSS_NB | SEPDEV_CROSS);
+	const int rc = put_fields(c, SEPDEV_X | SEPDEV_V | SEPDEV_F | SEPDEV_A | SEPDEV_XN |
+					   SEPDEV_SCALARS | SEPDEV_CROSS_NB | SEPDEV_CROSS, c->n);
 	/* a resident system looks its types up at the first call that needs them */
 	c->uniform_type_valid = 0;
 	return rc;
