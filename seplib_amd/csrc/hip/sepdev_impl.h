@@ -485,7 +485,7 @@ __device__ __forceinline__ void sepk_wave_level(double *v)
 // tree (partners 32, 16, 8, 4, 2, 1 apart), but a level halves the columns a
 // lane carries instead of repeating all of them in every lane, and moves them
 // with lane swaps and DPP: 16 columns take about 65 vector instructions and no
-// LDS where 16 butterflies took 96 additions and 192 LDS permutes, a fifth of
+// LDS where 16 butterflies took 96 additions and 192 LDS permutes, an eighth of
 // the fused step kernel's instructions (the same bits; per step, N = 1000:
 // 31.5 -> 27.3 us, 256000 mixed: 91.3 -> 81.5, 500000: 181.5 -> 177.8, water
 // 96000: 197.9 -> 186).  Column c is left in lanes
