@@ -937,6 +937,9 @@ extern "C" int sepdev_checkpoint_read(sepdev *d, void *file)
 	SEPK_CHECK(hipStreamSynchronize(d->st));
 	if (h.list_built && (rc = sepdev_reserve_list(d, h.cap)))
 		return rc;
+	// a new list's lengths are cleared on the stream, which the copies below
+	// do not wait for
+	SEPK_CHECK(hipStreamSynchronize(d->st));
 	if (h.has_partners && !d->s[0].partners) {
 		for (int b = 0; b < 2; b++)
 			if ((rc = dalloc(&d->s[b].partners, (size_t)40 * d->npad)))
